@@ -47,8 +47,8 @@ struct Sizes {
 
 // Device tables the fused kernels read (FP32 twiddles, half-sample shifts).
 struct FusedTables {
-    const void *tw1, *twW, *twZ, *tw2, *tw256, *h_ref, *h_zoom;
-    const void *tw256_64;          // FP64 e^{-2 pi i k/256} (peak refinement)
+    const void *tw1, *twW, *twZ, *tw2, *tws, *h_ref, *h_zoom;
+    const void *tws_64;            // FP64 e^{-2 pi i k/surface side} (peak refinement)
 };
 
 // Pointers of one fused launch: images and starts, per-window stage outputs,
@@ -75,11 +75,12 @@ struct Engine {
     ampcor_params p{};
     ampcor_sizes sz{};
     bool configured = false;
+    bool fused_auto = false;       // AMPCOR_MODE_AUTO runs the fused kernels (sz.fused: AMPCOR_MODE_FUSED may be asked for)
     std::string last_error;
     std::map<int, std::unique_ptr<FftPlan>> plans;
     std::map<std::string, std::unique_ptr<DevBuf>> bufs;
     DevBuf sinc_table;
-    int sinc_dec = 4096, sinc_len = 8;
+    int sinc_dec = 4096;
 
     // per-kernel event timing (ampcor_profile)
     struct ProfRec { std::string name; hipEvent_t a, b; int windows; };
@@ -184,7 +185,10 @@ struct Engine {
 
 // FFT schedule for length n (radices in pass order; direct DFT if a prime > 17 remains)
 FftDesc make_schedule(int n);
-// whether the fused kernels cover a configuration
+// whether the fused kernels can run a configuration (what AMPCOR_MODE_AUTO goes by), and
+// whether it is one of those that AMPCOR_MODE_FUSED and the allocation-free entry accept
+// (surface oversampling 16 by the FFT)
+bool fused_fits(const ampcor_params &p, const ampcor_sizes &s);
 bool fused_supported(const ampcor_params &p, const ampcor_sizes &s);
 
 }  // namespace ampcor

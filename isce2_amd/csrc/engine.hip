@@ -154,6 +154,7 @@ void Engine::setup(const ampcor_params &q) {
     configured = true;
     // the fused kernels' tables are built here, so that runs (the allocation-free
     // entry in particular) find them in place
+    fused_auto = fused_fits(q, s);
     if (s.fused) {
         HIP_OK(hipSetDevice(device));
         (void)fused_tables();
@@ -185,7 +186,8 @@ void Engine::ensure_sinc_table() {
     forbid_in_nosync("build the sinc table");
     // cuSincOverSamplerR2R table (cuSincOverSampler.cu:21-80, constants cuSincOverSampler.h:27-57)
     const double beta = 0.75, relfiltlen = 6.0, pedestal = 0.0, PI = 3.14159265359;
-    sinc_len = int(relfiltlen / beta + 0.5);
+    const int sinc_len = int(relfiltlen / beta + 0.5);
+    static_assert(int(6.0 / 0.75 + 0.5) == SincTable::TAPS, "taps of the interpolation kernels");
     sinc_dec = 4096;
     const int ncoef = sinc_len * sinc_dec;
     const double wgthgt = (1.0 - pedestal) / 2.0, soff = (ncoef - 1.0) / 2.0;
@@ -613,12 +615,15 @@ void Engine::run_staged_t(const RunArgs &a) {
                                th, sspec, sh, NL, L, rq, T(1.0 / double(L)));
         hipLaunchKernelGGL(k_lagrows_real<T>, dim3(idivup(n * NL, g)), dim3(256), lds, st, rq, n * NL, g, d, NLw, out);
     };
-    // the 16-sparse surface kernel needs no 256x256 buffers
-    const bool fast_surface = !p.surf_method && Z == 16 && So == 256;
-    cx<T> *c_surf_in = fast_surface ? nullptr : buf<cx<T>>(tn + "c_surf_in", size_t(nb) * Z * Z);
-    cx<T> *c_surf = fast_surface || p.surf_method ? nullptr : buf<cx<T>>(tn + "c_surf", size_t(nb) * So * So);
-    T *r_surf = fast_surface ? nullptr : buf<T>(tn + "r_surf", size_t(nb) * So * So);
-    T *r_adj = buf<T>(tn + "r_adj", size_t(nb) * Z * Z);
+    // the 16-sparse surface kernel and the sinc patch kernel keep no surface in HBM
+    // (190 windows of 256 at factor 32: 3.10 ms with 512 x 512 surfaces transformed and
+    // searched in HBM, 2.04 ms without; an FP64 G[16][SO] fits a workgroup's LDS up to
+    // factor 32, and factor 1 leaves nothing to interpolate)
+    const bool fast_surface = !p.surf_method && Z == 16 && p.surf_ovs >= 2 && p.surf_ovs <= 32;
+    const bool full_surface = !p.surf_method && !fast_surface;
+    cx<T> *c_surf_in = full_surface ? buf<cx<T>>(tn + "c_surf_in", size_t(nb) * Z * Z) : nullptr;
+    cx<T> *c_surf = full_surface ? buf<cx<T>>(tn + "c_surf", size_t(nb) * So * So) : nullptr;
+    T *r_surf = full_surface ? buf<T>(tn + "r_surf", size_t(nb) * So * So) : nullptr;
     if (p.surf_method) ensure_sinc_table();
 
     // windows from a.fine_from on have their coarse zoom start and shift given
@@ -717,27 +722,32 @@ void Engine::run_staged_t(const RunArgs &a) {
         // trim + surface oversampling + argmax + sub-pixel offset (cuAmpcorChunk.cpp:169-207)
         float *mf = a.margin_fine ? a.margin_fine + w0 : nullptr;
         const float ratio = 1.0f / float(p.surf_ovs * p.raw_ovs);
+        float *off = a.offset + 2 * size_t(w0);
         if (fast_surface) {
-            // 16-sparse spectrum: one kernel instead of trim, FFT, pad, 256x256 FFT, real part, argmax
-            const size_t lds = sizeof(cx<T>) * (2 * 256 + 16 * 256);
-            hipLaunchKernelGGL(k_surface<T>, dim3(n), dim3(256), lds, st, corr_os, sz.os_corr_h, sz.os_corr_w,
-                               start, p.hs_down, p.hs_across, ratio, static_cast<const cx<T> *>(plan(256).tw(T())),
-                               zidx, mf, a.offset + 2 * size_t(w0));
+            // 16-sparse spectrum: one kernel instead of trim, FFT, pad, inverse FFT, real part, argmax
+            const int M = p.surf_ovs;
+            const cx<T> *tw = static_cast<const cx<T> *>(plan(So).tw(T()));
+            const size_t lds = sizeof(cx<T>) * surface_cx(M);
+            if (M <= 16)
+                hipLaunchKernelGGL((k_surface<T, 256>), dim3(n), dim3(256), lds, st, corr_os, sz.os_corr_h, sz.os_corr_w, M,
+                                   start, p.hs_down, p.hs_across, ratio, tw, zidx, mf, off);
+            else
+                hipLaunchKernelGGL((k_surface<T, 512>), dim3(n), dim3(512), lds, st, corr_os, sz.os_corr_h, sz.os_corr_w, M,
+                                   start, p.hs_down, p.hs_across, ratio, tw, zidx, mf, off);
+        } else if (p.surf_method) {
+            // patch rows interpolated at a time: up to 64 KB of FP64 values
+            const int cap = std::max(1, std::min(4 * p.surf_ovs + 1, 65536 / (8 * Z)));
+            hipLaunchKernelGGL(k_sinc_peak<T>, dim3(n), dim3(256), size_t(cap) * Z * 8, st, corr_os, sz.os_corr_h,
+                               sz.os_corr_w, Z, So, start, shift, SincTable{sinc_table.as<float>(), sinc_dec}, p.surf_ovs,
+                               p.surf_ovs * p.raw_ovs, cap, p.hs_down, p.hs_across, ratio, zidx, mf, off);
         } else {
-            if (p.surf_method) {
-                hipLaunchKernelGGL(k_trim_real<T>, grid2(Z * Z, n), dim3(256), 0, st, corr_os, sz.os_corr_h,
-                                   sz.os_corr_w, r_adj, Z);
-                hipLaunchKernelGGL(k_sinc<T>, dim3(1, n), dim3(256), 0, st, r_adj, Z, r_surf, So, shift,
-                                   p.surf_ovs * p.raw_ovs, sinc_table.as<float>(), p.surf_ovs, sinc_dec, sinc_len);
-            } else {
-                hipLaunchKernelGGL(k_trim_complex<T>, grid2(Z * Z, n), dim3(256), 0, st, corr_os, sz.os_corr_h,
-                                   sz.os_corr_w, c_surf_in, Z);
-                fft2<T, +1>(*this, c_surf_in, n, Z, Z, st);
-                fft2_quad<T, -1, 2>(*this, c_surf_in, n, Z, Z, c_surf, So, So, r_surf, st);
-            }
+            hipLaunchKernelGGL(k_trim_complex<T>, grid2(Z * Z, n), dim3(256), 0, st, corr_os, sz.os_corr_h, sz.os_corr_w,
+                               c_surf_in, Z);
+            fft2<T, +1>(*this, c_surf_in, n, Z, Z, st);
+            fft2_quad<T, -1, 2>(*this, c_surf_in, n, Z, Z, c_surf, So, So, r_surf, st);
             hipLaunchKernelGGL(k_maxloc<T>, dim3(n), dim3(256), 0, st, r_surf, So, So, zidx, (T *)nullptr, mf);
             hipLaunchKernelGGL(k_subpixel, dim3(idivup(n, 64)), dim3(64), 0, st, start, zidx, n, ratio, p.hs_down,
-                               p.hs_across, a.offset + 2 * size_t(w0));
+                               p.hs_across, off);
         }
         if (a.refined)
             hipLaunchKernelGGL(k_refine<T>, dim3(n), dim3(64), refine_lds(Z), st, corr_os, sz.os_corr_h, sz.os_corr_w,
@@ -1002,7 +1012,7 @@ void Engine::run(const RunArgs &in) {
     if (a.refined && (p.surf_method != 0 || sz.zoom > 64))
         throw Error(AMPCOR_E_UNSUPPORTED, "the FP64 peak refinement needs FFT surface oversampling and a zoom "
                                           "window of at most 64");
-    const bool fused = (a.mode == AMPCOR_MODE_FUSED) || (a.mode == AMPCOR_MODE_AUTO && sz.fused);
+    const bool fused = (a.mode == AMPCOR_MODE_FUSED) || (a.mode == AMPCOR_MODE_AUTO && fused_auto);
     if (a.mode == AMPCOR_MODE_FUSED && !sz.fused)
         throw Error(AMPCOR_E_UNSUPPORTED, "the fused kernels do not cover this configuration");
     if (a.ref_h < p.window_h || a.ref_w < p.window_w || a.sec_h < sz.search_h || a.sec_w < sz.search_w)

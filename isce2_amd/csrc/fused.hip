@@ -400,22 +400,26 @@ __global__ void __launch_bounds__(NTH, (R1 * R2 == 64 && MEAN) ? 8 : 1) k_oversa
 // split together and the per-bin sums run over all template rows in one pass.
 // ---------------------------------------------------------------------------
 
+// complex values the surface stage holds: G[16][SO], the 16 x 16 spectrum, e^{-2 pi i k/SO}
+__host__ __device__ constexpr int surface_units(int SO) { return 16 * SO + 256 + SO; }
+
 struct FineLds {
     int spec, tchunk, nrm, corr, red, total, y_off;
-    __host__ __device__ FineLds(int P, int NL, int T) {
+    // SO: surface side (16 x the surface oversampling factor)
+    __host__ __device__ FineLds(int P, int NL, int T, int SO) {
         const int L = P, PP = L + 1, H = L / 2;
         const int nS = P / 2;
         y_off = (NL * H + 1) & ~1;
         int s_units = nS * PP;
         const int npair = (NL + 1) / 2;
         if (y_off + npair * PP > s_units) s_units = y_off + npair * PP;
-        if (s_units < 16 * 256) s_units = 16 * 256;            // surface G[16][256]
-        int t_units = (T / 2) * PP;                           // template row spectra
-        if (t_units < 2 * 256) t_units = 2 * 256;             // 16x16 surface + twiddles
+        const int t_units = (T / 2) * PP;                     // template row spectra
         spec = 0;
         tchunk = al16(s_units * 8);
-        nrm = al16(tchunk + t_units * 8);
-        corr = al16(nrm + NL * NL * 4);
+        // the surface's G[16][SO], 16x16 spectrum and twiddles reuse both regions
+        const int chips = tchunk + t_units * 8, surf = surface_units(SO) * 8;
+        nrm = al16(chips > surf ? chips : surf);
+        corr = al16(nrm + (NL * NL > SO ? NL * NL : SO) * 4);   // the column list of the surface reuses nrm
         red = al16(corr + NL * NL * 4);
         total = red + 64 * 8;          // block sums + workgroup argmax scratch (up to 1024 threads)
     }
@@ -427,32 +431,58 @@ struct FineArgs {
     const int32_t *start;
     int hs_d, hs_a;
     float ratio;                               // 1/(surf_ovs*raw_ovs)
-    const cf *tw256;                           // e^{-2 pi i k/256}
+    int ovs;                                   // surface oversampling factor
+    const cf *tws;                             // e^{-2 pi i k/(16 ovs)} (FFT surface)
+    SincTable sinc;                            // windowed-sinc surface
+    const int32_t *shift;
     int32_t *zoom_idx; float *offset;
     float *margin;                             // [n] top-1 minus top-2 of the surface, or null
     float *surf;                               // [n][16][16] trimmed surface for the FP64 refinement, or null
 };
 
+// the surface's argmax over the workgroup -> zoom index, offset, margin
+template <int NTH>
+__device__ __forceinline__ void fine_peak(const FineArgs &a, Top2<float> &top, int SO, double *red, int win) {
+    // red: [0, 16) block sums, then NTH/64 top-1 values, runner-up values and keys
+    top.reduce<NTH>(reinterpret_cast<float *>(red + 16), reinterpret_cast<float *>(red + 16) + 16,
+                    reinterpret_cast<uint64_t *>(red + 32));
+    if (threadIdx.x == 0) {
+        const int idx = top.index();
+        const int px = idx / SO, py = idx % SO;
+        a.zoom_idx[2 * win] = px;
+        a.zoom_idx[2 * win + 1] = py;
+        a.offset[2 * win] = a.ratio * float(px) + float(a.start[2 * win]) - float(a.hs_d);
+        a.offset[2 * win + 1] = a.ratio * float(py) + float(a.start[2 * win + 1]) - float(a.hs_a);
+        if (a.margin) a.margin[win] = top.margin();
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Surface stage of the fine kernels: trimmed 16x16 normalized surface (corr,
-// row pitch NL) -> 16x16 +i DFT -> 16-sparse spectrum G[16][256] -> column
+// row pitch NL) -> 16x16 +i DFT -> 16-sparse spectrum G[16][SO] -> column
 // bounds -> evaluation of the kept columns with 16-point DFTs -> argmax with the
-// reference tie rule -> zoom index, offset, margin. LDS: G (16*256 cf), abuf
-// (512 cf: the 16x16 spectrum and 256 twiddles), cols (256 ints), red (64 doubles).
+// reference tie rule -> zoom index, offset, margin. SO = 16 M for a surface
+// oversampling factor M; with p = M a + b, q = M c + d and signed bins ks,
+//   G[k1][M c + d]  = DFT16_k2( A[k1][k2] e^{-2 pi i d ks2/SO} )[c]
+//   out[M a + b][q] = Re DFT16_k1( G[k1][q] e^{-2 pi i b ks1/SO} )[a].
+// OVS: M when known at compile time, 0 to take it from the arguments (2..32).
+// LDS: G (16*SO cf), abuf (256 + SO cf: the 16x16 spectrum and the twiddles),
+// cols (SO ints), red (64 doubles).
 // ---------------------------------------------------------------------------
-template <int NTH>
+template <int NTH, int OVS>
 __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *corr, int NL, cf *G, cf *abuf, int *cols,
                                              double *red, int win) {
-    constexpr int Z = 16, SO = 256;
+    constexpr int Z = 16;
+    const int M = OVS ? OVS : a.ovs, SO = 16 * M;
     // trimmed 16x16 surface -> 2-D +i DFT / 256 (cuOverSampler.cpp:141-145)
     cf *a16 = abuf;          // [16][16]
-    cf *tws = abuf + 256;    // e^{-2 pi i k/256}
+    cf *tws = abuf + 256;    // e^{-2 pi i k/SO}
     for (int i = threadIdx.x; i < Z * Z; i += NTH) {
         const int r = i / Z, c = i - r * Z;
         a16[i] = {corr[r * NL + c] * (1.0f / 256.0f), 0.f};
         if (a.surf) a.surf[size_t(win) * Z * Z + i] = corr[r * NL + c];
     }
-    for (int i = threadIdx.x; i < SO; i += NTH) tws[i] = a.tw256[i];
+    for (int i = threadIdx.x; i < SO; i += NTH) tws[i] = a.tws[i];
     __syncthreads();
     if (threadIdx.x < 16) {
         cf x[16];
@@ -472,18 +502,18 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
         for (int r = 0; r < 16; ++r) a16[r * 16 + threadIdx.x] = x[r];
     }
     __syncthreads();
-    // G[k1][16c+dd] = DFT16_c( A[k1][k2] e^{-2 pi i dd ks2/256} ), ks2 = signed k2
-    if (threadIdx.x < 256) {
-        const int k1 = threadIdx.x >> 4, dd = threadIdx.x & 15;
+    // G[k1][Mc+dd] = DFT16_c( A[k1][k2] e^{-2 pi i dd ks2/SO} ), ks2 = signed k2 (|dd ks2| < SO / 2)
+    if (threadIdx.x < 16 * M) {
+        const int k1 = threadIdx.x / M, dd = threadIdx.x - k1 * M;
         cf x[16];
 #pragma unroll
         for (int k2 = 0; k2 < 16; ++k2) {
-            const int ks = k2 < 8 ? k2 : k2 - 16;
-            x[k2] = cmul(a16[k1 * 16 + k2], tws[(dd * ks + 4096) & 255]);
+            const int t = dd * (k2 < 8 ? k2 : k2 - 16);
+            x[k2] = cmul(a16[k1 * 16 + k2], tws[t < 0 ? t + SO : t]);
         }
         dft16<float, -1>(x);
 #pragma unroll
-        for (int c = 0; c < 16; ++c) G[k1 * SO + 16 * c + dd] = x[c];
+        for (int c = 0; c < 16; ++c) G[k1 * SO + M * c + dd] = x[c];
     }
     __syncthreads();
     // Column pruning. Every value of surface column q is at most
@@ -493,7 +523,8 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
     // value within 2^-12 |a|max of it (the slack covers FP32 rounding many times
     // over): it is skipped, which leaves the argmax, the tie rule and every
     // margin below 2^-12 |a|max unchanged. NaN bounds keep their column.
-    static_assert(NTH >= SO, "one thread per surface column for the bounds");
+    static_assert(NTH >= 512 && OVS <= 32, "one thread per surface column for the bounds");
+    constexpr int NBW = OVS ? (16 * OVS + 63) / 64 : 8;         // waves that hold columns
     float amax = -FLT_MAX, amag = 0.f;
     for (int i = threadIdx.x & 63; i < Z * Z; i += 64) {
         const float v = corr[(i / Z) * NL + (i % Z)];
@@ -505,7 +536,7 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
         amax = fmaxf(amax, __shfl_xor(amax, o));
         amag = fmaxf(amag, __shfl_xor(amag, o));
     }
-    uint64_t *masks = reinterpret_cast<uint64_t *>(red + 48);   // ballots of the SO/64 bound waves
+    uint64_t *masks = reinterpret_cast<uint64_t *>(red + 48);   // ballots of the bound waves
     bool keep = false;
     if (threadIdx.x < SO) {
         float bq = 0.f;
@@ -517,27 +548,27 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
         keep = !(bq * (1.0f + 0x1p-10f) + 0x1p-11f * amag < amax);
     }
     const uint64_t wm = __ballot(keep);
-    if (threadIdx.x < SO && (threadIdx.x & 63) == 0) masks[threadIdx.x >> 6] = wm;
+    if (threadIdx.x < 64 * NBW && (threadIdx.x & 63) == 0) masks[threadIdx.x >> 6] = wm;
     __syncthreads();
     int ncols = 0, before = 0;
 #pragma unroll
-    for (int w = 0; w < SO / 64; ++w) {
+    for (int w = 0; w < NBW; ++w) {
         const int c = __popcll(masks[w]);
         if (w < (threadIdx.x >> 6)) before += c;
         ncols += c;
     }
     if (keep) cols[before + __popcll(wm & ((uint64_t(1) << (threadIdx.x & 63)) - 1))] = threadIdx.x;
     __syncthreads();
-    // out[16aa+b][q] = Re DFT16_aa( G[k1][q] e^{-2 pi i b ks1/256} ) over the kept
+    // out[Maa+b][q] = Re DFT16_aa( G[k1][q] e^{-2 pi i b ks1/SO} ) over the kept
     // columns q; task t = (b, column list entry); running argmax
     Top2<float> top;
     #pragma unroll 1
-    for (int t = threadIdx.x; t < 16 * ncols; t += NTH) {
+    for (int t = threadIdx.x; t < M * ncols; t += NTH) {
         const int b = t / ncols, qq = cols[t - b * ncols];
-        // e^{-2 pi i b k/256} for k = 1..8 (negative bins use the conjugate)
+        // e^{-2 pi i b k/SO} for k = 1..8 (negative bins use the conjugate)
         cf w[9];
 #pragma unroll
-        for (int k = 1; k <= 8; ++k) w[k] = tws[(b * k) & 255];
+        for (int k = 1; k <= 8; ++k) w[k] = tws[b * k];
         cf x[16];
         x[0] = G[qq];
 #pragma unroll
@@ -547,33 +578,44 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
         }
         dft16<float, -1>(x);
 #pragma unroll
-        for (int aa = 0; aa < 16; ++aa) top.add_idx(x[aa].x, uint32_t((16 * aa + b) * SO + qq));
+        for (int aa = 0; aa < 16; ++aa) top.add_idx(x[aa].x, uint32_t((M * aa + b) * SO + qq));
     }
-    // red: [0, 16) block sums, then NTH/64 top-1 values, runner-up values and keys
-    top.reduce<NTH>(reinterpret_cast<float *>(red + 16), reinterpret_cast<float *>(red + 16) + 16,
-                    reinterpret_cast<uint64_t *>(red + 32));
-    if (threadIdx.x == 0) {
-        const int idx = top.index();
-        const int px = idx / SO, py = idx % SO;
-        a.zoom_idx[2 * win] = px;
-        a.zoom_idx[2 * win + 1] = py;
-        a.offset[2 * win] = a.ratio * float(px) + float(a.start[2 * win]) - float(a.hs_d);
-        a.offset[2 * win + 1] = a.ratio * float(py) + float(a.start[2 * win + 1]) - float(a.hs_a);
-        if (a.margin) a.margin[win] = top.margin();
-    }
+    fine_peak<NTH>(a, top, SO, red, win);
 }
 
-template <int T, int R1, int R2, int K, int NTH>
+// Windowed-sinc surface (cuSincOverSampler.cu:84-195) and its peak: the values of
+// the interpolated patch around the (shifted) centre, zero elsewhere, are never
+// stored. LDS: R (size * 16 doubles, size = 4 ovs + 1), corr as in fine_surface.
+template <int NTH>
+__device__ __forceinline__ void fine_sinc(const FineArgs &a, const float *corr, int NL, double *R, double *red, int win) {
+    constexpr int Z = 16;
+    const int SO = Z * a.ovs;
+    if (a.surf)
+        for (int i = threadIdx.x; i < Z * Z; i += NTH) a.surf[size_t(win) * Z * Z + i] = corr[(i / Z) * NL + i % Z];
+    Top2<float> top;
+    sinc_patch_peak<NTH>([&](int x, int y) { return corr[x * NL + y]; }, Z, SO, a.shift[2 * win], a.shift[2 * win + 1], a.sinc,
+                         a.ovs, 2 * a.ovs, R, 4 * a.ovs + 1, top);
+    fine_peak<NTH>(a, top, SO, red, win);
+}
+
+// the surface stage by kind: SURF = 16 (FFT, factor 16), 0 (FFT, any factor of 2..32), -1 (windowed sinc)
+template <int NTH, int SURF>
+__device__ __forceinline__ void fine_finish(const FineArgs &a, const float *corr, int NL, cf *work, int *cols, double *red,
+                                            int win) {
+    if constexpr (SURF < 0) fine_sinc<NTH>(a, corr, NL, reinterpret_cast<double *>(work), red, win);
+    else fine_surface<NTH, SURF>(a, corr, NL, work, work + 256 * (SURF ? SURF : a.ovs), cols, red, win);
+}
+
+template <int T, int R1, int R2, int K, int NTH, int SURF>
 __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int P = R1 * R2, L = P, PP = L + 1, H = L / 2, nS = P / 2;
     constexpr int NL = P - T + 1;      // 17
     constexpr int Z = NL - 1;          // 16 (trimmed surface)
-    constexpr int SO = 256;            // oversampled surface side
     static_assert(Z == 16, "fused surface stage assumes a 16x16 zoom surface");
     // mac_rows reads up to K - 2 rows past the search; the template spectra follow it
     static_assert(T / 2 >= K / 2 + 1, "the template region follows the search rows");
-    const FineLds lay(P, NL, T);
+    const FineLds lay(P, NL, T, SURF > 0 ? 16 * SURF : 16 * a.ovs);
     cf *S = reinterpret_cast<cf *>(smem + lay.spec);
     cf *Tb = reinterpret_cast<cf *>(smem + lay.tchunk);
     float *nrm = reinterpret_cast<float *>(smem + lay.nrm);
@@ -648,7 +690,7 @@ __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) 
     __syncthreads();
     inverse_lags<R1, R2, NTH>(Qs, NL, NL, S + lay.y_off, PP, tw, nrm, corr);
 
-    fine_surface<NTH>(a, corr, NL, S, Tb, reinterpret_cast<int *>(nrm), red, win);
+    fine_finish<NTH, SURF>(a, corr, NL, S, reinterpret_cast<int *>(nrm), red, win);
 }
 
 // ---------------------------------------------------------------------------
@@ -661,21 +703,23 @@ __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) 
 // ---------------------------------------------------------------------------
 struct Fine2Lds {
     int sr, tb, save, nrm, corr, red, tw, total;   // bytes
-    __host__ __device__ Fine2Lds(int P, int NL, int TC) {
+    __host__ __device__ Fine2Lds(int P, int NL, int TC, int SO) {
         const int PP = P + 1;
         const int srp = (TC + NL - 1 + 1) / 2, tcp = TC / 2;
         sr = 0;
         tb = sr + srp * PP * 8;                    // template pairs directly after the search pairs
         save = tb + tcp * PP * 8;
-        nrm = al16(save + 2 * (NL - 1) * P * 4);
-        corr = al16(nrm + NL * NL * 4);
+        // the surface stage reuses everything below nrm, and its column list nrm itself
+        const int chips = save + 2 * (NL - 1) * P * 4, surf = surface_units(SO) * 8;
+        nrm = al16(chips > surf ? chips : surf);
+        corr = al16(nrm + (NL * NL > SO ? NL * NL : SO) * 4);
         red = al16(corr + NL * NL * 4);
         tw = red + 64 * 8;                         // the row transform's twiddles
         total = tw + P * 8;
     }
 };
 
-template <int T, int R1, int R2, int K, int NTH, int TC>
+template <int T, int R1, int R2, int K, int NTH, int TC, int SURF>
 __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, int w0) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int P = R1 * R2, L = P, PP = L + 1, H = L / 2;
@@ -693,7 +737,7 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
     static_assert(TCP >= K / 2 + 1, "the template chunk follows the search rows");
     static_assert(3 * P <= NTH, "one thread per column and row-pair phase");
     static_assert(6 * P * 8 <= (TC / 2) * (P + 1) * 8, "column-sum partials fit the template chunk region");
-    const Fine2Lds lay(P, NL, TC);
+    const Fine2Lds lay(P, NL, TC, SURF > 0 ? 16 * SURF : 16 * a.ovs);
     cf *SR = reinterpret_cast<cf *>(smem + lay.sr);
     cf *TB = reinterpret_cast<cf *>(smem + lay.tb);
     float *save = reinterpret_cast<float *>(smem + lay.save);   // rows [0, NS) then [T, T + NS), pitch P
@@ -826,7 +870,7 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
         [&](int r, int c) -> double { return double(r < NS ? save[r * P + c] : save[(NS + r - T) * P + c]); },
         part, 3, P, T, T, NL, NL, t2, nrm);
     inverse_lags<R1, R2, NTH>(Qs, NL, NL, SR + ((NL * H + 1) & ~1), PP, tw, nrm, corr);
-    fine_surface<NTH>(a, corr, NL, SR, SR + 16 * 256, reinterpret_cast<int *>(nrm), red, win);
+    fine_finish<NTH, SURF>(a, corr, NL, SR, reinterpret_cast<int *>(nrm), red, win);
 }
 
 // ---------------------------------------------------------------------------
@@ -852,12 +896,23 @@ void launch_coarse(int K, const CoarseArgs &a, const cf *tw, int n, int w0, size
     }
 }
 
+// k_fine2 for the surfaces other than factor 16 by the FFT
+void launch_fine2(int surf, const FineArgs &a, const cf *tw, int n, int w0, size_t lds, hipStream_t st) {
+    if (surf == 0) hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, 0>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+    else hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, -1>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+}
+
 }  // namespace fused
 
-bool fused_supported(const ampcor_params &p, const ampcor_sizes &s) {
+// Surface oversampling factors the fused kernels evaluate: 2..32 (FFT: one thread
+// per surface column of a 512-thread workgroup; sinc: the patch's rows fit in LDS).
+// Factor 1 and above 32 stay with the staged pipeline. 3,844 windows of 64, half
+// search 20, factor 32: staged 11.8 ms, fused 1.36 ms; 900 with the sinc surface:
+// staged 1.96 ms, fused 0.55 ms.
+bool fused_fits(const ampcor_params &p, const ampcor_sizes &s) {
     using namespace fused;
     if (p.window_h != p.window_w || (p.window_h != 32 && p.window_h != 64)) return false;
-    if (p.raw_ovs != 2 || s.zoom != 16 || p.surf_ovs != 16 || p.surf_method != 0) return false;
+    if (p.raw_ovs != 2 || s.zoom != 16 || p.surf_ovs < 2 || p.surf_ovs > 32) return false;
     const int L = coarse_L(s.search_w);
     if (L == 0) return false;
     if (pick_k(s.raw_corr_h, NT / (L / 2)) == 0) return false;
@@ -865,8 +920,12 @@ bool fused_supported(const ampcor_params &p, const ampcor_sizes &s) {
     // the window sums' block sums (doubles) live in the template chunk's region (cf)
     if (2 * ((s.search_h + NORM_BLK - 1) / NORM_BLK) * s.search_w > coarse_tc(p.window_w) / 2 * (L + 1)) return false;
     const int P = 2 * s.zoom_in_w;
-    if (FineLds(P, P - 2 * p.window_w + 1, 2 * p.window_w).total > 160 * 1024) return false;
+    if (FineLds(P, P - 2 * p.window_w + 1, 2 * p.window_w, s.surf_out).total > 160 * 1024) return false;
     return true;
+}
+
+bool fused_supported(const ampcor_params &p, const ampcor_sizes &s) {
+    return p.surf_ovs == 16 && p.surf_method == 0 && fused_fits(p, s);
 }
 
 // Tables the fused kernels read (twiddles, half-sample shifts). Built on first
@@ -902,8 +961,9 @@ FusedTables Engine::fused_tables() {
     t.twW = tw(W);
     t.twZ = tw(Zc);
     t.tw2 = tw(2 * Zc);
-    t.tw256 = tw(256);
-    t.tw256_64 = plan(256).tw64.ptr;
+    t.tws = tw(sz.surf_out);
+    t.tws_64 = plan(sz.surf_out).tw64.ptr;
+    if (p.surf_method) ensure_sinc_table();
     return t;
 }
 
@@ -917,9 +977,9 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
     const int L1 = coarse_L(sz.search_w);
     const int K1 = pick_k(sz.raw_corr_h, NT / (L1 / 2));
     const int mode = p.image_complex ? (p.deramp == 0 ? 1 : 0) : 2;
+    const int surf = p.surf_method ? -1 : (p.surf_ovs == 16 ? 16 : 0);   // surface stage (fine_finish)
     const cf *tw1 = static_cast<const cf *>(tb.tw1), *twW = static_cast<const cf *>(tb.twW);
     const cf *twZ = static_cast<const cf *>(tb.twZ), *tw2 = static_cast<const cf *>(tb.tw2);
-    const cf *tw256 = static_cast<const cf *>(tb.tw256);
     const cf *h_ref = static_cast<const cf *>(tb.h_ref), *h_zoom = static_cast<const cf *>(tb.h_zoom);
     float *tamp = c.tamp - size_t(w0) * T2 * T2;          // indexed by absolute window inside the kernels
     double *tmean = c.tmean - 2 * size_t(w0);
@@ -930,8 +990,8 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                   c.loc, c.val, c.start, c.shift, c.snr, c.cov, c.mc};
     const size_t lds_c = CoarseLds(W, L1, sz.search_h, sz.raw_corr_h, sz.raw_corr_w).total;
     const size_t lds_or = os_lds_bytes(W), lds_oz = os_lds_bytes(Zc);
-    const size_t lds_f = FineLds(P, P - T2 + 1, T2).total;
-    const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32).total;
+    const size_t lds_f = FineLds(P, P - T2 + 1, T2, sz.surf_out).total;
+    const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32, sz.surf_out).total;
     {
         timed("k_coarse", n, st, [&] {
             if (W == 64) launch_coarse<64, 8, 16>(K1, ca, tw1, n, w0, lds_c, st);
@@ -941,7 +1001,8 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
         OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, h_ref, tamp, tmean};
         OsArgs osec{c.sec, c.sec_pitch, mode, c.sec_d, c.sec_a, c.start, p.deramp, h_zoom, samp, nullptr};
         FineArgs fa{tamp, tmean, samp, c.start, p.hs_down, p.hs_across, 1.0f / float(p.surf_ovs * p.raw_ovs),
-                    tw256, c.zidx, c.offset, c.mf, c.surf ? c.surf - size_t(w0) * 256 : nullptr};
+                    p.surf_ovs, static_cast<const cf *>(tb.tws), SincTable{sinc_table.as<float>(), sinc_dec}, c.shift,
+                    c.zidx, c.offset, c.mf, c.surf ? c.surf - size_t(w0) * 256 : nullptr};
         if (W == 64) {
             timed("k_oversample_ref", n, st, [&] {
                 hipLaunchKernelGGL((k_oversample<8, 8, true>), dim3(n), dim3(NT), lds_or, st, oref, twW, w0);
@@ -950,12 +1011,15 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                 hipLaunchKernelGGL((k_oversample<8, 9, false>), dim3(n), dim3(NT), lds_oz, st, osec, twZ, w0);
             });
             timed("k_fine", n, st, [&] {
-                if (fine_kernel == 2)
-                    hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32>), dim3(n), dim3(NT), lds_f2, st, fa, tw2, w0);
+                // the whole-template kernel is built for the surfaces AMPCOR_MODE_FUSED accepts
+                if (surf != 16)
+                    launch_fine2(surf, fa, tw2, n, w0, lds_f2, st);
+                else if (fine_kernel == 2)
+                    hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, 16>), dim3(n), dim3(NT), lds_f2, st, fa, tw2, w0);
                 else if (fine_threads == 1024)
-                    hipLaunchKernelGGL((k_fine<128, 9, 16, 2, 1024>), dim3(n), dim3(1024), lds_f, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine<128, 9, 16, 2, 1024, 16>), dim3(n), dim3(1024), lds_f, st, fa, tw2, w0);
                 else
-                    hipLaunchKernelGGL((k_fine<128, 16, 9, 3, NT>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine<128, 16, 9, 3, NT, 16>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
             });
         } else {
             timed("k_oversample_ref", n, st, [&] {
@@ -965,14 +1029,19 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                 hipLaunchKernelGGL((k_oversample<8, 5, false>), dim3(n), dim3(NT), lds_oz, st, osec, twZ, w0);
             });
             timed("k_fine", n, st, [&] {
-                hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                if (surf == 16)
+                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, 16>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                else if (surf == 0)
+                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, 0>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                else
+                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, -1>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
             });
         }
         if (c.refined)
             hipLaunchKernelGGL(k_refine<float>, dim3(n), dim3(64), refine_lds(16), st, c.surf, 16, 16, 16,
                                p.surf_ovs, 1.0 / double(p.surf_ovs * p.raw_ovs), c.zidx + 2 * size_t(w0),
                                c.start + 2 * size_t(w0), p.hs_down, p.hs_across,
-                               static_cast<const cx<double> *>(tb.tw256_64), c.refined + 2 * size_t(w0));
+                               static_cast<const cx<double> *>(tb.tws_64), c.refined + 2 * size_t(w0));
         HIP_OK(hipGetLastError());
     }
 }

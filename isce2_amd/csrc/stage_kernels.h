@@ -1059,83 +1059,157 @@ __global__ void k_trim_complex(const T *in, int ih, int iw, cx<T> *out, int z) {
     }
 }
 
-template <class T>
-__global__ void k_trim_real(const T *in, int ih, int iw, T *out, int z) {
-    const int win = blockIdx.y;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < z * z; i += gridDim.x * blockDim.x) {
-        const int r = i / z, c = i - r * z;
-        out[size_t(win) * z * z + i] = in[size_t(win) * ih * iw + r * iw + c];
+// table of the windowed-sinc surface interpolation: taps * dec coefficients
+// (cuSincOverSampler.cu:21-80), TAPS taps of dec phases each
+struct SincTable {
+    static constexpr int TAPS = 8;
+    const float *coef;
+    int dec;
+};
+
+// Windowed-sinc surface oversampling (cuSincOverSampler.cu:84-195) and its argmax.
+// The reference writes a (2*2*covs+1)^2 patch around out/2 + shift*factor into a
+// zeroed nout x nout surface and searches all of it; here only the patch is
+// evaluated (the weights separate: R[i][y] interpolates along x for `cap` patch
+// rows at a time, then each thread keeps one patch column's weights and walks the
+// rows) and the zeros enter the argmax as one candidate, the zero that the tie
+// rule prefers, and one runner-up. Sums in FP64. a(x, y): the nin x nin trimmed
+// surface. Every thread of the workgroup calls it; the caller reduces `top`.
+template <int NTH, class T, class A>
+__device__ __forceinline__ void sinc_patch_peak(A a, int nin, int nout, int shift0, int shift1, SincTable tb, int covs,
+                                                int factor, double *R, int cap, Top2<T> &top) {
+    constexpr int TAPS = SincTable::TAPS;
+    const int rng = 2 * covs;
+    const int x0 = nout / 2 - rng + shift0 * factor, y0 = nout / 2 - rng + shift1 * factor;
+    const int size = min(2 * rng + 1, nout);           // distinct positions per axis
+    auto wrap = [&](int o) { return o >= nout ? o - nout : o; };
+    // integer part and phase of an output position, as the reference computes them
+    auto split = [&](int o, int &i, int &f) {
+        i = o / covs;
+        f = int((float(o) / covs - i) * tb.dec);
+    };
+    auto tap = [&](int i, int p) {
+        int x = i - p + TAPS / 2;
+        if (x < 0) x += nin;
+        if (x >= nin) x -= nin;
+        return x;
+    };
+    const int lanes = min(size, NTH), groups = NTH / lanes;
+    const int jt = threadIdx.x % lanes, g = threadIdx.x / lanes;
+    for (int i0 = 0; i0 < size; i0 += cap) {
+        const int ni = min(cap, size - i0);
+        for (int t = threadIdx.x; t < ni * nin; t += NTH) {
+            const int i = t / nin, y = t - i * nin;
+            int xi, xf;
+            split(wrap(x0 + i0 + i), xi, xf);
+            double acc = 0.0, ws = 0.0;
+#pragma unroll
+            for (int p = 0; p < TAPS; ++p) {
+                const double w = tb.coef[p * tb.dec + xf];
+                ws += w;
+                acc += w * double(a(tap(xi, p), y));
+            }
+            R[t] = acc / ws;
+        }
+        __syncthreads();
+        for (int j = jt; j < size && g < groups; j += lanes) {
+            const int oy = wrap(y0 + j);
+            int yi, yf, yy[TAPS];
+            double w[TAPS], ws = 0.0;
+            split(oy, yi, yf);
+#pragma unroll
+            for (int q = 0; q < TAPS; ++q) {
+                w[q] = tb.coef[q * tb.dec + yf];
+                ws += w[q];
+                yy[q] = tap(yi, q);
+            }
+#pragma unroll
+            for (int q = 0; q < TAPS; ++q) w[q] /= ws;
+            for (int i = g; i < ni; i += groups) {
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < TAPS; ++q) acc += w[q] * R[i * nin + yy[q]];
+                top.add(T(acc), maxloc_key(uint32_t(wrap(x0 + i0 + i) * nout + oy)));
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && size < nout) {
+        // the zeros outside the patch: the first in the tie rule's order, and another
+        auto inside = [&](int o, int s) { return (o - s + nout) % nout < size; };
+        const int n = nout * nout, s0 = wrap(x0), s1 = wrap(y0);
+        for (uint32_t r = 0; r < 512; ++r) {
+            int idx = int(bitrev9(r));
+            while (idx < n && inside(idx / nout, s0) && inside(idx % nout, s1)) idx += 512;
+            if (idx < n) {
+                top.add(T(0), maxloc_key(uint32_t(idx)));
+                top.add(T(0), (uint64_t(511) << 32) | 0xffffffffu);
+                break;
+            }
+        }
     }
 }
 
-// windowed-sinc surface oversampling (cuSincOverSampler.cu:84-195): zero output,
-// then the (2*2*covs+1)^2 patch around out/2 + shift*factor
+// windowed-sinc surface, argmax and sub-pixel offset of the top-left nin x nin of
+// corr ([n][ch][cw]); one 256-thread block per window; LDS: cap * nin doubles
 template <class T>
-__global__ void k_sinc(const T *in, int nin, T *out, int nout, const int32_t *shift, int factor,
-                       const float *filt, int covs, int dec, int intplength) {
-    const int win = blockIdx.y;
-    const int rng = 2 * covs, st = nout / 2 - rng, size = 2 * rng + 1;
-    T *o = out + size_t(win) * nout * nout;
-    const T *a = in + size_t(win) * nin * nin;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nout * nout; i += gridDim.x * blockDim.x) o[i] = T(0);
-    __syncthreads();   // same block writes zeros then values only for its own indices below
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < size * size; i += gridDim.x * blockDim.x) {
-        const int ix = i / size, iy = i - ix * size;
-        int ox = ix + st + shift[2 * win] * factor;
-        if (ox >= nout) ox -= nout;
-        int oy = iy + st + shift[2 * win + 1] * factor;
-        if (oy >= nout) oy -= nout;
-        const int xo = ox / covs, yo = oy / covs;
-        const int xf = int((float(ox) / covs - xo) * dec);
-        const int yf = int((float(oy) / covs - yo) * dec);
-        double acc = 0.0, wsum = 0.0;
-        for (int p = 0; p < intplength; ++p) {
-            int x = xo - p + intplength / 2;
-            if (x < 0) x += nin;
-            if (x >= nin) x -= nin;
-            const double wx = filt[p * dec + xf];
-            for (int q = 0; q < intplength; ++q) {
-                int y = yo - q + intplength / 2;
-                if (y < 0) y += nin;
-                if (y >= nin) y -= nin;
-                const double wgt = wx * double(filt[q * dec + yf]);
-                wsum += wgt;
-                acc += double(a[x * nin + y]) * wgt;
-            }
-        }
-        o[ox * nout + oy] = T(acc / wsum);
+__global__ void __launch_bounds__(256) k_sinc_peak(const T *corr, int ch, int cw, int nin, int nout, const int32_t *start,
+                                                   const int32_t *shift, SincTable tb, int covs, int factor, int cap,
+                                                   int hs_down, int hs_across, float ratio, int32_t *zidx, float *margin,
+                                                   float *offset) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ T shv[4], shv2[4];
+    __shared__ uint64_t shk[4];
+    const int win = blockIdx.x;
+    const T *c = corr + size_t(win) * ch * cw;
+    Top2<T> top;
+    sinc_patch_peak<256>([&](int x, int y) { return c[x * cw + y]; }, nin, nout, shift[2 * win], shift[2 * win + 1], tb, covs,
+                         factor, reinterpret_cast<double *>(smem_raw), cap, top);
+    top.template reduce<256>(shv, shv2, shk);
+    if (threadIdx.x == 0) {
+        const int idx = top.index(), px = idx / nout, py = idx - px * nout;
+        zidx[2 * win] = px;
+        zidx[2 * win + 1] = py;
+        offset[2 * win] = ratio * float(px) + float(start[2 * win]) - float(hs_down);
+        offset[2 * win + 1] = ratio * float(py) + float(start[2 * win + 1]) - float(hs_across);
+        if (margin) margin[win] = top.margin();
     }
 }
 
 // final offset (cuOffset.cu:137-146)
 // ---------------------------------------------------------------------------
-// 16x16 -> 256x256 surface oversampling (cuOverSampler.cpp:141-148, real part
-// cuArraysCopy.cu:326-339), argmax (cuOffset.cu:23-84) and sub-pixel offset
-// (cuOffset.cu:137-187) in one kernel, one 256-thread block per window. The
-// padded 256x256 spectrum has only 16x16 non-zero bins, so with p = 16a + b,
-// q = 16c + d and signed bins ks:
-//   G[k1][16c+d]   = DFT16_k2( A[k1][k2] e^{-2 pi i d ks2/256} )[c]
-//   out[16a+b][q]  = Re DFT16_k1( G[k1][q] e^{-2 pi i b ks1/256} )[a]
-// where A = (+i 2-D DFT of the trimmed patch) / 256. Needs zoom = 16 and a
-// surface oversampling factor of 16. LDS: (2*256 + 16*256) cx<T>.
+// 16x16 -> SO x SO surface oversampling, SO = 16 M (cuOverSampler.cpp:141-148, real
+// part cuArraysCopy.cu:326-339), argmax (cuOffset.cu:23-84) and sub-pixel offset
+// (cuOffset.cu:137-187) in one kernel, one NTH-thread block per window. The
+// padded SO x SO spectrum has only 16x16 non-zero bins, so with p = M a + b,
+// q = M c + d and signed bins ks:
+//   G[k1][Mc+d]   = DFT16_k2( A[k1][k2] e^{-2 pi i d ks2/SO} )[c]
+//   out[Ma+b][q]  = Re DFT16_k1( G[k1][q] e^{-2 pi i b ks1/SO} )[a]
+// where A = (+i 2-D DFT of the trimmed patch) / 256. Needs zoom = 16 and
+// 16 M <= NTH, M >= 2 (one thread per surface column). LDS: surface_cx(M) cx<T>.
 // ---------------------------------------------------------------------------
-template <class T>
-__global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, const int32_t *start, int hs_down,
-                                                 int hs_across, float ratio, const cx<T> *tw256, int32_t *zidx,
+// cx<T> values: G[16][SO], the twiddles (tws below), the 16x16 spectrum
+__host__ __device__ constexpr int surface_cx(int M) { return 256 + 16 * M + 256 * M; }
+
+template <class T, int NTH>
+__global__ void __launch_bounds__(NTH) k_surface(const T *corr, int ch, int cw, int M, const int32_t *start, int hs_down,
+                                                 int hs_across, float ratio, const cx<T> *tw, int32_t *zidx,
                                                  float *margin, float *offset) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *a16 = reinterpret_cast<cx<T> *>(smem_raw);
+    const int SO = 16 * M;
     cx<T> *tws = a16 + 256;
-    cx<T> *G = tws + 256;
-    __shared__ T shv[4], shv2[4];
-    __shared__ uint64_t shk[4];
+    cx<T> *G = tws + SO;
+    constexpr int NW = NTH / 64;
+    __shared__ T shv[NW], shv2[NW];
+    __shared__ uint64_t shk[NW];
     const int win = blockIdx.x;
     const T *c = corr + size_t(win) * ch * cw;
-    {
+    if (threadIdx.x < 256) {
         const int r = threadIdx.x >> 4, q = threadIdx.x & 15;
         a16[threadIdx.x] = {c[r * cw + q] * T(1.0 / 256.0), T(0)};
-        tws[threadIdx.x] = tw256[threadIdx.x];
     }
+    if (threadIdx.x < SO) tws[threadIdx.x] = tw[threadIdx.x];
     __syncthreads();
     if (threadIdx.x < 16) {
         cx<T> x[16];
@@ -1155,17 +1229,17 @@ __global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, 
         for (int r = 0; r < 16; ++r) a16[r * 16 + threadIdx.x] = x[r];
     }
     __syncthreads();
-    {
-        const int k1 = threadIdx.x >> 4, dd = threadIdx.x & 15;
+    if (threadIdx.x < SO) {
+        const int k1 = threadIdx.x / M, dd = threadIdx.x - k1 * M;
         cx<T> x[16];
 #pragma unroll
         for (int k2 = 0; k2 < 16; ++k2) {
-            const int ks = k2 < 8 ? k2 : k2 - 16;
-            x[k2] = cmul(a16[k1 * 16 + k2], tws[(dd * ks + 4096) & 255]);
+            const int t = dd * (k2 < 8 ? k2 : k2 - 16);         // |t| < SO / 2
+            x[k2] = cmul(a16[k1 * 16 + k2], tws[t < 0 ? t + SO : t]);
         }
         dft16<T, -1>(x);
 #pragma unroll
-        for (int cc = 0; cc < 16; ++cc) G[k1 * 256 + 16 * cc + dd] = x[cc];
+        for (int cc = 0; cc < 16; ++cc) G[k1 * SO + M * cc + dd] = x[cc];
     }
     __syncthreads();
     // Column pruning: every value of column q is at most B_q = sum_k1 |G[k1][q]|
@@ -1174,8 +1248,8 @@ __global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, 
     // < amax hold neither the argmax nor any value within 2^-12 |a|max of it, and
     // are skipped (argmax, tie rule and margins below that are unchanged; NaN
     // bounds keep their column).
-    __shared__ uint64_t masks[4];
-    __shared__ int cols[256];
+    __shared__ uint64_t masks[NW];
+    __shared__ int cols[NTH];
     T amax = -INFINITY, amag = T(0);
     for (int i = threadIdx.x & 63; i < 256; i += 64) {
         const T v = c[(i >> 4) * cw + (i & 15)];
@@ -1187,12 +1261,12 @@ __global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, 
         amax = fmax(amax, __shfl_xor(amax, o));
         amag = fmax(amag, __shfl_xor(amag, o));
     }
-    bool keep;
-    {
+    bool keep = false;
+    if (threadIdx.x < SO) {
         T bq = T(0);
 #pragma unroll
         for (int k1 = 0; k1 < 16; ++k1) {
-            const cx<T> g = G[k1 * 256 + threadIdx.x];
+            const cx<T> g = G[k1 * SO + threadIdx.x];
             bq += ampcor::amag(g);
         }
         keep = !(bq * T(1.0 + 0x1p-10) + T(0x1p-11) * amag < amax);
@@ -1202,7 +1276,7 @@ __global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, 
     __syncthreads();
     int ncols = 0, before = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
         const int n = __popcll(masks[w]);
         if (w < (threadIdx.x >> 6)) before += n;
         ncols += n;
@@ -1211,22 +1285,22 @@ __global__ void __launch_bounds__(256) k_surface(const T *corr, int ch, int cw, 
     __syncthreads();
     Top2<T> top;
     #pragma unroll 1
-    for (int t = threadIdx.x; t < 16 * ncols; t += 256) {
+    for (int t = threadIdx.x; t < M * ncols; t += NTH) {
         const int b = t / ncols, qq = cols[t - b * ncols];
         cx<T> x[16];
 #pragma unroll
         for (int k1 = 0; k1 < 16; ++k1) {
-            const int ks = k1 < 8 ? k1 : k1 - 16;
-            x[k1] = cmul(G[k1 * 256 + qq], tws[(b * ks + 4096) & 255]);
+            const int k = b * (k1 < 8 ? k1 : k1 - 16);
+            x[k1] = cmul(G[k1 * SO + qq], tws[k < 0 ? k + SO : k]);
         }
         dft16<T, -1>(x);
 #pragma unroll
-        for (int aa = 0; aa < 16; ++aa) top.add_idx(x[aa].x, uint32_t((16 * aa + b) * 256 + qq));
+        for (int aa = 0; aa < 16; ++aa) top.add_idx(x[aa].x, uint32_t((M * aa + b) * SO + qq));
     }
-    top.template reduce<256>(shv, shv2, shk);
+    top.template reduce<NTH>(shv, shv2, shk);
     if (threadIdx.x == 0) {
         const int idx = top.index();
-        const int px = idx >> 8, py = idx & 255;
+        const int px = idx / SO, py = idx - px * SO;
         zidx[2 * win] = px;
         zidx[2 * win + 1] = py;
         offset[2 * win] = ratio * float(px) + float(start[2 * win]) - float(hs_down);
