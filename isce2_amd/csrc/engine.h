@@ -47,7 +47,7 @@ struct Sizes {
 
 // Device tables the fused kernels read (FP32 twiddles, half-sample shifts).
 struct FusedTables {
-    const void *tw1, *twW, *twZ, *tw2, *tws, *h_ref, *h_zoom;
+    const void *tw1, *tw2, *tws, *tw_ref, *shift_ref, *tw_zoom, *shift_zoom;
     const void *tws_64;            // FP64 e^{-2 pi i k/surface side} (peak refinement)
 };
 

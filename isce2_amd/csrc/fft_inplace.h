@@ -266,4 +266,61 @@ __device__ __forceinline__ void fft_dr2nat(cx<T> *buf, int nsig, int ss, int es,
     __syncthreads();
 }
 
+// Half-sample interpolation of `nsig` signals of n = R1 * R2 samples held in LDS as
+// above, y = (1/n) FFT_-(FFT_+(x) e^{-i pi k_s/n}) with shift[k] = e^{-i pi k_s/n}/n,
+// in three passes: the second pass of the forward transform and the first of the
+// inverse one work on the same R2 values (bins k1 + R1 k2 for one k1), so each work
+// item takes both, with the shift between them, and the values make one LDS round trip
+// less than in fft_nat2dr followed by fft_dr2nat. load(s, q, v) sees every sample as it
+// is first read; store(s, q, v) receives every result (in place: buf[s*ss + q*es] = v).
+template <class T, int R1, int R2, int NTH, class L, class S>
+__device__ __forceinline__ void fft_half_sample(cx<T> *buf, int nsig, int ss, int es, const cx<T> *tw, const cx<T> *shift,
+                                                L load, S store) {
+    #pragma unroll 1
+    for (int t = threadIdx.x; t < nsig * R2; t += NTH) {
+        const int s = t % nsig, n2 = t / nsig;
+        cx<T> *b = buf + s * ss + n2 * es;
+        cx<T> x[R1];
+#pragma unroll
+        for (int n1 = 0; n1 < R1; ++n1) {
+            x[n1] = b[(R2 * n1) * es];
+            load(s, n2 + R2 * n1, x[n1]);
+        }
+        dft_r<T, +1, R1>(x);
+#pragma unroll
+        for (int k1 = 1; k1 < R1; ++k1) x[k1] = cmul(x[k1], twid<T, +1>(tw, n2 * k1));
+#pragma unroll
+        for (int k1 = 0; k1 < R1; ++k1) b[(R2 * k1) * es] = x[k1];
+    }
+    __syncthreads();
+    #pragma unroll 1
+    for (int t = threadIdx.x; t < nsig * R1; t += NTH) {
+        const int s = t % nsig, k1 = t / nsig;
+        cx<T> *b = buf + s * ss + (R2 * k1) * es;
+        cx<T> x[R2];
+#pragma unroll
+        for (int n2 = 0; n2 < R2; ++n2) x[n2] = b[n2 * es];
+        dft_r<T, +1, R2>(x);
+#pragma unroll
+        for (int k2 = 0; k2 < R2; ++k2) x[k2] = cmul(x[k2], shift[k1 + R1 * k2]);
+        dft_r<T, -1, R2>(x);
+#pragma unroll
+        for (int m2 = 1; m2 < R2; ++m2) x[m2] = cmul(x[m2], twid<T, -1>(tw, m2 * k1));
+#pragma unroll
+        for (int m2 = 0; m2 < R2; ++m2) b[m2 * es] = x[m2];
+    }
+    __syncthreads();
+    #pragma unroll 1
+    for (int t = threadIdx.x; t < nsig * R2; t += NTH) {
+        const int s = t % nsig, m2 = t / nsig;
+        cx<T> *b = buf + s * ss + m2 * es;
+        cx<T> x[R1];
+#pragma unroll
+        for (int k1 = 0; k1 < R1; ++k1) x[k1] = b[(R2 * k1) * es];
+        dft_r<T, -1, R1>(x);
+#pragma unroll
+        for (int m1 = 0; m1 < R1; ++m1) store(s, m2 + R2 * m1, x[m1]);
+    }
+}
+
 }  // namespace ampcor

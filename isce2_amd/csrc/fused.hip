@@ -212,177 +212,170 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
 // even samples = x. Output pixel (2r+p, 2c+q) comes from:
 //   p=0,q=0: X;  p=1,q=0: columns of X interpolated;
 //   p=0,q=1: Y = rows of X interpolated;  p=1,q=1: columns of Y interpolated.
-// Only one N x N complex chip lives in LDS (so several workgroups share a CU):
-// the chip is gathered (and deramped) twice, once for the X column pass and
-// once for the Y passes. |.| goes to HBM.
+// One N x N complex chip lives in LDS (so several workgroups share a CU) and each
+// thread keeps its pixels of X in registers, from which X is written a second time
+// after its columns have been interpolated in place. |.| goes to HBM from the
+// registers that hold each value on its way: X's as it is loaded, Y's as its columns
+// are first read, the others' as their last pass ends.
+// Bound by vector instructions (about 12.2k a window at N = 64, 17k at N = 72, deramped)
+// and LDS round trips, three an interpolation (fft_half_sample). 31,248 windows of 64:
+// reference chips (N = 64) 1516 -> 822 us, search chips (N = 72) 1661 -> 1118 us against
+// the form with four passes, two gathers and separate amplitude passes; the same
+// interpolations as products with the half-sample matrix on v_mfma_f32_16x16x4_f32,
+// which shares the vector ALU's throughput here: 902 and 1596 us.
 // ---------------------------------------------------------------------------
 struct OsArgs {
     const void *img; int64_t pitch; int mode;
     const int32_t *sd, *sa, *start;   // start may be null
     int deramp;
-    const cf *hsh;                    // [N] e^{-i pi k_s/N} / N
+    const cf *tw, *shift;             // [N] e^{-2 pi i k/N}, e^{-i pi k_s/N} / N
     float *out;                       // [n][4][N][N]: pixel (2r+p, 2c+q) in plane 2p+q at (r, c)
     double *mean;                     // [n][2]: mean and sum of squared deviations of |.| (MEAN kernels)
 };
 
-// chip (pitch N+1), shift table, deramp row/column rotation factors, reduction scratch, twiddles
-__host__ __device__ inline int os_lds_bytes(int N) { return al16(N * (N + 1) * 8 + N * 8) + 2 * N * 8 + 48 * 8 + N * 8; }
+// chip (pitch N+1), deramp row/column rotation factors, reduction scratch, twiddles, shifts
+__host__ __device__ inline int os_lds_bytes(int N) { return al16(N * (N + 1) * 8) + 4 * N * 8 + 32 * 8; }
 
-template <int R1, int R2, bool MEAN, int NTH = NT>
-__global__ void __launch_bounds__(NTH, (R1 * R2 == 64 && MEAN) ? 8 : 1) k_oversample(OsArgs a, const cf *tw_g, int w0) {
+// threads per workgroup, and waves per SIMD to fit its registers to: as many as the LDS
+// of the workgroups that share a CU leaves room for (four of N = 64, three of N = 72)
+__host__ __device__ constexpr int os_threads(int N) { return N >= 64 ? 512 : N == 40 ? 320 : 256; }
+
+template <int R1, int R2, bool MEAN, int NTH = os_threads(R1 * R2)>
+__global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArgs a, int w0) {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr int N = R1 * R2, PC = N + 1;
+    constexpr int N = R1 * R2, PC = N + 1, NW = NTH / 64;
     static_assert(2 * N <= NTH, "one thread per deramp row and column factor");
+    static_assert(4 * NW <= 32, "wave sums fit the reduction scratch");
     cf *C = reinterpret_cast<cf *>(smem);
-    cf *hsh = C + N * PC;
-    cf *rowf = reinterpret_cast<cf *>(smem + al16(N * PC * 8 + N * 8));   // e^{i r phy}
+    cf *rowf = reinterpret_cast<cf *>(smem + al16(N * PC * 8));           // e^{i r phy}
     cf *colf = rowf + N;                                                  // e^{i c phx}
     double *red = reinterpret_cast<double *>(colf + N);
-    cf *twl = reinterpret_cast<cf *>(red + 48);                           // twiddles, read from LDS
-    const cf *tw = twl;
+    cf *twl = reinterpret_cast<cf *>(red + 32), *shl = twl + N;           // twiddles and shifts, read from LDS
+    if (threadIdx.x < N) {
+        twl[threadIdx.x] = a.tw[threadIdx.x];
+        shl[threadIdx.x] = a.shift[threadIdx.x];
+    }
     const int win = w0 + xcd_window(blockIdx.x, gridDim.x);
     int64_t r0 = a.sd[win], c0 = a.sa[win];
     if (a.start) { r0 += a.start[2 * win]; c0 += a.start[2 * win + 1]; }
-    // deramp of pixel (r, c) (float2's operator*= (float2.h:71-75): the imaginary part
-    // uses the new real part); the phases and their sines and cosines are FP64, the
-    // factors and the rotation FP32
-    auto deramp_px = [&](cf z, int r, int c) -> cf {
-        const cf f = cmul(colf[c], rowf[r]);
-        const float nx = z.x * f.x - z.y * f.y;
-        return {nx, z.y * f.x + nx * f.y};
-    };
-    // chip into LDS; rot: deramped as it loads (the factors are in place)
-    auto gather = [&](bool rot) {
-#pragma unroll 4
-        for (int i = threadIdx.x; i < N * N; i += NTH) {
-            const int r = i / N, c = i - r * N;
-            const cf z = pixel_cx(a.img, a.mode, (r0 + r) * a.pitch + c0 + c);
-            C[r * PC + c] = rot ? deramp_px(z, r, c) : z;
-        }
-    };
-    double *psum = red + 16;             // [NTH/64][2] per-wave FP64 sums of |.| and |.|^2 (MEAN)
-    static_assert(16 + 2 * (NTH / 64) <= 48, "wave slots fit the reduction scratch");
-    if (MEAN && threadIdx.x < 2 * (NTH / 64)) psum[threadIdx.x] = 0.0;
-    gather(false);
-    for (int i = threadIdx.x; i < N; i += NTH) {
-        hsh[i] = a.hsh[i];
-        twl[i] = tw_g[i];
-    }
-    __syncthreads();
-    if (a.deramp == 1) {
-        double ayr = 0, ayi = 0, axr = 0, axi = 0;
-        for (int i = threadIdx.x; i < N * N; i += NTH) {
-            const int r = i / N, c = i - r * N;
-            const cf z = C[r * PC + c];
-            const double zr = z.x, zi = z.y;
-            if (c < N - 1) {
-                const cf b = C[r * PC + c + 1];
-                ayr += zr * b.x + zi * b.y; ayi += zi * b.x - zr * b.y;
-            }
-            if (r < N - 1) {
-                const cf b = C[(r + 1) * PC + c];
-                axr += zr * b.x + zi * b.y; axi += zi * b.x - zr * b.y;
-            }
-        }
-        ayr = block_sum<NTH>(ayr, red); ayi = block_sum<NTH>(ayi, red);
-        axr = block_sum<NTH>(axr, red); axi = block_sum<NTH>(axi, red);
-        const double phy = atan2(ayi, ayr), phx = atan2(axi, axr);
-        // the phase c*phx + r*phy is separable: one FP64 sincos per row and per column
-        if (threadIdx.x < 2 * N) {
-            const int k = threadIdx.x < N ? threadIdx.x : threadIdx.x - N;
-            double sn, cs;
-            sincos(double(k) * (threadIdx.x < N ? phy : phx), &sn, &cs);
-            (threadIdx.x < N ? rowf : colf)[k] = {float(cs), float(sn)};
-        }
-        __syncthreads();
+    // a thread keeps one chip column and RP consecutive rows of it in registers; where the
+    // workgroup is not whole columns of RP pixels, its last threads repeat rows of others
+    // (the same values to the same places: no access needs a condition), and only the
+    // phase sums leave the repeated rows out (k < first)
+    constexpr int GR = NTH / N, RP = (N + GR - 1) / GR;
+    constexpr bool EXACT = GR * N == NTH && GR * RP == N;
+    static_assert(EXACT || !MEAN, "the amplitude sums count every row once");
+    const int c = threadIdx.x % N, grp = threadIdx.x / N, rb = EXACT ? grp * RP : min(grp * RP, N - RP);
+    const int first = EXACT ? 0 : (grp < GR ? grp * RP - rb : RP);
+    cf z[RP];
+    {
+        auto load = [&](auto pixel) {
+            const int64_t off = (r0 + rb) * a.pitch + c0 + c;
+#pragma unroll
+            for (int k = 0; k < RP; ++k) z[k] = pixel(off + k * a.pitch);
+        };
+        if (a.mode == 2) load([&](int64_t o) { return cf{static_cast<const float *>(a.img)[o], 0.f}; });
+        else load([&](int64_t o) { return static_cast<const cf *>(a.img)[o]; });
+        if (a.mode == 1)
+#pragma unroll
+            for (int k = 0; k < RP; ++k) z[k] = {fast_sqrt(z[k].x * z[k].x + z[k].y * z[k].y), 0.f};
     }
     float *out = a.out + size_t(win) * 4 * N * N;
-    // FP64 sums of |.| and |.|^2: each emit reduces its own over the wave and
-    // adds them to the wave's LDS slot, so no FP64 accumulator stays live
-    // through the transforms (the reference-chip kernel is held to 64 VGPRs)
-    static_assert(N % 4 == 0, "four output columns per store");
-    // |C| -> output pixels (2r+p, 2c+q), four columns per thread; rot: C is deramped
-    // in place first (each thread rewrites the pixels it reads)
-    auto emit = [&](int p, int q, bool rot) {
-        double s1 = 0.0, s2 = 0.0;
-        float *plane = out + size_t(2 * p + q) * N * N;           // whole lines per phase
-        for (int i = threadIdx.x; i < N * N / 4; i += NTH) {
-            const int r = (4 * i) / N, c = 4 * i - r * N;
-            float amp[4];
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                cf v = C[r * PC + c + m];
-                if (rot) {
-                    v = deramp_px(v, r, c + m);
-                    C[r * PC + c + m] = v;
-                }
-                amp[m] = fast_sqrt(v.x * v.x + v.y * v.y);
-                if (MEAN) {
-                    s1 += amp[m];
-                    s2 += double(amp[m]) * amp[m];
-                }
-            }
-            *reinterpret_cast<float4 *>(plane + r * N + c) = make_float4(amp[0], amp[1], amp[2], amp[3]);
-        }
+    double s1 = 0.0, s2 = 0.0;           // FP64 sums of |.| and |.|^2 (MEAN)
+    auto add = [&](float v) {
         if (MEAN) {
+            s1 += v;
+            s2 += double(v) * v;
+        }
+    };
+    cf *own = C + rb * PC + c;
+    if (a.deramp == 1) {
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                s1 += __shfl_xor(s1, o);
-                s2 += __shfl_xor(s2, o);
-            }
-            if ((threadIdx.x & 63) == 0) {
-                psum[2 * (threadIdx.x >> 6)] += s1;
-                psum[2 * (threadIdx.x >> 6) + 1] += s2;
-            }
+        for (int k = 0; k < RP; ++k) own[k * PC] = z[k];
+        __syncthreads();
+        // FP64 sums of z conj(right neighbour) and z conj(neighbour below): the one to the
+        // right comes from LDS, the one below is the thread's own next pixel
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        // (neighbours past the last column or row count as zero)
+        const bool right = c < N - 1, below = rb + RP < N;
+        double zr = z[0].x, zi = z[0].y;
+#pragma unroll
+        for (int k = 0; k < RP; ++k) {
+            const bool once = EXACT || k >= first;
+            const cf w = own[k * PC + 1], d = k + 1 < RP ? z[(k + 1) % RP] : own[(below ? k + 1 : k) * PC];
+            const double br = right && once ? w.x : 0.f, bi = right && once ? w.y : 0.f;
+            t[0] += zr * br + zi * bi; t[1] += zi * br - zr * bi;
+            const bool dn = once && (k + 1 < RP || below);
+            const double dr = dn ? d.x : 0.f, di = dn ? d.y : 0.f;
+            t[2] += zr * dr + zi * di; t[3] += zi * dr - zr * di;
+            if (EXACT) { zr = dr; zi = di; }
+            else { zr = d.x; zi = d.y; }
         }
-    };
-    // the half-sample shift multiplies each bin as the forward transform stores it,
-    // except in the 64-VGPR reference kernel, where its own pass spills less
-    constexpr bool FOLD = !(N == 64 && MEAN);
-    auto interp_cols = [&]() {          // C <- C at half-row positions (every column)
-        fft_nat2dr<float, +1, R1, R2, NTH>(C, N, 1, PC, tw, FOLD ? hsh : nullptr);
-        if (!FOLD) {
-            for (int i = threadIdx.x; i < N * N; i += NTH) {
-                const int k = i / N, c = i - k * N;
-                cf &z = C[dr_pos<R1, R2>(k) * PC + c];
-                z = cmul(z, hsh[k]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] = wave_scan_f64(t[j]);
+        if ((threadIdx.x & 63) == 63)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[4 * (threadIdx.x >> 6) + j] = t[j];
+        __syncthreads();
+        // the phase c*phx + r*phy is separable: one FP64 sincos per row (phy, from the sums to
+        // the right) and per column (phx, from the sums below)
+        if (threadIdx.x < 2 * N) {
+            const bool row = threadIdx.x < N;
+            double ar = 0.0, ai = 0.0;
+#pragma unroll
+            for (int w = 0; w < NTH / 64; ++w) {
+                ar += red[4 * w + (row ? 0 : 2)];
+                ai += red[4 * w + (row ? 1 : 3)];
             }
-            __syncthreads();
-        }
-        fft_dr2nat<float, -1, R1, R2, NTH>(C, N, 1, PC, tw);
-    };
-    // X: even rows, even columns; then its column interpolation: odd rows, even columns
-    emit(0, 0, a.deramp == 1);
-    __syncthreads();
-    interp_cols();
-    emit(1, 0, false);
-    __syncthreads();
-    // Y = X interpolated along rows: even rows, odd columns; then its columns: odd rows, odd columns
-    gather(a.deramp == 1);
-    __syncthreads();
-    fft_nat2dr<float, +1, R1, R2, NTH>(C, N, PC, 1, tw, FOLD ? hsh : nullptr);
-    if (!FOLD) {
-        for (int i = threadIdx.x; i < N * N; i += NTH) {
-            const int r = i / N, k = i - r * N;
-            cf &z = C[r * PC + dr_pos<R1, R2>(k)];
-            z = cmul(z, hsh[k]);
+            const int k = row ? threadIdx.x : threadIdx.x - N;
+            double sn, cs;
+            sincos(double(k) * atan2(ai, ar), &sn, &cs);
+            (row ? rowf : colf)[k] = {float(cs), float(sn)};
         }
         __syncthreads();
+        // rotation through float2's operator*= (float2.h:71-75: the imaginary part uses the new
+        // real part); the phases and their sines and cosines are FP64, the factors and the
+        // rotation FP32
+        const cf fc = colf[c];
+#pragma unroll
+        for (int k = 0; k < RP; ++k) {
+            // read again from LDS: held through the FP64 sines, the pixels spill
+            z[k] = own[k * PC];
+            const cf f = cmul(fc, rowf[rb + k]);
+            const float nx = z[k].x * f.x - z[k].y * f.y;
+            z[k] = {nx, z[k].y * f.x + nx * f.y};
+        }
     }
-    fft_dr2nat<float, -1, R1, R2, NTH>(C, N, PC, 1, tw);
-    emit(0, 1, false);
+    // X: even rows, even columns
+#pragma unroll
+    for (int k = 0; k < RP; ++k) {
+        const float v = fast_sqrt(z[k].x * z[k].x + z[k].y * z[k].y);
+        add(v);
+        out[(rb + k) * N + c] = v;
+    }
+    if (!EXACT && a.deramp == 1) __syncthreads();     // a repeated row has two readers above
+#pragma unroll
+    for (int k = 0; k < RP; ++k) own[k * PC] = z[k];
     __syncthreads();
-    interp_cols();
-    emit(1, 1, false);
+    auto emit = [&](int plane, int r, int col, cf v) {
+        const float m = fast_sqrt(v.x * v.x + v.y * v.y);
+        add(m);
+        out[plane * N * N + r * N + col] = m;
+    };
+    auto skip = [](int, int, cf) {};
+    // columns of X (the registers keep X), then X again and its rows in place, then the columns of those
+    fft_half_sample<float, R1, R2, NTH>(C, N, 1, PC, twl, shl, skip, [&](int s, int m, cf v) { emit(2, m, s, v); });
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RP; ++k) own[k * PC] = z[k];
+    __syncthreads();
+    fft_half_sample<float, R1, R2, NTH>(C, N, PC, 1, twl, shl, skip, [&](int s, int m, cf v) { C[s * PC + m] = v; });
+    __syncthreads();
+    fft_half_sample<float, R1, R2, NTH>(C, N, 1, PC, twl, shl, [&](int s, int m, cf v) { emit(1, m, s, v); },
+                                        [&](int s, int m, cf v) { emit(3, m, s, v); });
     if (MEAN) {
         // FP64 mean and sum of squared deviations (sum2 - sum^2 / count)
-        __syncthreads();
-        double sum = 0.0, sum2 = 0.0;
-#pragma unroll
-        for (int w = 0; w < NTH / 64; ++w) {
-            sum += psum[2 * w];
-            sum2 += psum[2 * w + 1];
-        }
+        const double sum = block_sum<NTH>(s1, red), sum2 = block_sum<NTH>(s2, red);
         const double cnt = double(4 * N * N);
         if (threadIdx.x == 0) {
             a.mean[2 * win] = sum / cnt;
@@ -934,16 +927,15 @@ bool fused_supported(const ampcor_params &p, const ampcor_sizes &s) {
 FusedTables Engine::fused_tables() {
     using namespace fused;
     const int W = p.window_w, Zc = sz.zoom_in_w;
-    // half-sample shift tables h[k] = e^{-i pi k_s/N}/N for the chip sizes
-    auto hshift = [&](int N) -> const void * {
+    // half-sample shifts e^{-i pi k_s/N}/N of the chip sides (k_oversample)
+    auto half_sample_shifts = [&](int N) -> const void * {
         const std::string key = "f_hsh" + std::to_string(N);
         auto &b = bufs[key];
         if (!b) {
             forbid_in_nosync("build a shift table");
             std::vector<float> h(2 * N);
             for (int k = 0; k < N; ++k) {
-                const int ks = k < N / 2 ? k : k - N;
-                const long double ang = -3.14159265358979323846264338327950288L * ks / N;
+                const long double ang = -3.14159265358979323846264338327950288L * (k < N / 2 ? k : k - N) / N;
                 h[2 * k] = float(cosl(ang) / N);
                 h[2 * k + 1] = float(sinl(ang) / N);
             }
@@ -955,11 +947,11 @@ FusedTables Engine::fused_tables() {
     };
     auto tw = [&](int n) { return static_cast<const void *>(plan(n).tw32.ptr); };
     FusedTables t;
-    t.h_ref = hshift(W);
-    t.h_zoom = hshift(Zc);
+    t.tw_ref = tw(W);
+    t.shift_ref = half_sample_shifts(W);
+    t.tw_zoom = tw(Zc);
+    t.shift_zoom = half_sample_shifts(Zc);
     t.tw1 = tw(coarse_L(sz.search_w));
-    t.twW = tw(W);
-    t.twZ = tw(Zc);
     t.tw2 = tw(2 * Zc);
     t.tws = tw(sz.surf_out);
     t.tws_64 = plan(sz.surf_out).tw64.ptr;
@@ -978,9 +970,9 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
     const int K1 = pick_k(sz.raw_corr_h, NT / (L1 / 2));
     const int mode = p.image_complex ? (p.deramp == 0 ? 1 : 0) : 2;
     const int surf = p.surf_method ? -1 : (p.surf_ovs == 16 ? 16 : 0);   // surface stage (fine_finish)
-    const cf *tw1 = static_cast<const cf *>(tb.tw1), *twW = static_cast<const cf *>(tb.twW);
-    const cf *twZ = static_cast<const cf *>(tb.twZ), *tw2 = static_cast<const cf *>(tb.tw2);
-    const cf *h_ref = static_cast<const cf *>(tb.h_ref), *h_zoom = static_cast<const cf *>(tb.h_zoom);
+    const cf *tw1 = static_cast<const cf *>(tb.tw1), *tw2 = static_cast<const cf *>(tb.tw2);
+    const cf *tw_ref = static_cast<const cf *>(tb.tw_ref), *shift_ref = static_cast<const cf *>(tb.shift_ref);
+    const cf *tw_zoom = static_cast<const cf *>(tb.tw_zoom), *shift_zoom = static_cast<const cf *>(tb.shift_zoom);
     float *tamp = c.tamp - size_t(w0) * T2 * T2;          // indexed by absolute window inside the kernels
     double *tmean = c.tmean - 2 * size_t(w0);
     float *samp = c.samp - size_t(w0) * P * P;
@@ -998,17 +990,17 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
             else if (L1 == 128) launch_coarse<32, 8, 16>(K1, ca, tw1, n, w0, lds_c, st);
             else launch_coarse<32, 8, 8>(K1, ca, tw1, n, w0, lds_c, st);
         });
-        OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, h_ref, tamp, tmean};
-        OsArgs osec{c.sec, c.sec_pitch, mode, c.sec_d, c.sec_a, c.start, p.deramp, h_zoom, samp, nullptr};
+        OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, tw_ref, shift_ref, tamp, tmean};
+        OsArgs osec{c.sec, c.sec_pitch, mode, c.sec_d, c.sec_a, c.start, p.deramp, tw_zoom, shift_zoom, samp, nullptr};
         FineArgs fa{tamp, tmean, samp, c.start, p.hs_down, p.hs_across, 1.0f / float(p.surf_ovs * p.raw_ovs),
                     p.surf_ovs, static_cast<const cf *>(tb.tws), SincTable{sinc_table.as<float>(), sinc_dec}, c.shift,
                     c.zidx, c.offset, c.mf, c.surf ? c.surf - size_t(w0) * 256 : nullptr};
         if (W == 64) {
             timed("k_oversample_ref", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 8, true>), dim3(n), dim3(NT), lds_or, st, oref, twW, w0);
+                hipLaunchKernelGGL((k_oversample<8, 8, true>), dim3(n), dim3(os_threads(64)), lds_or, st, oref, w0);
             });
             timed("k_oversample_search", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 9, false>), dim3(n), dim3(NT), lds_oz, st, osec, twZ, w0);
+                hipLaunchKernelGGL((k_oversample<9, 8, false>), dim3(n), dim3(os_threads(72)), lds_oz, st, osec, w0);
             });
             timed("k_fine", n, st, [&] {
                 // the whole-template kernel is built for the surfaces AMPCOR_MODE_FUSED accepts
@@ -1023,10 +1015,10 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
             });
         } else {
             timed("k_oversample_ref", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 4, true>), dim3(n), dim3(NT), lds_or, st, oref, twW, w0);
+                hipLaunchKernelGGL((k_oversample<8, 4, true>), dim3(n), dim3(os_threads(32)), lds_or, st, oref, w0);
             });
             timed("k_oversample_search", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 5, false>), dim3(n), dim3(NT), lds_oz, st, osec, twZ, w0);
+                hipLaunchKernelGGL((k_oversample<5, 8, false>), dim3(n), dim3(os_threads(40)), lds_oz, st, osec, w0);
             });
             timed("k_fine", n, st, [&] {
                 if (surf == 16)
