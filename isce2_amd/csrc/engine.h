@@ -114,6 +114,16 @@ struct Engine {
                                           "; run the same call once before capturing it");
     }
     const FftPlan &plan(int n);
+    // [n] half-sample shifts e^{-i pi k_s/n}/n, k_s = k below n/2 and k - n from there on, in device memory
+    template <class T> const cx<T> *half_shifts(int n) {
+        const std::string key = (sizeof(T) == 8 ? "d_hsh" : "f_hsh") + std::to_string(n);
+        const bool have = bufs.count(key) != 0;
+        cx<T> *dst = buf<cx<T>>(key, n);
+        if (!have) put_half_shifts(dst, n);
+        return dst;
+    }
+    void put_half_shifts(cx<float> *dst, int n);
+    void put_half_shifts(cx<double> *dst, int n);
     void set_fft_radices(int n, const int32_t *radices, int count);
     template <class U> U *buf(const std::string &name, size_t count) {
         auto &b = bufs[name];

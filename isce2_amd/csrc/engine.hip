@@ -102,6 +102,20 @@ const FftPlan &Engine::plan(int n) {
     return ref;
 }
 
+namespace {
+template <class T>
+void upload_half_shifts(cx<T> *dst, int n) {
+    std::vector<cx<T>> h(n);
+    for (int k = 0; k < n; ++k) {
+        const long double t = -3.14159265358979323846264338327950288L * (k < n / 2 ? k : k - n) / n;
+        h[k] = {T(cosl(t) / n), T(sinl(t) / n)};
+    }
+    HIP_OK(hipMemcpy(dst, h.data(), n * sizeof(cx<T>), hipMemcpyHostToDevice));
+}
+}  // namespace
+void Engine::put_half_shifts(cx<float> *dst, int n) { upload_half_shifts(dst, n); }
+void Engine::put_half_shifts(cx<double> *dst, int n) { upload_half_shifts(dst, n); }
+
 // cuAmpcorParameter::setupParameters (cuAmpcorParameter.cpp:70-98), with each
 // axis sized by its own half search range (the reference swaps them, :90-91).
 void Engine::setup(const ampcor_params &q) {
@@ -317,9 +331,9 @@ template <class T, int R1, int R2, int CB = 16, int NTH = 256>
 void os2_cols_launch(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab,
                      int nimg, int w, cx<T> *Y, hipStream_t st) {
     constexpr int N = R1 * R2;
-    const size_t lds = (size_t(N) * (CB + 1) + N) * sizeof(cx<T>);
+    const size_t lds = size_t(N) * (CB + 1) * sizeof(cx<T>);
     hipLaunchKernelGGL((k_os2_cols_f<T, R1, R2, CB, NTH>), dim3(idivup(w, CB), nimg), dim3(NTH), lds, st, src, ih, iw,
-                       start, tab, w, tw_of<T>(e, N), Y);
+                       start, tab, w, tw_of<T>(e, N), e.half_shifts<T>(N), Y);
 }
 
 // output rows per block of k_os2_rows_f: 16 where the second factor is a long
@@ -338,9 +352,9 @@ void os2_rows_launch(Engine &e, const cx<T> *src, int ih, int iw, const int32_t 
     constexpr int N = R1 * R2, G = os2_rows_g<T, R2>();
     // k_mean_parts reads one block sum per G rows: the width table must agree
     if (G != os2_rows_per_block<T>(N)) throw Error(AMPCOR_E_ARG, "row block size table out of step");
-    const size_t lds = (size_t(G) * (N + 1) + N) * sizeof(cx<T>) + size_t(G) * N * sizeof(T);
+    const size_t lds = size_t(G) * (N + 1) * sizeof(cx<T>) + size_t(G) * N * sizeof(T);
     hipLaunchKernelGGL((k_os2_rows_f<T, R1, R2, G, NTH>), dim3(idivup(nimg * 2 * h, G)), dim3(NTH), lds, st, src, ih, iw,
-                       start, tab, Y, nimg, h, tw_of<T>(e, N), out, part);
+                       start, tab, Y, nimg, h, tw_of<T>(e, N), e.half_shifts<T>(N), out, part);
 }
 
 template <class T>

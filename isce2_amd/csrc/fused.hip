@@ -927,30 +927,12 @@ bool fused_supported(const ampcor_params &p, const ampcor_sizes &s) {
 FusedTables Engine::fused_tables() {
     using namespace fused;
     const int W = p.window_w, Zc = sz.zoom_in_w;
-    // half-sample shifts e^{-i pi k_s/N}/N of the chip sides (k_oversample)
-    auto half_sample_shifts = [&](int N) -> const void * {
-        const std::string key = "f_hsh" + std::to_string(N);
-        auto &b = bufs[key];
-        if (!b) {
-            forbid_in_nosync("build a shift table");
-            std::vector<float> h(2 * N);
-            for (int k = 0; k < N; ++k) {
-                const long double ang = -3.14159265358979323846264338327950288L * (k < N / 2 ? k : k - N) / N;
-                h[2 * k] = float(cosl(ang) / N);
-                h[2 * k + 1] = float(sinl(ang) / N);
-            }
-            b.reset(new DevBuf());
-            b->reserve(h.size() * sizeof(float));
-            HIP_OK(hipMemcpy(b->ptr, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));
-        }
-        return b->ptr;
-    };
     auto tw = [&](int n) { return static_cast<const void *>(plan(n).tw32.ptr); };
     FusedTables t;
     t.tw_ref = tw(W);
-    t.shift_ref = half_sample_shifts(W);
+    t.shift_ref = half_shifts<float>(W);
     t.tw_zoom = tw(Zc);
-    t.shift_zoom = half_sample_shifts(Zc);
+    t.shift_zoom = half_shifts<float>(Zc);
     t.tw1 = tw(coarse_L(sz.search_w));
     t.tw2 = tw(2 * Zc);
     t.tws = tw(sz.surf_out);

@@ -913,39 +913,34 @@ __global__ void __launch_bounds__(256) k_os2_rows(const cx<T> *src, int ih, int 
     }
 }
 
-// The same two passes for chip sides N = R1 * R2 with the transforms in place
-// (fft_nat2dr, which applies the shift factors as it stores each bin, then
-// fft_dr2nat: the spectrum stays in digit-reversed order), one chip line per
-// LDS row of odd pitch.
+// The same two passes for chip sides N = R1 * R2 with the interpolation in place
+// (fft_half_sample: three LDS passes), one chip line per LDS row of odd pitch.
+// `tw`, `shift`: e^{-2 pi i k/N} and the half-sample shifts, copied into LDS.
 
 // CB chip columns per block (blockIdx.x), one chip per blockIdx.y; chip height
 // R1 * R2; Y: [nimg][R1 * R2][w]
 template <class T, int R1, int R2, int CB, int NTH = 256>
 __global__ void __launch_bounds__(NTH) k_os2_cols_f(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                                    const cx<double> *tab, int w, const cx<T> *tw, cx<T> *Y) {
+                                                    const cx<double> *tab, int w, const cx<T> *tw, const cx<T> *shift,
+                                                    cx<T> *Y) {
     constexpr int N = R1 * R2, PC = CB + 1;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *C = reinterpret_cast<cx<T> *>(smem_raw);   // [N][PC]: column c at C[c + r * PC]
-    cx<T> *sh = C + N * PC;                            // shift factors in bin order
-    __shared__ cx<T> twl[N];                           // twiddles, read from LDS
+    __shared__ cx<T> twl[N], sh[N];
     const int win = blockIdx.y, c0 = blockIdx.x * CB, nc = min(CB, w - c0);
     for (int i = threadIdx.x; i < N * CB; i += NTH) {
         const int r = i / CB, c = i - r * CB;
         if (c < nc) C[r * PC + c] = chip_pixel(src, ih, iw, start, tab, win, N, w, r, c0 + c);
     }
     for (int k = threadIdx.x; k < N; k += NTH) {
-        sh[k] = half_shift<T>(k, N);
+        sh[k] = shift[k];
         twl[k] = tw[k];
     }
     __syncthreads();
-    // the shift multiplies each bin as the forward transform stores it
-    fft_nat2dr<T, +1, R1, R2, NTH>(C, nc, 1, PC, twl, sh);
-    fft_dr2nat<T, -1, R1, R2, NTH>(C, nc, 1, PC, twl);
+    // consecutive work items hold consecutive columns: the results go out as they are made
     cx<T> *y = Y + size_t(win) * N * w + c0;
-    for (int i = threadIdx.x; i < N * CB; i += NTH) {
-        const int r = i / CB, c = i - r * CB;
-        if (c < nc) y[size_t(r) * w + c] = C[r * PC + c];
-    }
+    fft_half_sample<T, R1, R2, NTH>(C, nc, 1, PC, twl, sh, [](int, int, cx<T>) {},
+                                    [&](int c, int r, cx<T> v) { y[size_t(r) * w + c] = v; });
 }
 
 // G output rows per block over the nimg * 2h rows; chip width R1 * R2;
@@ -955,13 +950,12 @@ __global__ void __launch_bounds__(NTH) k_os2_cols_f(const cx<T> *src, int ih, in
 template <class T, int R1, int R2, int G, int NTH = 256>
 __global__ void __launch_bounds__(NTH) k_os2_rows_f(const cx<T> *src, int ih, int iw, const int32_t *start,
                                                     const cx<double> *tab, const cx<T> *Y, int nimg, int h,
-                                                    const cx<T> *tw, T *out, double *part) {
+                                                    const cx<T> *tw, const cx<T> *shift, T *out, double *part) {
     constexpr int N = R1 * R2, PR = N + 1;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *C = reinterpret_cast<cx<T> *>(smem_raw);   // [G][PR]
-    cx<T> *sh = C + G * PR;                            // shift factors in bin order
-    T *amp = reinterpret_cast<T *>(sh + N);            // [G][N]
-    __shared__ cx<T> twl[N];                           // twiddles, read from LDS
+    T *amp = reinterpret_cast<T *>(C + G * PR);        // [G][N]
+    __shared__ cx<T> twl[N], sh[N];
     const int t0 = blockIdx.x * G;
     const int nr = min(G, nimg * 2 * h - t0);
     for (int i = threadIdx.x; i < nr * N; i += NTH) {
@@ -972,13 +966,13 @@ __global__ void __launch_bounds__(NTH) k_os2_rows_f(const cx<T> *src, int ih, in
         amp[i] = amag(v);
     }
     for (int k = threadIdx.x; k < N; k += NTH) {
-        sh[k] = half_shift<T>(k, N);
+        sh[k] = shift[k];
         twl[k] = tw[k];
     }
     __syncthreads();
-    // the shift multiplies each bin as the forward transform stores it
-    fft_nat2dr<T, +1, R1, R2, NTH>(C, nr, PR, 1, twl, sh);
-    fft_dr2nat<T, -1, R1, R2, NTH>(C, nr, PR, 1, twl);
+    fft_half_sample<T, R1, R2, NTH>(C, nr, PR, 1, twl, sh, [](int, int, cx<T>) {},
+                                    [&](int k, int c, cx<T> v) { C[k * PR + c] = v; });
+    __syncthreads();
     T *o = out + size_t(t0) * 2 * N;
     double s1 = 0.0, s2 = 0.0;
     for (int i = threadIdx.x; i < nr * N; i += NTH) {
