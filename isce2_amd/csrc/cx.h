@@ -36,10 +36,48 @@ template <class T, int DIR> __host__ __device__ __forceinline__ cx<T> mul_i(cx<T
 __device__ __forceinline__ float fast_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
 template <class T> __device__ __forceinline__ T amag(cx<T> a);
-template <> __device__ __forceinline__ float amag<float>(cx<float> a) { return fast_sqrt(a.x * a.x + a.y * a.y); }
+// |z| of FP32 chips with the rounding fixed (which product the addition fuses is otherwise
+// the compiler's choice in each kernel, and the same pixel could differ in its last bit)
+__device__ __forceinline__ float fast_abs(float x, float y) { return fast_sqrt(fmaf(x, x, y * y)); }
+template <> __device__ __forceinline__ float amag<float>(cx<float> a) { return fast_abs(a.x, a.y); }
 template <> __device__ __forceinline__ double amag<double>(cx<double> a) { return sqrt(a.x * a.x + a.y * a.y); }
 
 __host__ __device__ __forceinline__ int idivup(int a, int b) { return (a + b - 1) / b; }
+
+// DPP move of an FP64 value (both halves); lanes the row mask leaves out keep 0
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWMASK, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWMASK, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// DPP row shift of an FP64 value with every lane written: lanes whose source
+// lies before the start of their row read 0 (bound_ctrl), so no zeroed
+// destination is needed
+template <int CTRL>
+__device__ __forceinline__ double dpp_shr_f64(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// inclusive wave64 prefix sum: row_shr 1, 2, 4, 8 within rows of 16 lanes, then
+// row_bcast:15 into rows 1 and 3 and row_bcast:31 into rows 2 and 3
+__device__ __forceinline__ double wave_scan_f64(double x) {
+    x += dpp_shr_f64<0x111>(x);
+    x += dpp_shr_f64<0x112>(x);
+    x += dpp_shr_f64<0x114>(x);
+    x += dpp_shr_f64<0x118>(x);
+    x += dpp_f64<0x142, 0xa>(x);
+    x += dpp_f64<0x143, 0xc>(x);
+    return x;
+}
+
+__device__ __forceinline__ double lane63_f64(double x) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                            __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
 
 // 9-bit bit reversal: tie-break key of the 512-thread argmax of cuOffset.cu:23-84
 __device__ __forceinline__ uint32_t bitrev9(uint32_t v) { return __brev(v) >> 23; }

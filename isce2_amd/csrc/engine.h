@@ -153,10 +153,14 @@ struct Engine {
         float *margin_coarse = nullptr, *margin_fine = nullptr;   // debug: top-1 minus top-2
         bool nosync = false;                                       // AMPCOR_FLAG_NOSYNC
         // windows [fine_from, n) take their coarse zoom start and shift from these
-        // (the staged pipeline skips its raw stage for chunks of such windows only)
+        // (the staged pipeline runs its raw stage for the windows before them only)
         const int32_t *fine_start = nullptr, *fine_shift = nullptr;
         int32_t fine_from = 0;
         double *refined = nullptr;   // [n][2] FP64 parabolic refinement of the offset, or null
+        // a re-run: window i's results go to window scatter[i] of the output arrays, all of
+        // them for i < full, offset, refined offset and zoom peak only from there on
+        const int32_t *scatter = nullptr;
+        int32_t full = 0;
     };
     // precision: 0 FP32 only; 1 FP32 + FP64 re-run of windows whose argmax
     // margins fall below the thresholds; 2 FP64 staged pipeline for every window
@@ -194,7 +198,7 @@ struct Engine {
 };
 
 // FFT schedule for length n (radices in pass order; direct DFT if a prime > 17 remains)
-FftDesc make_schedule(int n);
+FftDesc make_schedule(int n, bool f64);
 // whether the fused kernels can run a configuration (what AMPCOR_MODE_AUTO goes by), and
 // whether it is one of those that AMPCOR_MODE_FUSED and the allocation-free entry accept
 // (surface oversampling 16 by the FFT)

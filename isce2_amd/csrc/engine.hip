@@ -58,11 +58,13 @@ Engine::~Engine() {
     for (auto e : event_pool) (void)hipEventDestroy(e);
 }
 
-FftDesc make_schedule(int n) {
+// FP64 rows are few (re-runs of near ties): radices of at most 4 spread a row over more
+// threads (a radix-16 pass of 144 points has 9 butterflies)
+FftDesc make_schedule(int n, bool f64) {
     FftDesc d{};
     d.n = n;
     int m = n;
-    const int pow2[] = {16, 8, 4, 2};
+    const int pow2[] = {f64 ? 4 : 16, f64 ? 4 : 8, 4, 2};
     const int odd[] = {3, 5, 7, 11, 13, 17};
     for (int r : pow2)
         while (m % r == 0 && m > 1) { d.radix[d.npass++] = r; m /= r; }
@@ -81,7 +83,8 @@ const FftPlan &Engine::plan(int n) {
     forbid_in_nosync("build an FFT plan");
     std::unique_ptr<FftPlan> p(new FftPlan());
     p->n = n;
-    p->desc32 = p->desc64 = make_schedule(n);
+    p->desc32 = make_schedule(n, false);
+    p->desc64 = make_schedule(n, true);
     std::vector<float> t32(2 * n);
     std::vector<double> t64(2 * n);
     for (int k = 0; k < n; ++k) {
@@ -318,117 +321,116 @@ void fft2_chip(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start
     fft_cols<T, DIR>(e.plan(h), dst, nimg, w, fft_elems<T>(e), st, cols_width<T>(e));
 }
 
-// x2 oversampled amplitude `out` ([nimg][2h][2w]) of h x w chips read from
-// [nimg][ih][iw] sources (cropped at `start`, deramped with `tab` when given),
-// by the separable interpolation (k_os2_cols, then k_os2_rows); `Y` holds the
-// [nimg][h][w] odd rows between the passes
-// in-place kernels for the chip sides of the common windows (32, 64, 128, 256
-// and their zoom chips, 8 pixels wider); false for other sides
 template <class T>
 const cx<T> *tw_of(Engine &e, int n) { return static_cast<const cx<T> *>(sizeof(T) == 4 ? e.plan(n).tw32.ptr : e.plan(n).tw64.ptr); }
 
-template <class T, int R1, int R2, int CB = 16, int NTH = 256>
-void os2_cols_launch(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab,
-                     int nimg, int w, cx<T> *Y, hipStream_t st) {
-    constexpr int N = R1 * R2;
-    const size_t lds = size_t(N) * (CB + 1) * sizeof(cx<T>);
-    hipLaunchKernelGGL((k_os2_cols_f<T, R1, R2, CB, NTH>), dim3(idivup(w, CB), nimg), dim3(NTH), lds, st, src, ih, iw,
-                       start, tab, w, tw_of<T>(e, N), e.half_shifts<T>(N), Y);
-}
-
-// output rows per block of k_os2_rows_f: 16 where the second factor is a long
-// odd DFT (its pass has G * R1 work items), else 8 (measured on window-256 pairs)
-template <class T, int R2>
-constexpr int os2_rows_g() { return sizeof(T) == 4 && R2 >= 17 ? 16 : 8; }
-
-// the same count by chip width (the widths os2_rows_fast runs: 136 = 8 x 17 is the
-// one with a long second factor)
-template <class T>
-int os2_rows_per_block(int w) { return sizeof(T) == 4 && w == 136 ? 16 : 8; }
-
-template <class T, int R1, int R2, int NTH = 256>
-void os2_rows_launch(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab,
-                     const cx<T> *Y, int nimg, int h, T *out, double *part, hipStream_t st) {
-    constexpr int N = R1 * R2, G = os2_rows_g<T, R2>();
-    // k_mean_parts reads one block sum per G rows: the width table must agree
-    if (G != os2_rows_per_block<T>(N)) throw Error(AMPCOR_E_ARG, "row block size table out of step");
-    const size_t lds = size_t(G) * (N + 1) * sizeof(cx<T>) + size_t(G) * N * sizeof(T);
-    hipLaunchKernelGGL((k_os2_rows_f<T, R1, R2, G, NTH>), dim3(idivup(nimg * 2 * h, G)), dim3(NTH), lds, st, src, ih, iw,
-                       start, tab, Y, nimg, h, tw_of<T>(e, N), e.half_shifts<T>(N), out, part);
-}
-
-template <class T>
-bool os2_cols_fast(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab,
-                   int nimg, int h, int w, cx<T> *Y, hipStream_t st) {
-    switch (h) {
-        case 32: os2_cols_launch<T, 8, 4>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 40: os2_cols_launch<T, 8, 5>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 64: os2_cols_launch<T, 8, 8>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 72: os2_cols_launch<T, 8, 9>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 128: os2_cols_launch<T, 16, 8>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 136: os2_cols_launch<T, 8, 17>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 256: os2_cols_launch<T, 16, 16>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        case 264: os2_cols_launch<T, 11, 24>(e, src, ih, iw, start, tab, nimg, w, Y, st); return true;
-        default: return false;
-    }
-}
-
-// chip widths with an in-place row kernel
-bool os2_rows_has(int w) {
-    switch (w) {
+// x2 oversampled amplitudes of chips read in place (cropped at the zoom start and deramped
+// as they load) by the separable interpolation: column pass, then row pass, with the odd
+// rows between them in OsJob::Y. In-place kernels for the chip sides of the common windows
+// (32, 64, 128, 256 and their zoom chips, 8 pixels wider), else the Stockham ones.
+bool os2_has(int n) {
+    switch (n) {
         case 32: case 40: case 64: case 72: case 128: case 136: case 256: case 264: return true;
         default: return false;
     }
 }
 
+// output rows per block of k_os2_rows_f: 16 where the second factor is a long odd DFT
+// (136 = 8 x 17: its pass has G * R1 work items), else 8 (measured on window-256 pairs)
 template <class T>
-bool os2_rows_fast(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab,
-                   const cx<T> *Y, int nimg, int h, int w, T *out, double *part, hipStream_t st) {
-    switch (w) {
-        case 32: os2_rows_launch<T, 8, 4>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 40: os2_rows_launch<T, 8, 5>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 64: os2_rows_launch<T, 8, 8>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 72: os2_rows_launch<T, 8, 9>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 128: os2_rows_launch<T, 16, 8>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 136: os2_rows_launch<T, 8, 17>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 256: os2_rows_launch<T, 16, 16>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        case 264: os2_rows_launch<T, 24, 11, 192>(e, src, ih, iw, start, tab, Y, nimg, h, out, part, st); return true;
-        default: return false;
+int os2_rows_per_block(int w) { return sizeof(T) == 4 && w == 136 ? 16 : 8; }
+
+template <class T, int R1, int R2, int CB = 16>
+void os2_cols_launch(OsJob<T> j, int nimg, hipStream_t st) {
+    hipLaunchKernelGGL((k_os2_cols_f<T, R1, R2, CB>), dim3(idivup(j.w, CB), nimg), dim3(256), os2_cols_lds<T>(R1 * R2, CB), st,
+                       j);
+}
+template <class T, int R1, int R2, int G, int NTH = 256>
+void os2_rows_launch(OsJob<T> j, int nimg, hipStream_t st) {
+    hipLaunchKernelGGL((k_os2_rows_f<T, R1, R2, G, NTH>), dim3(idivup(nimg * 2 * j.h, G)), dim3(NTH),
+                       os2_rows_f_lds<T>(R1 * R2, G), st, j, nimg);
+}
+
+void os2_cols_fast(const OsJob<float> &j, int nimg, hipStream_t st) {
+    switch (j.h) {
+        case 32: os2_cols_launch<float, 8, 4>(j, nimg, st); break;
+        case 40: os2_cols_launch<float, 8, 5>(j, nimg, st); break;
+        case 64: os2_cols_launch<float, 8, 8>(j, nimg, st); break;
+        case 72: os2_cols_launch<float, 8, 9>(j, nimg, st); break;
+        case 128: os2_cols_launch<float, 16, 8>(j, nimg, st); break;
+        case 136: os2_cols_launch<float, 8, 17>(j, nimg, st); break;
+        case 256: os2_cols_launch<float, 16, 16>(j, nimg, st); break;
+        default: os2_cols_launch<float, 11, 24>(j, nimg, st); break;
+    }
+}
+void os2_rows_fast(const OsJob<float> &j, int nimg, hipStream_t st) {
+    switch (j.w) {
+        case 32: os2_rows_launch<float, 8, 4, 8>(j, nimg, st); break;
+        case 40: os2_rows_launch<float, 8, 5, 8>(j, nimg, st); break;
+        case 64: os2_rows_launch<float, 8, 8, 8>(j, nimg, st); break;
+        case 72: os2_rows_launch<float, 8, 9, 8>(j, nimg, st); break;
+        case 128: os2_rows_launch<float, 16, 8, 8>(j, nimg, st); break;
+        case 136: os2_rows_launch<float, 8, 17, 16>(j, nimg, st); break;
+        case 256: os2_rows_launch<float, 16, 16, 8>(j, nimg, st); break;
+        default: os2_rows_launch<float, 24, 11, 8, 192>(j, nimg, st); break;
     }
 }
 
-// `part`: block sums for k_mean_parts (in-place row kernel only; null for none)
+// column and row passes of both kinds of chips, FP32: a launch each
+void os2_both(Engine &, OsJob<float> a, OsJob<float> b, int nimg, hipStream_t st) {
+    for (OsJob<float> *j : {&a, &b}) {
+        os2_cols_fast(*j, nimg, st);
+        os2_rows_fast(*j, nimg, st);
+    }
+}
+
+// FP64: one launch for both kinds (the search side is the reference side + 8)
+template <int A1, int A2, int B1, int B2>
+void os2_cols_pair(OsJob<double> a, OsJob<double> b, int nimg, hipStream_t st) {
+    constexpr int CB = 16;
+    a.blocks = idivup(a.w, CB);
+    hipLaunchKernelGGL((k_os2_cols_pair<double, A1, A2, B1, B2, CB>), dim3(a.blocks + idivup(b.w, CB), nimg), dim3(256),
+                       os2_cols_lds<double>(B1 * B2, CB), st, a, b);
+}
+template <int A1, int A2, int B1, int B2>
+void os2_rows_pair(OsJob<double> a, OsJob<double> b, int nimg, hipStream_t st) {
+    constexpr int G = 8;
+    a.blocks = idivup(nimg * 2 * a.h, G);
+    hipLaunchKernelGGL((k_os2_rows_pair<double, A1, A2, B1, B2, G>), dim3(a.blocks + idivup(nimg * 2 * b.h, G)), dim3(256),
+                       os2_rows_f_lds<double>(B1 * B2, G), st, a, b, nimg);
+}
+void os2_both(Engine &, OsJob<double> a, OsJob<double> b, int nimg, hipStream_t st) {
+    switch (a.h) {
+        case 32: os2_cols_pair<8, 4, 8, 5>(a, b, nimg, st); break;
+        case 64: os2_cols_pair<8, 8, 8, 9>(a, b, nimg, st); break;
+        case 128: os2_cols_pair<16, 8, 8, 17>(a, b, nimg, st); break;
+        default: os2_cols_pair<16, 16, 11, 24>(a, b, nimg, st); break;
+    }
+    switch (a.w) {
+        case 32: os2_rows_pair<8, 4, 8, 5>(a, b, nimg, st); break;
+        case 64: os2_rows_pair<8, 8, 8, 9>(a, b, nimg, st); break;
+        case 128: os2_rows_pair<16, 8, 8, 17>(a, b, nimg, st); break;
+        default: os2_rows_pair<16, 16, 24, 11>(a, b, nimg, st); break;
+    }
+}
+
+// any even sides, Stockham transforms
 template <class T>
-void os2_separable(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start, const cx<double> *tab, int nimg,
-                   int h, int w, cx<T> *Y, T *out, hipStream_t st, double *part = nullptr) {
+void os2_general(Engine &e, const OsJob<T> &j, int nimg, hipStream_t st) {
     const bool f32 = std::is_same<T, float>::value;
-    const FftPlan &pc = e.plan(h), &pr = e.plan(w);
-    const int elems = fft_elems<T>(e);
-    if (e.oversampler == 2) {
-        const bool cols = os2_cols_fast<T>(e, src, ih, iw, start, tab, nimg, h, w, Y, st);
-        if (cols && os2_rows_fast<T>(e, src, ih, iw, start, tab, Y, nimg, h, w, out, part, st)) return;
-        if (cols) {
-            const int g = std::max(1, std::min(elems / w, (81920 - w * int(sizeof(cx<T>))) /
-                                                              (w * int(2 * sizeof(cx<T>) + sizeof(T)))));
-            hipLaunchKernelGGL(k_os2_rows<T>, dim3(idivup(nimg * 2 * h, g)), dim3(256),
-                               (2 * size_t(g) + 1) * w * sizeof(cx<T>) + size_t(g) * w * sizeof(T), st, src, ih, iw,
-                               start, tab, Y, nimg, h, g, f32 ? pr.desc32 : pr.desc64, out);
-            return;
-        }
-    }
+    const FftPlan &pc = e.plan(j.h), &pr = e.plan(j.w);
     // up to 16 columns per block (whole 128-byte row segments) within 80 KB of LDS
-    const int cb = std::max(1, std::min(w, std::min(16, (81920 / int(h * sizeof(cx<T>)) - 1) / 2)));
-    hipLaunchKernelGGL(k_os2_cols<T>, dim3(idivup(w, cb), nimg), dim3(256), (2 * size_t(cb) + 1) * h * sizeof(cx<T>),
-                       st, src, ih, iw, start, tab, w, cb, f32 ? pc.desc32 : pc.desc64, Y);
+    const int cb = std::max(1, std::min(j.w, std::min(16, (81920 / int(j.h * sizeof(cx<T>)) - 1) / 2)));
+    hipLaunchKernelGGL(k_os2_cols<T>, dim3(idivup(j.w, cb), nimg), dim3(256), (2 * size_t(cb) + 1) * j.h * sizeof(cx<T>), st,
+                       j.chip, j.tab, j.w, cb, f32 ? pc.desc32 : pc.desc64, j.Y);
     // rows per block from the element budget, within 80 KB of LDS
-    const int row_bytes = w * int(2 * sizeof(cx<T>) + sizeof(T));
-    const int g = std::max(1, std::min(elems / w, (81920 - w * int(sizeof(cx<T>))) / row_bytes));
-    hipLaunchKernelGGL(k_os2_rows<T>, dim3(idivup(nimg * 2 * h, g)), dim3(256),
-                       (2 * size_t(g) + 1) * w * sizeof(cx<T>) + size_t(g) * w * sizeof(T), st, src, ih, iw, start, tab,
-                       Y, nimg, h, g, f32 ? pr.desc32 : pr.desc64, out);
+    const int row_bytes = j.w * int(2 * sizeof(cx<T>) + sizeof(T)) + 8;
+    const int g = std::max(1, std::min(fft_elems<T>(e) / j.w, (81920 - 8 - j.w * int(sizeof(cx<T>))) / row_bytes));
+    hipLaunchKernelGGL(k_os2_rows<T>, dim3(idivup(nimg * 2 * j.h, g)), dim3(256), os2_rows_lds<T>(g, j.w), st, j.chip, j.tab,
+                       j.Y, nimg, j.h, g, f32 ? pr.desc32 : pr.desc64, j.out);
 }
 
-// Row-spectrum transform lengths with an in-place kernel (k_rowspec_f, FP32):
+// Row-spectrum transform lengths with an in-place kernel (k_rowspec_f):
 // L = R1 * R2, listed by L. The correlation is the same for any L of at least
 // the search width; these cover the uneven windows' search widths with little
 // padding and prime factors <= 17 (which the lag-row inverse needs).
@@ -444,50 +446,73 @@ int row_len_fast(int sw) {
     return 0;
 }
 
-template <int R1, int R2, int G = 8, int NTH = 256>
-void rowspec_launch(Engine &e, const float *img, int nimg, int h, int w, const double *mean, cx<float> *spec,
-                    hipStream_t st) {
-    constexpr int L = R1 * R2;
-    hipLaunchKernelGGL((k_rowspec_f<float, R1, R2, G, NTH>), dim3(idivup(nimg * ((h + 1) / 2), G)), dim3(NTH),
-                       size_t(G) * (L + 1) * sizeof(cx<float>), st, img, nimg, h, w, tw_of<float>(e, L), mean, spec);
+// row pairs per block: 8 (7 of 528 points, one round of work items a pass); 4 in FP64,
+// whose few windows need the workgroups
+template <int R1, int R2, int GF = 8, class T>
+void rowspec_launch(Engine &e, RowJob<T> t, const RowJob<T> &s, int nimg, hipStream_t st) {
+    constexpr int G = sizeof(T) == 8 ? 4 : GF;
+    t.blocks = idivup(nimg * ((t.h + 1) / 2), G);
+    hipLaunchKernelGGL((k_rowspec_f<T, R1, R2, G>), dim3(t.blocks + idivup(nimg * ((s.h + 1) / 2), G)), dim3(256), 0, st, t,
+                       s, nimg, tw_of<T>(e, R1 * R2));
 }
 
-// `mean`: per-image mean subtracted on load (null for none)
-void rowspec_fast(Engine &e, int L, const float *img, int nimg, int h, int w, const double *mean, cx<float> *spec,
-                  hipStream_t st) {
+// half spectra of template and search rows at a listed length
+template <class T>
+void rowspec_fast(Engine &e, int L, const RowJob<T> &t, const RowJob<T> &s, int nimg, hipStream_t st) {
     switch (L) {
-        case 72: rowspec_launch<8, 9>(e, img, nimg, h, w, mean, spec, st); break;
-        case 80: rowspec_launch<16, 5>(e, img, nimg, h, w, mean, spec, st); break;
-        case 104: rowspec_launch<8, 13>(e, img, nimg, h, w, mean, spec, st); break;
-        case 128: rowspec_launch<16, 8>(e, img, nimg, h, w, mean, spec, st); break;
-        case 144: rowspec_launch<16, 9>(e, img, nimg, h, w, mean, spec, st); break;
-        case 168: rowspec_launch<8, 21>(e, img, nimg, h, w, mean, spec, st); break;
-        case 195: rowspec_launch<13, 15>(e, img, nimg, h, w, mean, spec, st); break;
-        case 256: rowspec_launch<16, 16>(e, img, nimg, h, w, mean, spec, st); break;
-        case 272: rowspec_launch<16, 17>(e, img, nimg, h, w, mean, spec, st); break;
-        case 289: rowspec_launch<17, 17>(e, img, nimg, h, w, mean, spec, st); break;
-        case 325: rowspec_launch<13, 25>(e, img, nimg, h, w, mean, spec, st); break;
-        case 528: rowspec_launch<16, 33, 7, 256>(e, img, nimg, h, w, mean, spec, st); break;
+        case 72: rowspec_launch<8, 9>(e, t, s, nimg, st); break;
+        case 80: rowspec_launch<16, 5>(e, t, s, nimg, st); break;
+        case 104: rowspec_launch<8, 13>(e, t, s, nimg, st); break;
+        case 128: rowspec_launch<16, 8>(e, t, s, nimg, st); break;
+        case 144: rowspec_launch<16, 9>(e, t, s, nimg, st); break;
+        case 168: rowspec_launch<8, 21>(e, t, s, nimg, st); break;
+        case 195: rowspec_launch<13, 15>(e, t, s, nimg, st); break;
+        case 256: rowspec_launch<16, 16>(e, t, s, nimg, st); break;
+        case 272: rowspec_launch<16, 17>(e, t, s, nimg, st); break;
+        case 289: rowspec_launch<17, 17>(e, t, s, nimg, st); break;
+        case 325: rowspec_launch<13, 25>(e, t, s, nimg, st); break;
+        case 528: rowspec_launch<16, 33, 7>(e, t, s, nimg, st); break;
         default: throw Error(AMPCOR_E_ARG, "no in-place row transform of length " + std::to_string(L));
     }
 }
 
-// per-window copies of a chunk's outputs (pairs of int32, one T -> float); a
-// null destination or source skips that output
+// a chunk's per-window results to the caller's arrays (pairs of int32; null arrays are
+// skipped). With `to`, the chunk is part of a re-run: window i goes to window to[i] of the
+// caller's arrays, offset, refined offset and zoom peak for every window, the rest for the
+// first `full` only (the others kept their raw stage's results).
 template <class T>
-__global__ void k_chunk_out(int n, const int32_t *loc, int32_t *o_loc, const int32_t *start, int32_t *o_start,
-                            const int32_t *shift, int32_t *o_shift, const int32_t *zidx, int32_t *o_zidx, const T *val,
-                            float *o_val) {
+struct ChunkOut {
+    const int32_t *loc, *start, *shift, *zidx;
+    const T *val;
+    const float *offset, *snr, *cov;          // with `to` only (else written in place)
+    const double *refined;
+    int32_t *o_loc, *o_start, *o_shift, *o_zidx;
+    float *o_val, *o_offset, *o_snr, *o_cov;
+    double *o_refined;
+};
+template <class T>
+__global__ void k_chunk_out(ChunkOut<T> c, int n, const int32_t *to, int full) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    auto pair = [&](const int32_t *s, int32_t *d) {
-        if (s && d) { d[2 * i] = s[2 * i]; d[2 * i + 1] = s[2 * i + 1]; }
+    const size_t w = to ? to[i] : i;
+    auto copy = [&](auto *s, auto *d, int k) {
+        if (s && d)
+            for (int m = 0; m < k; ++m) d[k * w + m] = s[k * size_t(i) + m];
     };
-    pair(loc, o_loc);
-    pair(start, o_start);
-    pair(shift, o_shift);
-    pair(zidx, o_zidx);
-    if (val && o_val) o_val[i] = float(val[i]);
+    copy(c.zidx, c.o_zidx, 2);
+    if (to) {
+        copy(c.offset, c.o_offset, 2);
+        copy(c.refined, c.o_refined, 2);
+    }
+    if (i >= full) return;
+    copy(c.loc, c.o_loc, 2);
+    copy(c.start, c.o_start, 2);
+    copy(c.shift, c.o_shift, 2);
+    if (c.val && c.o_val) c.o_val[w] = float(c.val[i]);
+    if (to) {
+        copy(c.snr, c.o_snr, 1);
+        copy(c.cov, c.o_cov, 3);
+    }
 }
 
 // start[i], shift[i] = the given values for windows f0 <= i < n
@@ -506,7 +531,8 @@ inline dim3 grid2(int per_img, int nimg) { return dim3(std::min(idivup(per_img, 
 // cuAmpcorChunk::run (cuAmpcorChunk.cpp:12-217) over chunks of windows.
 template <class T>
 void Engine::run_staged_t(const RunArgs &a) {
-    const std::string tn = sizeof(T) == 8 ? "d_" : "f_";
+    const bool f32 = sizeof(T) == 4;
+    const std::string tn = f32 ? "f_" : "d_";
     const hipStream_t st = a.stream;
     const int W_h = p.window_h, W_w = p.window_w;
     const int S_h = sz.search_h, S_w = sz.search_w;
@@ -515,28 +541,57 @@ void Engine::run_staged_t(const RunArgs &a) {
     // correlation transform sizes (5-smooth, >= the search chips)
     const int L1h = sz.fft_corr_raw_h, L1w = sz.fft_corr_raw_w, L2h = sz.fft_corr_os_h, L2w = sz.fft_corr_os_w;
     const int Z = sz.zoom, So = sz.surf_out;
+    const int OSh = sz.os_search_h, OSw = sz.os_search_w;   // oversampled zoom chip (fixed by the interpolation)
     const int nb = std::min(chunk, a.n);
-
-    cx<T> *c_ref = buf<cx<T>>(tn + "c_ref", size_t(nb) * W_h * W_w);
-    T *r_ref = buf<T>(tn + "r_ref", size_t(nb) * W_h * W_w);
-    cx<T> *c_sec = buf<cx<T>>(tn + "c_sec", size_t(nb) * S_h * S_w);
-    T *r_sec = buf<T>(tn + "r_sec", size_t(nb) * S_h * S_w);
     auto norm_lds = [](int sw) { return size_t(4 * sw + 2) * sizeof(double); };
-    // block size of the one-block-per-window reductions
-    auto per_window_threads = [](int size) { return size >= 16384 ? 1024 : 256; };
-    double *ssd_raw = buf<double>(tn + "ssd_raw", nb), *ssd_os = buf<double>(tn + "ssd_os", nb);
-    const size_t vmax = std::max(size_t(sz.raw_corr_h) * S_w, size_t(sz.os_corr_h) * sz.os_search_w);
-    double *V1 = buf<double>(tn + "V1", size_t(nb) * vmax), *V2 = buf<double>(tn + "V2", size_t(nb) * vmax);
-    // NCC normalization: barrier-free column/row passes up to 1024 search columns, else one block per window
-    auto normalize = [&](T *c, int ch, int cw, const T *tm, int th, int tw, const T *sr, int sh, int sw,
-                         const double *ssd, int nw) {
+    // block size of the one-block-per-window passes: all the waves a block can have where
+    // the windows alone leave the GPU idle
+    const int per_window = nb < 512 ? 1024 : 256;
+
+    // Correlations through row spectra (k_rowspec, k_mac_lags, k_lagrows_real): row
+    // FFTs of the template and search rows, per-bin sums over template rows for each
+    // lag row, and row IFFTs of the lag rows only. The padded 2-D FFT route remains
+    // for shapes whose row pairs outnumber the transform rows.
+    auto fits_rows = [&](int th, int sh, int Lh) { return (th + 1) / 2 + (sh + 1) / 2 <= Lh; };
+    const bool row_raw = fits_rows(W_h, S_h, L1h), row_os = fits_rows(sz.os_win_h, OSh, L2h);
+    // with them and the two-pass normalization (up to 1024 search columns) no mean-free
+    // template image is needed: the mean is subtracted as the template rows load, and the
+    // raw stage's rows are the amplitudes of chips read in place
+    const bool lean_raw = row_raw && S_w <= 1024, lean_os = row_os && OSw <= 1024;
+    // the separable oversampler covers the x2 interpolation of even-sided chips (an
+    // odd side loses its middle spectrum line to the quadrant padding, which does
+    // not factor into the half-sample form)
+    const bool sep_os = oversampler >= 2 && p.raw_ovs == 2 && sz.os_win_h == 2 * W_h && sz.os_win_w == 2 * W_w &&
+                        OSh == 2 * sz.zoom_in_h && OSw == 2 * sz.zoom_in_w && W_h % 2 == 0 && W_w % 2 == 0 &&
+                        sz.zoom_in_h % 2 == 0 && sz.zoom_in_w % 2 == 0;
+    const bool fast_os = sep_os && oversampler == 2 && os2_has(W_h) && os2_has(W_w) && sz.zoom_in_h == W_h + 8 &&
+                         sz.zoom_in_w == W_w + 8 && os2_has(W_h + 8) && os2_has(W_w + 8);
+    // the oversampled template's mean from the row kernel's block sums
+    const bool part_mean = fast_os && lean_os;
+    // row transform lengths: an in-place length where one is listed
+    const int R1w = row_len_fast(S_w) ? row_len_fast(S_w) : L1w;
+    const int R2w = row_len_fast(OSw) ? row_len_fast(OSw) : L2w;
+
+    cx<T> *c_ref = sep_os ? nullptr : buf<cx<T>>(tn + "c_ref", size_t(nb) * W_h * W_w);
+    cx<T> *c_sec = sep_os ? nullptr : buf<cx<T>>(tn + "c_sec", size_t(nb) * S_h * S_w);
+    T *r_ref = lean_raw ? nullptr : buf<T>(tn + "r_ref", size_t(nb) * W_h * W_w);
+    T *r_sec = buf<T>(tn + "r_sec", size_t(nb) * S_h * S_w);
+    double *mean_raw = buf<double>(tn + "mean_raw", nb), *ssd_raw = buf<double>(tn + "ssd_raw", nb);
+    // row ranges per chip of the raw template's sums
+    const int raw_ranges = nb < 512 ? std::min(8, idivup(W_h * W_w, 2048)) : 1;
+    double *raw_part = buf<double>(tn + "raw_part", size_t(nb) * 2 * raw_ranges);
+    double *mean_os = buf<double>(tn + "mean_os", nb), *ssd_os = buf<double>(tn + "ssd_os", nb);
+    // block sums of the search amplitudes for the window sums (up to 1024 search columns)
+    auto sum_rows = [](int sh) { return size_t(idivup(sh, SUM_BLK)) * 2; };
+    double *sums = buf<double>(tn + "sums", size_t(nb) * std::max(sum_rows(S_h) * S_w, sum_rows(OSh) * OSw));
+    // NCC normalization: lag rows per workgroup within 32 KB of column sums
+    auto normalize = [&](T *c, int ch, int cw, const T *tm, int th, int tw, const T *sr, int sh, int sw, const double *ssd,
+                         int nw) {
         if (sw <= 1024) {
-            hipLaunchKernelGGL(k_colsums<T>, dim3(idivup(sw, 64), nw), dim3(64), 0, st, sr, sh, sw, th, ch, V1, V2);
-            const dim3 g(idivup(nw * ch, 4)), b(256);
-            if (sw <= 128) hipLaunchKernelGGL((k_norm_rows<T, 2>), g, b, 0, st, c, nw, ch, cw, th, tw, V1, V2, sw, ssd);
-            else if (sw <= 256) hipLaunchKernelGGL((k_norm_rows<T, 4>), g, b, 0, st, c, nw, ch, cw, th, tw, V1, V2, sw, ssd);
-            else if (sw <= 576) hipLaunchKernelGGL((k_norm_rows<T, 9>), g, b, 0, st, c, nw, ch, cw, th, tw, V1, V2, sw, ssd);
-            else hipLaunchKernelGGL((k_norm_rows<T, 16>), g, b, 0, st, c, nw, ch, cw, th, tw, V1, V2, sw, ssd);
+            const int K = std::max(1, std::min(8, 32768 / (16 * sw)));
+            hipLaunchKernelGGL(k_block_sums<T>, dim3(idivup(block_sum_tasks(sh, sw), 4), nw), dim3(256), 0, st, sr, sh, sw, sums);
+            hipLaunchKernelGGL(k_norm_lags<T>, dim3(idivup(ch, K), nw), dim3(256), size_t(16) * K * sw, st, c, ch, cw, th, tw,
+                               sr, sh, sw, sums, ssd, K);
         } else {
             hipLaunchKernelGGL(k_normalize<T>, dim3(nw), dim3(256), norm_lds(sw), st, c, ch, cw, tm, th, tw, sr, sh, sw);
         }
@@ -544,83 +599,80 @@ void Engine::run_staged_t(const RunArgs &a) {
     T *corr = buf<T>(tn + "corr", size_t(nb) * sz.raw_corr_h * sz.raw_corr_w);
     int32_t *loc = buf<int32_t>(tn + "loc", size_t(nb) * 2);
     T *val = buf<T>(tn + "val", nb);
-    int32_t *start = buf<int32_t>(tn + "start", size_t(nb) * 2);
-    int32_t *shift = buf<int32_t>(tn + "shift", size_t(nb) * 2);
+    int32_t *start_buf = buf<int32_t>(tn + "start", size_t(nb) * 2), *shift_buf = buf<int32_t>(tn + "shift", size_t(nb) * 2);
     int32_t *zidx = buf<int32_t>(tn + "zidx", size_t(nb) * 2);
-    cx<T> *c_ref_os = buf<cx<T>>(tn + "c_ref_os", size_t(nb) * sz.os_win_h * sz.os_win_w);
+    // a re-run's outputs, scattered to the caller's windows at the end of the chunk
+    const bool scatter = a.scatter != nullptr;
+    float *o_off = scatter ? buf<float>(tn + "o_off", size_t(nb) * 2) : nullptr;
+    float *o_snr = scatter ? buf<float>(tn + "o_snr", nb) : nullptr, *o_cov = scatter ? buf<float>(tn + "o_cov", size_t(nb) * 3) : nullptr;
+    double *o_refined = scatter && a.refined ? buf<double>(tn + "o_refined", size_t(nb) * 2) : nullptr;
+    cx<T> *c_ref_os = buf<cx<T>>(tn + "c_ref_os", size_t(nb) * (sep_os ? size_t(W_h) * W_w : size_t(sz.os_win_h) * sz.os_win_w));
     T *r_ref_os = buf<T>(tn + "r_ref_os", size_t(nb) * sz.os_win_h * sz.os_win_w);
-    cx<T> *c_zoom = buf<cx<T>>(tn + "c_zoom", size_t(nb) * sz.zoom_in_h * sz.zoom_in_w);
+    cx<T> *c_zoom = sep_os ? nullptr : buf<cx<T>>(tn + "c_zoom", size_t(nb) * sz.zoom_in_h * sz.zoom_in_w);
     // deramp rotation tables (row then column factors per chip)
-    cx<double> *dtab = p.deramp == 1 ? buf<cx<double>>(tn + "dtab", size_t(nb) * (std::max(W_h + W_w,
-                                                                 sz.zoom_in_h + sz.zoom_in_w))) : nullptr;
-    const int OSh = sz.os_search_h, OSw = sz.os_search_w;   // oversampled zoom chip (fixed by the interpolation)
-    // the separable oversampler covers the x2 interpolation of even-sided chips (an
-    // odd side loses its middle spectrum line to the quadrant padding, which does
-    // not factor into the half-sample form)
-    const bool sep_os = oversampler >= 2 && p.raw_ovs == 2 && sz.os_win_h == 2 * W_h && sz.os_win_w == 2 * W_w &&
-                        OSh == 2 * sz.zoom_in_h && OSw == 2 * sz.zoom_in_w && W_h % 2 == 0 && W_w % 2 == 0 &&
-                        sz.zoom_in_h % 2 == 0 && sz.zoom_in_w % 2 == 0;
-    cx<T> *c_sec_os = buf<cx<T>>(tn + "c_sec_os", size_t(nb) * OSh * OSw);
+    cx<double> *dtab_r = p.deramp == 1 ? buf<cx<double>>(tn + "dtab_r", size_t(nb) * (W_h + W_w)) : nullptr;
+    cx<double> *dtab_s = p.deramp == 1 ? buf<cx<double>>(tn + "dtab_s", size_t(nb) * (sz.zoom_in_h + sz.zoom_in_w)) : nullptr;
+    cx<T> *c_sec_os = buf<cx<T>>(tn + "c_sec_os", size_t(nb) * (sep_os ? size_t(sz.zoom_in_h) * sz.zoom_in_w : size_t(OSh) * OSw));
     T *r_sec_os = buf<T>(tn + "r_sec_os", size_t(nb) * OSh * OSw);
     T *corr_os = buf<T>(tn + "corr_os", size_t(nb) * sz.os_corr_h * sz.os_corr_w);
-    // Correlations through row spectra (k_rowspec, k_mac_lags, k_lagrows_real): row
-    // FFTs of the template and search rows, per-bin sums over template rows for each
-    // lag row, and row IFFTs of the lag rows only. The padded 2-D FFT route remains
-    // for shapes whose row pairs outnumber the transform rows.
-    auto fits_rows = [&](int th, int sh, int Lh) { return (th + 1) / 2 + (sh + 1) / 2 <= Lh; };
-    const bool row_raw = fits_rows(W_h, S_h, L1h), row_os = fits_rows(sz.os_win_h, OSh, L2h);
-    // row transform lengths: an in-place length for the FP32 passes where one is listed
-    const bool f32 = sizeof(T) == 4;
-    const int R1w = f32 && row_len_fast(S_w) ? row_len_fast(S_w) : L1w;
-    const int R2w = f32 && row_len_fast(OSw) ? row_len_fast(OSw) : L2w;
-    // the oversampled template's mean from the row kernel's block sums, subtracted
-    // as the row spectra load it (no k_sub_mean pass), where every piece applies:
-    // FP32, separable in-place rows, whole-chip blocks, the in-place row spectra,
-    // and the normalization that needs no mean-free template image (search <= 1024)
-    const bool fuse_mean = f32 && sep_os && oversampler == 2 && os2_rows_has(W_w) && os2_rows_has(W_h) &&
-                           sz.os_win_h % os2_rows_per_block<T>(W_w) == 0 && row_os && R2w != L2w && OSw <= 1024;
-    double *os_part = fuse_mean ? buf<double>(tn + "os_part", size_t(nb) * 2 * (sz.os_win_h / os2_rows_per_block<T>(W_w)))
-                                : nullptr;
-    double *os_mean = fuse_mean ? buf<double>(tn + "os_mean", nb) : nullptr;
+    const int nparts = sz.os_win_h / os2_rows_per_block<T>(W_w);
+    double *os_part = part_mean ? buf<double>(tn + "os_part", size_t(nb) * 2 * nparts) : nullptr;
     size_t zmax = 0;
     if (!row_raw) zmax = size_t(L1h) * L1w;
     if (!row_os) zmax = std::max(zmax, size_t(L2h) * L2w);
     cx<T> *zc = zmax ? buf<cx<T>>(tn + "zc", size_t(nb) * zmax) : nullptr;
-    size_t spec_elems = 0, q_elems = 0;
+    // few windows (FP64): parts of the template rows whose lag sums are taken apart (k_lag_parts),
+    // enough of 16 rows or more to leave about 4096 waves
+    constexpr int KLAG = 9;
+    auto lag_parts = [&](int th, int NL, int H1, int n) {
+        const int tasks = n * idivup(H1, 64) * idivup(NL, KLAG);
+        return std::max(1, std::min(idivup(th, 16), idivup(4096, tasks)));
+    };
+    // most window parts of any chunk of up to nb windows
+    auto part_windows = [&](int th, int NL, int H1) {
+        return std::min(size_t(nb) * idivup(th, 16), size_t(nb) + 4096 / (idivup(H1, 64) * idivup(NL, KLAG)) + 1);
+    };
+    size_t spec_elems = 0, q_total = 0;
+    auto lag_rows = [&](bool lean, int th, int NL, int L) {
+        const int H1 = L / 2 + 1;
+        q_total = std::max(q_total, f32 || !lean ? size_t(nb) * NL * L : part_windows(th, NL, H1) * NL * H1);
+    };
     if (row_raw) {
         spec_elems = std::max(spec_elems, size_t(W_h + S_h) * (R1w / 2 + 1));
-        q_elems = std::max(q_elems, size_t(sz.raw_corr_h) * R1w);
+        lag_rows(lean_raw, W_h, sz.raw_corr_h, R1w);
     }
     if (row_os) {
         spec_elems = std::max(spec_elems, size_t(sz.os_win_h + OSh) * (R2w / 2 + 1));
-        q_elems = std::max(q_elems, size_t(sz.os_corr_h) * R2w);
+        lag_rows(lean_os, sz.os_win_h, sz.os_corr_h, R2w);
     }
     cx<T> *rspec = spec_elems ? buf<cx<T>>(tn + "rspec", size_t(nb) * spec_elems) : nullptr;
-    cx<T> *rq = q_elems ? buf<cx<T>>(tn + "rq", size_t(nb) * q_elems) : nullptr;
-    // tmean: the template's mean, subtracted as its rows load (FP32 in-place row path), or null
-    auto row_correlate = [&](const T *tm, int th, int tw, const T *sr, int sh, int sw, int L, int NL, int NLw,
-                             T *out, int n, const double *tmean) {
+    cx<T> *rq = q_total ? buf<cx<T>>(tn + "rq", q_total) : nullptr;
+    // row half spectra of the template (mean subtracted on load when given) and the search
+    auto row_spectra = [&](RowJob<T> t, RowJob<T> s, int L, int n) {
+        t.spec = rspec;
+        s.spec = rspec + size_t(n) * t.h * (L / 2 + 1);
+        if (row_len_fast(s.w) == L) {
+            rowspec_fast<T>(*this, L, t, s, n, st);
+            return;
+        }
+        const FftPlan &pl = plan(L);
+        const int g = std::max(1, fft_elems<T>(*this) / L);
+        t.blocks = idivup(n * ((t.h + 1) / 2), g);
+        hipLaunchKernelGGL(k_rowspec<T>, dim3(t.blocks + idivup(n * ((s.h + 1) / 2), g)), dim3(256),
+                           size_t(g) * (2 * L * sizeof(cx<T>) + sizeof(int64_t) + sizeof(T)), st, t, s, n, g,
+                           f32 ? pl.desc32 : pl.desc64);
+    };
+    // lag sums and their inverse transform (not normalized)
+    auto row_correlate = [&](int th, int sh, int L, int NL, int NLw, T *out, int n) {
         const int H1 = L / 2 + 1;
         const FftPlan &pl = plan(L);
-        const FftDesc &d = sizeof(T) == 4 ? pl.desc32 : pl.desc64;
+        const FftDesc &d = f32 ? pl.desc32 : pl.desc64;
         const int g = std::max(1, fft_elems<T>(*this) / L);
         const size_t lds = 2 * size_t(g) * L * sizeof(cx<T>);
         cx<T> *tspec = rspec, *sspec = rspec + size_t(n) * th * H1;
-        if (sizeof(T) == 4 && row_len_fast(sw) == L) {
-            rowspec_fast(*this, L, reinterpret_cast<const float *>(tm), n, th, tw, tmean,
-                         reinterpret_cast<cx<float> *>(tspec), st);
-            rowspec_fast(*this, L, reinterpret_cast<const float *>(sr), n, sh, sw, nullptr,
-                         reinterpret_cast<cx<float> *>(sspec), st);
-        } else {
-            hipLaunchKernelGGL(k_rowspec<T>, dim3(idivup(n * ((th + 1) / 2), g)), dim3(256), lds, st, tm, n, th, tw, g,
-                               d, tspec);
-            hipLaunchKernelGGL(k_rowspec<T>, dim3(idivup(n * ((sh + 1) / 2), g)), dim3(256), lds, st, sr, n, sh, sw, g,
-                               d, sspec);
-        }
         // lags per thread: 17 once there is more than one group of 9 (each group
         // re-reads every spectrum; the sums themselves do not depend on the
-        // grouping), unless that leaves too few workgroups to fill the GPU (the
-        // FP64 re-run of a few hundred windows)
+        // grouping), unless that leaves too few workgroups to fill the GPU
         if (NL > 9 && n * idivup(H1, 64) >= 2048)
             hipLaunchKernelGGL((k_mac_lags<T, 17, 2>), dim3(idivup(H1, 64), idivup(NL, 17), n), dim3(128), 0, st, tspec,
                                th, sspec, sh, NL, L, rq, T(1.0 / double(L)));
@@ -628,6 +680,37 @@ void Engine::run_staged_t(const RunArgs &a) {
             hipLaunchKernelGGL((k_mac_lags<T, 9, 4>), dim3(idivup(H1, 64), idivup(NL, 9), n), dim3(256), 0, st, tspec,
                                th, sspec, sh, NL, L, rq, T(1.0 / double(L)));
         hipLaunchKernelGGL(k_lagrows_real<T>, dim3(idivup(n * NL, g)), dim3(256), lds, st, rq, n * NL, g, d, NLw, out);
+    };
+    // normalized correlation through row spectra
+    auto row_ncc = [&](const RowJob<T> &t, const RowJob<T> &s, const T *tm, const T *sr, int L, int NL, int NLw, const double *ssd,
+                       T *out, bool lean, int n) {
+        row_spectra(t, s, L, n);
+        if constexpr (sizeof(T) == 8) {
+            if (lean) {
+                const int H1 = L / 2 + 1, parts = lag_parts(t.h, NL, H1, n);
+                const int lag_blocks = idivup(parts * idivup(H1, 64) * idivup(NL, KLAG), 4);
+                hipLaunchKernelGGL((k_lag_parts<T, KLAG>), dim3(lag_blocks + idivup(block_sum_tasks(s.h, s.w), 4), n), dim3(256),
+                                   0, st, rspec, t.h, rspec + size_t(n) * t.h * H1, s.h, NL, H1, parts, rq, lag_blocks, sr, s.w,
+                                   sums);
+                // lag rows per workgroup: one until the windows alone fill the GPU
+                const int K = n * NL >= 4096 && corr_lags_lds<T>(4, L, s.w) <= 64 * 1024 ? 4 : 1;
+                hipLaunchKernelGGL(k_corr_lags<T>, dim3(idivup(NL, K), n), dim3(256), corr_lags_lds<T>(K, L, s.w), st, rq, parts,
+                                   L, NL, NLw, t.h, t.w, sr, s.h, s.w, sums, ssd, tw_of<T>(*this, L), out, K);
+                return;
+            }
+        }
+        row_correlate(t.h, s.h, L, NL, NLw, out, n);
+        normalize(out, NL, NLw, tm, t.h, t.w, sr, s.h, s.w, ssd, n);
+    };
+    // ... through the padded 2-D FFT of two packed real images
+    auto fft_ncc = [&](const T *tm, int th, int tw, const T *sr, int sh, int sw, int Lh, int Lw, int NL, int NLw, const double *ssd,
+                       T *out, int n) {
+        hipLaunchKernelGGL(k_pack_corr<T>, grid2(Lh * Lw, n), dim3(256), 0, st, tm, th, tw, sr, sh, sw, zc, Lh, Lw);
+        fft2<T, -1>(*this, zc, n, Lh, Lw, st);
+        hipLaunchKernelGGL(k_spec_product<T>, grid2(Lh * Lw, n), dim3(256), 0, st, zc, Lh, Lw, T(1.0 / (double(Lh) * Lw)));
+        fft2_rows_kept<T, +1>(*this, zc, n, Lh, Lw, NL, st);
+        hipLaunchKernelGGL(k_crop_real<T>, grid2(NL * NLw, n), dim3(256), 0, st, zc, Lh, Lw, out, NL, NLw);
+        normalize(out, NL, NLw, tm, th, tw, sr, sh, sw, ssd, n);
     };
     // the 16-sparse surface kernel and the sinc patch kernel keep no surface in HBM
     // (190 windows of 256 at factor 32: 3.10 ms with 512 x 512 surfaces transformed and
@@ -640,103 +723,108 @@ void Engine::run_staged_t(const RunArgs &a) {
     T *r_surf = full_surface ? buf<T>(tn + "r_surf", size_t(nb) * So * So) : nullptr;
     if (p.surf_method) ensure_sinc_table();
 
-    // windows from a.fine_from on have their coarse zoom start and shift given
-    // (a re-run of windows whose coarse peak is not in doubt): chunks of only
-    // such windows skip the raw stage; in a mixed chunk they are overwritten
-    // after it
+    // windows from a.fine_from on have their coarse zoom start and shift given (a re-run
+    // of windows whose coarse peak is not in doubt): the raw stage runs for the others only
     const bool given = a.fine_start != nullptr;
     for (int w0 = 0; w0 < a.n; w0 += nb) {
         const int n = std::min(nb, a.n - w0);
-        const bool fine_only = given && w0 >= a.fine_from;
-        // chip load + amplitude + mean (cuAmpcorChunk.cpp:18-39)
-        hipLaunchKernelGGL(k_gather<T>, grid2(W_h * W_w, n), dim3(256), 0, st, a.ref, a.ref_pitch,
-                           a.ref_d + w0, a.ref_a + w0, W_h, W_w, mode, c_ref, fine_only ? nullptr : r_ref);
-        hipLaunchKernelGGL(k_gather<T>, grid2(S_h * S_w, n), dim3(256), 0, st, a.sec, a.sec_pitch,
-                           a.sec_d + w0, a.sec_a + w0, S_h, S_w, mode, c_sec, fine_only ? nullptr : r_sec);
-        if (fine_only) {
-            HIP_OK(hipMemcpyAsync(start, a.fine_start + 2 * size_t(w0), sizeof(int32_t) * 2 * n,
-                                  hipMemcpyDeviceToDevice, st));
-            HIP_OK(hipMemcpyAsync(shift, a.fine_shift + 2 * size_t(w0), sizeof(int32_t) * 2 * n,
-                                  hipMemcpyDeviceToDevice, st));
+        const int nraw = given ? std::min(n, std::max(0, a.fine_from - w0)) : n;
+        const ChipSrc ref{a.ref, a.ref_pitch, a.ref_d + w0, a.ref_a + w0, nullptr, mode};
+        const ChipSrc sec{a.sec, a.sec_pitch, a.sec_d + w0, a.sec_a + w0, nullptr, mode};
+        // chip load + amplitude + mean (cuAmpcorChunk.cpp:18-39), for the shapes that read
+        // no chip in place
+        if (!sep_os || (!lean_raw && nraw)) {
+            cx<T> *cr = c_ref ? c_ref : buf<cx<T>>(tn + "c_ref", size_t(nb) * W_h * W_w);
+            cx<T> *cs = c_sec ? c_sec : buf<cx<T>>(tn + "c_sec", size_t(nb) * S_h * S_w);
+            hipLaunchKernelGGL(k_gather<T>, grid2(W_h * W_w, n), dim3(256), 0, st, ref, W_h, W_w, cr, r_ref);
+            hipLaunchKernelGGL(k_gather<T>, grid2(S_h * S_w, n), dim3(256), 0, st, sec, S_h, S_w, cs, lean_raw ? nullptr : r_sec);
+        }
+        float *snr = scatter ? o_snr : a.snr + w0, *cov = scatter ? o_cov : a.cov + 3 * size_t(w0);
+        const int32_t *start = start_buf, *shift = shift_buf;
+        if (nraw == 0) {
+            start = a.fine_start + 2 * size_t(w0);
+            shift = a.fine_shift + 2 * size_t(w0);
         } else {
-            hipLaunchKernelGGL(k_sub_mean<T>, dim3(n), dim3(per_window_threads(W_h * W_w)), 0, st, r_ref, W_h * W_w,
-                               ssd_raw);
-            // raw correlation (cuAmpcorChunk.cpp:48-52)
-            if (row_raw) {
-                row_correlate(r_ref, W_h, W_w, r_sec, S_h, S_w, R1w, sz.raw_corr_h, sz.raw_corr_w, corr, n, nullptr);
+            // raw correlation, normalized (cuAmpcorChunk.cpp:48-60)
+            if (lean_raw) {
+                hipLaunchKernelGGL(k_chip_sums<T>, dim3(nraw, raw_ranges), dim3(256), 0, st, ref, W_h, W_w, raw_part);
+                hipLaunchKernelGGL(k_mean_parts, dim3(idivup(nraw, 4)), dim3(256), 0, st, raw_part, raw_ranges, W_h * W_w, nraw,
+                                   mean_raw, ssd_raw);
+                row_ncc(RowJob<T>{nullptr, ref, W_h, W_w, mean_raw, nullptr, nullptr, 0},
+                        RowJob<T>{nullptr, sec, S_h, S_w, nullptr, nullptr, r_sec, 0}, nullptr, r_sec, R1w, sz.raw_corr_h,
+                        sz.raw_corr_w, ssd_raw, corr, true, nraw);
             } else {
-                hipLaunchKernelGGL(k_pack_corr<T>, grid2(L1h * L1w, n), dim3(256), 0, st, r_ref, W_h, W_w, r_sec,
-                                   S_h, S_w, zc, L1h, L1w);
-                fft2<T, -1>(*this, zc, n, L1h, L1w, st);
-                hipLaunchKernelGGL(k_spec_product<T>, grid2(L1h * L1w, n), dim3(256), 0, st, zc, L1h, L1w,
-                                   T(1.0 / (double(L1h) * L1w)));
-                fft2_rows_kept<T, +1>(*this, zc, n, L1h, L1w, sz.raw_corr_h, st);
-                hipLaunchKernelGGL(k_crop_real<T>, grid2(sz.raw_corr_h * sz.raw_corr_w, n), dim3(256), 0, st, zc,
-                                   L1h, L1w, corr, sz.raw_corr_h, sz.raw_corr_w);
+                hipLaunchKernelGGL(k_sub_mean<T>, dim3(nraw), dim3(per_window), 0, st, r_ref, W_h * W_w,
+                                   ssd_raw);
+                if (row_raw)
+                    row_ncc(RowJob<T>{r_ref, {}, W_h, W_w, nullptr, nullptr, nullptr, 0},
+                            RowJob<T>{r_sec, {}, S_h, S_w, nullptr, nullptr, nullptr, 0}, r_ref, r_sec, R1w, sz.raw_corr_h,
+                            sz.raw_corr_w, ssd_raw, corr, false, nraw);
+                else
+                    fft_ncc(r_ref, W_h, W_w, r_sec, S_h, S_w, L1h, L1w, sz.raw_corr_h, sz.raw_corr_w, ssd_raw, corr, nraw);
             }
-            // normalize (cuAmpcorChunk.cpp:60)
-            normalize(corr, sz.raw_corr_h, sz.raw_corr_w, r_ref, W_h, W_w, r_sec, S_h, S_w, ssd_raw, n);
             // argmax, covariance, SNR, zoom start/shift (cuAmpcorChunk.cpp:69-106)
-            hipLaunchKernelGGL(k_maxloc<T>, dim3(n), dim3(256), 0, st, corr, sz.raw_corr_h, sz.raw_corr_w, loc, val,
-                               a.margin_coarse ? a.margin_coarse + w0 : nullptr);
-            hipLaunchKernelGGL(k_stats<T>, dim3(n), dim3(64), 0, st, corr, sz.raw_corr_h, sz.raw_corr_w, n,
-                               loc, val, W_h * W_w, sz.corr_raw_zoom_h, sz.corr_raw_zoom_w, p.hs_down, p.hs_across,
-                               sz.half_zoom, a.cov + 3 * size_t(w0), a.snr + w0, start, shift);
-            if (given && a.fine_from < w0 + n) {
-                const int f0 = a.fine_from - w0;
-                hipLaunchKernelGGL(k_given_starts, dim3(idivup(n - f0, 256)), dim3(256), 0, st,
-                                   a.fine_start + 2 * size_t(w0), a.fine_shift + 2 * size_t(w0), f0, n, start, shift);
+            hipLaunchKernelGGL(k_peak<T>, dim3(nraw), dim3(256), 0, st, corr, sz.raw_corr_h, sz.raw_corr_w, W_h * W_w,
+                               sz.corr_raw_zoom_h, sz.corr_raw_zoom_w, p.hs_down, p.hs_across, sz.half_zoom, loc, val,
+                               a.margin_coarse ? a.margin_coarse + w0 : nullptr, cov, snr, start_buf, shift_buf);
+            if (nraw < n)
+                hipLaunchKernelGGL(k_given_starts, dim3(idivup(n - nraw, 256)), dim3(256), 0, st,
+                                   a.fine_start + 2 * size_t(w0), a.fine_shift + 2 * size_t(w0), nraw, n, start_buf, shift_buf);
+        }
+        // oversampling of the reference chips and the zoom chips (cuAmpcorChunk.cpp:115-137)
+        ChipSrc zoom = sec;
+        zoom.start = start;
+        if (p.deramp == 1)
+            hipLaunchKernelGGL(k_deramp_phase, dim3(n, 2), dim3(per_window), 0, st,
+                               PhaseJob{ref, W_h, W_w, dtab_r}, PhaseJob{zoom, sz.zoom_in_h, sz.zoom_in_w, dtab_s});
+        if (sep_os) {
+            OsJob<T> jr{ref, dtab_r, W_h, W_w, nullptr, nullptr, nullptr, nullptr, c_ref_os, r_ref_os, os_part, 0};
+            OsJob<T> js{zoom, dtab_s, sz.zoom_in_h, sz.zoom_in_w, nullptr, nullptr, nullptr, nullptr, c_sec_os, r_sec_os,
+                        nullptr, 0};
+            if (fast_os) {
+                for (OsJob<T> *j : {&jr, &js}) {
+                    j->tw_h = tw_of<T>(*this, j->h);
+                    j->tw_w = tw_of<T>(*this, j->w);
+                    j->shift_h = half_shifts<T>(j->h);
+                    j->shift_w = half_shifts<T>(j->w);
+                }
+                os2_both(*this, jr, js, n, st);
+            } else {
+                os2_general<T>(*this, jr, n, st);
+                os2_general<T>(*this, js, n, st);
             }
-        }
-        // reference oversampling (cuAmpcorChunk.cpp:115-126)
-        if (p.deramp == 1)
-            hipLaunchKernelGGL(k_deramp_phase<T>, dim3(n), dim3(per_window_threads(W_h * W_w)), 0, st, c_ref, W_h, W_w,
-                               (const int32_t *)nullptr, W_h, W_w, dtab);
-        if (sep_os) {
-            os2_separable<T>(*this, c_ref, W_h, W_w, nullptr, p.deramp == 1 ? dtab : nullptr, n, W_h, W_w, c_ref_os,
-                             r_ref_os, st, fuse_mean ? os_part : nullptr);
         } else {
-            fft2_chip<T, +1>(*this, c_ref, W_h, W_w, nullptr, p.deramp == 1 ? dtab : nullptr, c_ref, n, W_h, W_w, st);
+            fft2_chip<T, +1>(*this, c_ref, W_h, W_w, nullptr, dtab_r, c_ref, n, W_h, W_w, st);
             fft2_quad<T, -1, 1>(*this, c_ref, n, W_h, W_w, c_ref_os, sz.os_win_h, sz.os_win_w, r_ref_os, st);
-        }
-        if (fuse_mean)
-            hipLaunchKernelGGL(k_mean_parts, dim3(idivup(n, 256)), dim3(256), 0, st, os_part,
-                               sz.os_win_h / os2_rows_per_block<T>(W_w), sz.os_win_h * sz.os_win_w, n, os_mean, ssd_os);
-        else
-            hipLaunchKernelGGL(k_sub_mean<T>, dim3(n), dim3(per_window_threads(sz.os_win_h * sz.os_win_w)), 0, st,
-                               r_ref_os, sz.os_win_h * sz.os_win_w, ssd_os);
-        // secondary zoom-in crop and oversampling (cuAmpcorChunk.cpp:134-137)
-        if (p.deramp == 1)
-            hipLaunchKernelGGL(k_deramp_phase<T>, dim3(n), dim3(per_window_threads(sz.zoom_in_h * sz.zoom_in_w)), 0,
-                               st, c_sec, S_h, S_w, start, sz.zoom_in_h, sz.zoom_in_w, dtab);
-        if (sep_os) {
-            os2_separable<T>(*this, c_sec, S_h, S_w, start, p.deramp == 1 ? dtab : nullptr, n, sz.zoom_in_h,
-                             sz.zoom_in_w, c_sec_os, r_sec_os, st);
-        } else {
-            fft2_chip<T, +1>(*this, c_sec, S_h, S_w, start, p.deramp == 1 ? dtab : nullptr, c_zoom, n, sz.zoom_in_h,
-                             sz.zoom_in_w, st);
+            fft2_chip<T, +1>(*this, c_sec, S_h, S_w, start, dtab_s, c_zoom, n, sz.zoom_in_h, sz.zoom_in_w, st);
             fft2_quad<T, -1, 1>(*this, c_zoom, n, sz.zoom_in_h, sz.zoom_in_w, c_sec_os, OSh, OSw, r_sec_os, st);
         }
-        // oversampled correlation + normalize (cuAmpcorChunk.cpp:148-161)
-        if (row_os) {
-            row_correlate(r_ref_os, sz.os_win_h, sz.os_win_w, r_sec_os, OSh, OSw, R2w, sz.os_corr_h, sz.os_corr_w,
-                          corr_os, n, fuse_mean ? os_mean : nullptr);
+        // oversampled correlation, normalized (cuAmpcorChunk.cpp:148-161)
+        if (lean_os) {
+            if (part_mean)
+                hipLaunchKernelGGL(k_mean_parts, dim3(idivup(n, 4)), dim3(256), 0, st, os_part, nparts, sz.os_win_h * sz.os_win_w,
+                                   n, mean_os, ssd_os);
+            else
+                hipLaunchKernelGGL(k_array_mean<T>, dim3(n), dim3(per_window), 0, st,
+                                   r_ref_os, sz.os_win_h * sz.os_win_w, mean_os, ssd_os);
+            row_ncc(RowJob<T>{r_ref_os, {}, sz.os_win_h, sz.os_win_w, mean_os, nullptr, nullptr, 0},
+                    RowJob<T>{r_sec_os, {}, OSh, OSw, nullptr, nullptr, nullptr, 0}, nullptr, r_sec_os, R2w, sz.os_corr_h,
+                    sz.os_corr_w, ssd_os, corr_os, true, n);
         } else {
-            hipLaunchKernelGGL(k_pack_corr<T>, grid2(L2h * L2w, n), dim3(256), 0, st, r_ref_os, sz.os_win_h,
-                               sz.os_win_w, r_sec_os, OSh, OSw, zc, L2h, L2w);
-            fft2<T, -1>(*this, zc, n, L2h, L2w, st);
-            hipLaunchKernelGGL(k_spec_product<T>, grid2(L2h * L2w, n), dim3(256), 0, st, zc, L2h, L2w,
-                               T(1.0 / (double(L2h) * L2w)));
-            fft2_rows_kept<T, +1>(*this, zc, n, L2h, L2w, sz.os_corr_h, st);
-            hipLaunchKernelGGL(k_crop_real<T>, grid2(sz.os_corr_h * sz.os_corr_w, n), dim3(256), 0, st, zc, L2h, L2w,
-                               corr_os, sz.os_corr_h, sz.os_corr_w);
+            hipLaunchKernelGGL(k_sub_mean<T>, dim3(n), dim3(per_window), 0, st, r_ref_os,
+                               sz.os_win_h * sz.os_win_w, ssd_os);
+            if (row_os)
+                row_ncc(RowJob<T>{r_ref_os, {}, sz.os_win_h, sz.os_win_w, nullptr, nullptr, nullptr, 0},
+                        RowJob<T>{r_sec_os, {}, OSh, OSw, nullptr, nullptr, nullptr, 0}, r_ref_os, r_sec_os, R2w, sz.os_corr_h,
+                        sz.os_corr_w, ssd_os, corr_os, false, n);
+            else
+                fft_ncc(r_ref_os, sz.os_win_h, sz.os_win_w, r_sec_os, OSh, OSw, L2h, L2w, sz.os_corr_h, sz.os_corr_w, ssd_os,
+                        corr_os, n);
         }
-        normalize(corr_os, sz.os_corr_h, sz.os_corr_w, r_ref_os, sz.os_win_h, sz.os_win_w, r_sec_os, OSh, OSw,
-                  ssd_os, n);
         // trim + surface oversampling + argmax + sub-pixel offset (cuAmpcorChunk.cpp:169-207)
         float *mf = a.margin_fine ? a.margin_fine + w0 : nullptr;
         const float ratio = 1.0f / float(p.surf_ovs * p.raw_ovs);
-        float *off = a.offset + 2 * size_t(w0);
+        float *off = scatter ? o_off : a.offset + 2 * size_t(w0);
         if (fast_surface) {
             // 16-sparse spectrum: one kernel instead of trim, FFT, pad, inverse FFT, real part, argmax
             const int M = p.surf_ovs;
@@ -763,17 +851,20 @@ void Engine::run_staged_t(const RunArgs &a) {
             hipLaunchKernelGGL(k_subpixel, dim3(idivup(n, 64)), dim3(64), 0, st, start, zidx, n, ratio, p.hs_down,
                                p.hs_across, off);
         }
-        if (a.refined)
+        double *refined = !a.refined ? nullptr : scatter ? o_refined : a.refined + 2 * size_t(w0);
+        if (refined)
             hipLaunchKernelGGL(k_refine<T>, dim3(n), dim3(64), refine_lds(Z), st, corr_os, sz.os_corr_h, sz.os_corr_w,
                                Z, p.surf_ovs, 1.0 / double(p.surf_ovs * p.raw_ovs), zidx, start, p.hs_down,
-                               p.hs_across, static_cast<const cx<double> *>(plan(So).tw64.ptr),
-                               a.refined + 2 * size_t(w0));
-        // the chunk's integer results and peak value to the caller's arrays, one launch
+                               p.hs_across, static_cast<const cx<double> *>(plan(So).tw64.ptr), refined);
+        // the chunk's integer results and peak value to the caller's arrays (all results of a
+        // re-run), one launch
         {
-            auto at = [&](int32_t *o) { return o ? o + 2 * size_t(w0) : nullptr; };
-            hipLaunchKernelGGL(k_chunk_out<T>, dim3(idivup(n, 256)), dim3(256), 0, st, n, fine_only ? nullptr : loc,
-                               at(a.maxloc), start, at(a.start), shift, at(a.shift), zidx, at(a.zoom_idx),
-                               fine_only ? nullptr : val, a.maxval ? a.maxval + w0 : nullptr);
+            auto at = [&](auto *o, int k) { return o && !scatter ? o + size_t(k) * w0 : o; };
+            const ChunkOut<T> o{loc, start, shift, zidx, val, o_off, o_snr, o_cov, refined,
+                                at(a.maxloc, 2), at(a.start, 2), at(a.shift, 2), at(a.zoom_idx, 2), at(a.maxval, 1),
+                                a.offset, a.snr, a.cov, a.refined};
+            hipLaunchKernelGGL(k_chunk_out<T>, dim3(idivup(n, 256)), dim3(256), 0, st, o, n,
+                               scatter ? a.scatter + w0 : nullptr, scatter ? std::max(0, a.full - w0) : nraw);
         }
         HIP_OK(hipGetLastError());
     }
@@ -918,11 +1009,6 @@ __global__ void k_first_bad(const int32_t *rd, const int32_t *ra, const int32_t 
 }
 
 __global__ void k_set_i32(int32_t *p, int v) { *p = v; }
-template <class U>
-__global__ void k_put(const U *src, const int32_t *idx, U *dst, int n, int width) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n * width) dst[size_t(idx[i / width]) * width + i % width] = src[i];
-}
 }  // namespace
 
 // Re-run in FP64 (staged pipeline, T = double) every window whose coarse or
@@ -962,43 +1048,21 @@ void Engine::rerun_fp64(const RunArgs &a, const float *mc, const float *mf, cons
     int32_t *st4 = buf<int32_t>("p_starts", size_t(8) * m);
     hipLaunchKernelGGL(k_take_starts, dim3(idivup(m, 256)), dim3(256), 0, a.stream, a.ref_d, a.ref_a, a.sec_d,
                        a.sec_a, m_full < m ? start32 : nullptr, m_full < m ? shift32 : nullptr, d_idx, m, st4);
-    float *o_off = buf<float>("p_off", size_t(2) * m), *o_snr = buf<float>("p_snr", m);
-    float *o_cov = buf<float>("p_cov", size_t(3) * m), *o_val = buf<float>("p_val", m);
-    int32_t *o_i = buf<int32_t>("p_ints", size_t(8) * m);
     RunArgs sub = a;
     sub.ref_d = st4; sub.ref_a = st4 + m; sub.sec_d = st4 + 2 * m; sub.sec_a = st4 + 3 * m;
     sub.n = m;
     sub.margin_coarse = sub.margin_fine = nullptr;
-    sub.offset = o_off; sub.snr = o_snr; sub.cov = o_cov; sub.maxval = o_val;
-    sub.maxloc = o_i; sub.start = o_i + 2 * m; sub.shift = o_i + 4 * m; sub.zoom_idx = o_i + 6 * m;
     sub.chunk = 0;
     sub.fine_start = sub.fine_shift = nullptr;
-    double *o_ref = a.refined ? buf<double>("p_refined", size_t(2) * m) : nullptr;
-    sub.refined = o_ref;
+    // offsets and zoom peaks of every re-run window go back to its place; the rest of the full ones only
+    sub.scatter = d_idx;
+    sub.full = m_full;
     if (m_full < m) {
         sub.fine_start = st4 + 4 * m;
         sub.fine_shift = st4 + 6 * m;
         sub.fine_from = m_full;
     }
     run_staged_t<double>(sub);
-    // offsets and zoom peaks of every re-run window; the rest of the full ones only
-    auto put_f = [&](const float *src, float *dst, int cnt, int width) {
-        if (dst && cnt) hipLaunchKernelGGL(k_put<float>, dim3(idivup(cnt * width, 256)), dim3(256), 0, a.stream, src, d_idx, dst, cnt, width);
-    };
-    auto put_i = [&](const int32_t *src, int32_t *dst, int cnt) {
-        if (dst && cnt) hipLaunchKernelGGL(k_put<int32_t>, dim3(idivup(cnt * 2, 256)), dim3(256), 0, a.stream, src, d_idx, dst, cnt, 2);
-    };
-    put_f(o_off, a.offset, m, 2);
-    if (o_ref)
-        hipLaunchKernelGGL(k_put<double>, dim3(idivup(m * 2, 256)), dim3(256), 0, a.stream, o_ref, d_idx, a.refined, m, 2);
-    put_i(sub.zoom_idx, a.zoom_idx, m);
-    put_f(o_snr, a.snr, m_full, 1);
-    put_f(o_cov, a.cov, m_full, 3);
-    put_f(o_val, a.maxval, m_full, 1);
-    put_i(sub.maxloc, a.maxloc, m_full);
-    put_i(sub.start, a.start, m_full);
-    put_i(sub.shift, a.shift, m_full);
-    HIP_OK(hipGetLastError());
 }
 
 void Engine::run(const RunArgs &in) {

@@ -79,41 +79,6 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 // ---------------------------------------------------------------------------
 constexpr int NORM_BLOCKS = 4;
 
-// DPP move of an FP64 value (both halves); lanes the row mask leaves out keep 0
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ double dpp_f64(double x) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, ROWMASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, ROWMASK, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-// DPP row shift of an FP64 value with every lane written: lanes whose source
-// lies before the start of their row read 0 (bound_ctrl), so no zeroed
-// destination is needed
-template <int CTRL>
-__device__ __forceinline__ double dpp_shr_f64(double x) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-
-// inclusive wave64 prefix sum: row_shr 1, 2, 4, 8 within rows of 16 lanes, then
-// row_bcast:15 into rows 1 and 3 and row_bcast:31 into rows 2 and 3
-__device__ __forceinline__ double wave_scan_f64(double x) {
-    x += dpp_shr_f64<0x111>(x);
-    x += dpp_shr_f64<0x112>(x);
-    x += dpp_shr_f64<0x114>(x);
-    x += dpp_shr_f64<0x118>(x);
-    x += dpp_f64<0x142, 0xa>(x);
-    x += dpp_f64<0x143, 0xc>(x);
-    return x;
-}
-
-__device__ __forceinline__ double lane63_f64(double x) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
-                            __builtin_amdgcn_readlane(__double2loint(x), 63));
-}
-
 // Lag-row phase of window_norms: part holds, for NB row blocks, the column sums
 // of s ([b][SW]) then of s^2 ([NB + b][SW]). With blk = 0 the blocks cover rows
 // [0, TH) and every wave slides its window down from row 0; with blk > 0 they

@@ -3,6 +3,7 @@
 // function whose arithmetic it performs (paths under contrib/PyCuAmpcor/src/).
 #pragma once
 #include <cfloat>
+#include <type_traits>
 #include "cx.h"
 #include "fft_inplace.h"
 #include "fft_lds.h"
@@ -144,30 +145,58 @@ __global__ void __launch_bounds__(512) k_fft_cols_quad(const cx<T> *data, int w,
 }
 
 // ---------------------------------------------------------------------------
-// chip gather (cuArraysCopy.cu:70-165): mode 0 complex copy, 1 (|z|,0), 2 real -> (x,0);
-// with `amp`, also the amplitude of the gathered chip (cuArraysAbs, cuArraysCopy.cu:510-529)
+// chips read straight from the images: window w's chip starts at row d[w], column
+// a[w] (plus the zoom chip's origin start[w] when given); mode as k_gather's
 // ---------------------------------------------------------------------------
+struct ChipSrc {
+    const void *img;
+    int64_t pitch;
+    const int32_t *d, *a, *start;
+    int mode;
+};
+
+// image offset of the chip's first pixel
+__device__ __forceinline__ int64_t chip_origin(const ChipSrc &s, int w) {
+    int64_t r = s.d[w], c = s.a[w];
+    if (s.start) { r += s.start[2 * w]; c += s.start[2 * w + 1]; }
+    return r * s.pitch + c;
+}
+
+// A chip's pixel in two steps, so that the loads of several pixels can be in flight
+// before the first is converted: the raw value at image offset `off` (REAL: (x, 0)),
+// and the pixel as the pipeline's chips hold it. with_kind(src, f) calls f with
+// std::true_type for real images, so that the choice is made once and not per load.
+template <bool REAL>
+__device__ __forceinline__ float2 chip_raw(const ChipSrc &s, int64_t off) {
+    if constexpr (REAL) return {static_cast<const float *>(s.img)[off], 0.f};
+    else return static_cast<const float2 *>(s.img)[off];
+}
 template <class T>
-__global__ void k_gather(const void *img, int64_t pitch, const int32_t *sd, const int32_t *sa,
-                         int h, int w, int mode, cx<T> *out, T *amp) {
+__device__ __forceinline__ cx<T> chip_value(const ChipSrc &s, float2 z) {
+    if (s.mode == 1) return {T(fast_abs(z.x, z.y)), T(0)};
+    return {T(z.x), T(z.y)};
+}
+template <class F>
+__device__ __forceinline__ void with_kind(const ChipSrc &s, F f) {
+    if (s.mode == 2) f(std::true_type{});
+    else f(std::false_type{});
+}
+
+template <class T>
+__global__ void k_gather(ChipSrc src, int h, int w, cx<T> *out, T *amp) {
     const int win = blockIdx.y;
     const int tot = h * w;
-    const int64_t r0 = sd[win], c0 = sa[win];
+    const int64_t o0 = chip_origin(src, win);
     cx<T> *o = out + size_t(win) * tot;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
-        const int r = i / w, c = i - r * w;
-        const int64_t off = (r0 + r) * pitch + c0 + c;
-        cx<T> v;
-        if (mode == 2) {
-            v = {T(static_cast<const float *>(img)[off]), T(0)};
-        } else {
-            const float2 z = static_cast<const float2 *>(img)[off];
-            v = {T(z.x), T(z.y)};
-            if (mode == 1) v = {T(fast_sqrt(z.x * z.x + z.y * z.y)), T(0)};
+    with_kind(src, [&](auto real) {
+        #pragma unroll 2
+        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
+            const int r = i / w, c = i - r * w;
+            const cx<T> v = chip_value<T>(src, chip_raw<decltype(real)::value>(src, o0 + r * src.pitch + c));
+            o[i] = v;
+            if (amp) amp[size_t(win) * tot + i] = amag(v);
         }
-        o[i] = v;
-        if (amp) amp[size_t(win) * tot + i] = amag(v);
-    }
+    });
 }
 
 // No-sync bounds check: copy the start arrays ([4][n] out), replacing every
@@ -236,6 +265,81 @@ __global__ void __launch_bounds__(1024) k_sub_mean(T *data, int size, double *ss
     }
 }
 
+// f(r, c) for the pixels of an h x w chip that fall to this thread of the block, U at a
+// time so that their loads are in flight together; past the last pixel f gets ok = false
+// (and the last pixel again)
+template <int U, class F>
+__device__ __forceinline__ void chip_pixels(int h, int w, F f) {
+    const int n = h * w, nt = blockDim.x, dr = nt / w, dc = nt - dr * w;
+    int r = threadIdx.x / w, c = threadIdx.x - r * w;
+    for (int i = threadIdx.x; i < n; i += U * nt) {
+        int rr[U], cc[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            ok[u] = r < h;
+            rr[u] = ok[u] ? r : h - 1;
+            cc[u] = ok[u] ? c : w - 1;
+            r += dr;
+            c += dc;
+            if (c >= w) { c -= w; ++r; }
+        }
+        f(rr, cc, ok);
+    }
+}
+
+// FP64 mean and sum of squared deviations of [nimg][size] images, which are left as
+// they are (their consumer subtracts the mean as it loads them); one block per image
+template <class T>
+__global__ void __launch_bounds__(1024) k_array_mean(const T *data, int size, double *mean, double *ssd) {
+    __shared__ double sh[16];
+    const T *img = data + size_t(blockIdx.x) * size;
+    double s1 = 0.0, s2 = 0.0;
+    #pragma unroll 8
+    for (int i = threadIdx.x; i < size; i += blockDim.x) {
+        const double v = double(img[i]);
+        s1 += v;
+        s2 += v * v;
+    }
+    s1 = block_sum256(s1, sh);
+    s2 = block_sum256(s2, sh);
+    if (threadIdx.x == 0) {
+        mean[blockIdx.x] = s1 / size;
+        ssd[blockIdx.x] = fmax(s2 - s1 * s1 / size, 0.0);
+    }
+}
+
+// FP64 sums of chips' amplitudes and of their squares, read from the image, over
+// gridDim.y row ranges of each chip: part[(w * ranges + range) * 2 + (0, 1)] (k_mean_parts)
+template <class T>
+__global__ void __launch_bounds__(256) k_chip_sums(ChipSrc src, int h, int w, double *part) {
+    __shared__ double sh[16];
+    const int per = (h + gridDim.y - 1) / gridDim.y, r0 = blockIdx.y * per, rows = max(0, min(h, r0 + per) - r0);
+    const int64_t o0 = chip_origin(src, blockIdx.x) + r0 * src.pitch;
+    double s1 = 0.0, s2 = 0.0;
+    constexpr int U = 8;
+    with_kind(src, [&](auto real) {
+        chip_pixels<U>(rows, w, [&](const int (&r)[U], const int (&c)[U], const bool (&ok)[U]) {
+            float2 z[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) z[u] = chip_raw<decltype(real)::value>(src, o0 + r[u] * src.pitch + c[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const double v = ok[u] ? double(amag(chip_value<T>(src, z[u]))) : 0.0;
+                s1 += v;
+                s2 += v * v;
+            }
+        });
+    });
+    s1 = block_sum256(s1, sh);
+    s2 = block_sum256(s2, sh);
+    if (threadIdx.x == 0) {
+        double *o = part + (size_t(blockIdx.x) * gridDim.y + blockIdx.y) * 2;
+        o[0] = s1;
+        o[1] = s2;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // correlation via one complex 2D FFT of z = t_pad + i*s (cuCorrFrequency.cu:63-111)
 // ---------------------------------------------------------------------------
@@ -286,83 +390,118 @@ __global__ void k_spec_product(cx<T> *z, int Lh, int Lw, T scale) {
 // and only the NL lag rows go back through a row IFFT (k_lagrows_real).
 // ---------------------------------------------------------------------------
 
-// Half spectra of the rows of [nimg][h][w] real images ([nimg][h][L/2+1]):
-// rows 2j and 2j+1 are loaded as one complex row z = r_2j + i r_2j+1 of length
-// L = d.n (zero beyond w and h), transformed in LDS, and split with
-// A = (Z[k] + conj Z[-k]) / 2, B = (Z[k] - conj Z[-k]) / (2i). `g` row pairs per block.
+// Half spectra of the rows of real images ([nimg][h][L/2+1]): rows 2j and 2j+1 are
+// loaded as one complex row z = r_2j + i r_2j+1 of length L (zero beyond w and h),
+// transformed in LDS, and split with A = (Z[k] + conj Z[-k]) / 2, B = (Z[k] -
+// conj Z[-k]) / (2i). One launch does the template rows and the search rows: a RowJob
+// each, the first `blocks` workgroups the first. The rows come from an array
+// ([nimg][h][w]) or are the amplitudes of chips read in place (img null), which also go
+// to `amp` when given; `mean`: per-image mean subtracted on load when given.
 template <class T>
-__global__ void __launch_bounds__(256) k_rowspec(const T *img, int nimg, int h, int w, int g, FftDesc d,
-                                                 cx<T> *spec) {
-    extern __shared__ unsigned char smem_raw[];
-    cx<T> *a = reinterpret_cast<cx<T> *>(smem_raw);
-    cx<T> *b = a + g * d.n;
-    const int L = d.n, np = (h + 1) / 2, H1 = L / 2 + 1;
-    const int t0 = blockIdx.x * g;
-    const int nr = min(g, nimg * np - t0);
-    for (int i = threadIdx.x; i < nr * L; i += blockDim.x) {
-        const int k = i / L, x = i - k * L;
-        const int t = t0 + k, win = t / np, r = 2 * (t - win * np);
-        const T *im = img + size_t(win) * h * w;
-        a[i] = {x < w ? im[r * w + x] : T(0), (x < w && r + 1 < h) ? im[(r + 1) * w + x] : T(0)};
+struct RowJob {
+    const T *img;
+    ChipSrc chip;
+    int h, w;
+    const double *mean;
+    cx<T> *spec;
+    T *amp;
+    int blocks;
+};
+
+// row pairs [t0, t0 + nr) of the job into z(k, x); org and mu hold a value per pair in LDS
+template <class T, class Z>
+__device__ __forceinline__ void load_row_pairs(const RowJob<T> &j, int t0, int nr, int L, int64_t *org, T *mu, Z z) {
+    const int np = (j.h + 1) / 2;
+    if (threadIdx.x < nr) {
+        const int t = t0 + threadIdx.x, win = t / np, r = 2 * (t - win * np);
+        org[threadIdx.x] = j.img ? (int64_t(win) * j.h + r) * j.w : chip_origin(j.chip, win) + r * j.chip.pitch;
+        mu[threadIdx.x] = j.mean ? T(j.mean[win]) : T(0);
     }
     __syncthreads();
-    const cx<T> *Z = fft_lds<T, -1>(a, b, d, nr, 1, L);
+    auto rows = [&](auto pixels) {
+        #pragma unroll 4
+        for (int i = threadIdx.x; i < nr * L; i += blockDim.x) {
+            const int k = i / L, x = i - k * L;
+            const int t = t0 + k, win = t / np, r = 2 * (t - win * np);
+            const bool in = x < j.w, two = in && r + 1 < j.h;
+            cx<T> v = {T(0), T(0)};
+            if (in) v = pixels(k, x, win, r, two);
+            if (in) v.x -= mu[k];
+            if (two) v.y -= mu[k];
+            z(k, x, v);
+        }
+    };
+    if (j.img)
+        rows([&](int k, int x, int, int, bool two) {
+            const T *p = j.img + org[k] + x;
+            return cx<T>{p[0], two ? p[j.w] : T(0)};
+        });
+    else
+        with_kind(j.chip, [&](auto real) {
+            rows([&](int k, int x, int win, int r, bool two) {
+                constexpr bool R = decltype(real)::value;
+                const float2 a = chip_raw<R>(j.chip, org[k] + x);
+                const float2 b = two ? chip_raw<R>(j.chip, org[k] + j.chip.pitch + x) : float2{0.f, 0.f};
+                const cx<T> v = {amag(chip_value<T>(j.chip, a)), amag(chip_value<T>(j.chip, b))};
+                if (j.amp) {
+                    T *o = j.amp + (size_t(win) * j.h + r) * j.w + x;
+                    o[0] = v.x;
+                    if (two) o[j.w] = v.y;
+                }
+                return v;
+            });
+        });
+    __syncthreads();
+}
+
+// the split half spectra of pairs [t0, t0 + nr) to memory; z(k, bin) reads the transform
+template <class T, class Z>
+__device__ __forceinline__ void store_row_spectra(const RowJob<T> &j, int t0, int nr, int L, Z z) {
+    const int np = (j.h + 1) / 2, H1 = L / 2 + 1;
     for (int i = threadIdx.x; i < nr * H1; i += blockDim.x) {
         const int k = i / H1, kk = i - k * H1;
-        const int t = t0 + k, win = t / np, j = t - win * np;
-        const cx<T> za = Z[k * L + kk], bc = conj(Z[k * L + (kk ? L - kk : 0)]);
-        cx<T> *sp = spec + size_t(win) * h * H1;
-        sp[size_t(2 * j) * H1 + kk] = (za + bc) * T(0.5);
-        if (2 * j + 1 < h) {
+        const int t = t0 + k, win = t / np, p = t - win * np;
+        const cx<T> za = z(k, kk), bc = conj(z(k, kk ? L - kk : 0));
+        cx<T> *sp = j.spec + (size_t(win) * j.h + 2 * p) * H1 + kk;
+        sp[0] = (za + bc) * T(0.5);
+        if (2 * p + 1 < j.h) {
             const cx<T> dd = (za - bc) * T(0.5);
-            sp[size_t(2 * j + 1) * H1 + kk] = {dd.y, -dd.x};
+            sp[H1] = {dd.y, -dd.x};
         }
     }
 }
 
-// The same half spectra with the row transform in place (fft_nat2dr, length
-// L = R1 * R2, read back from digit-reversed order), G row pairs per block of
-// odd LDS pitch
-template <class T, int R1, int R2, int G, int NTH = 256>
-__global__ void __launch_bounds__(NTH) k_rowspec_f(const T *img, int nimg, int h, int w, const cx<T> *tw,
-                                                   const double *mean, cx<T> *spec) {
-    constexpr int L = R1 * R2, PR = L + 1, H1 = L / 2 + 1;
+// general lengths (Stockham), `g` row pairs per block; LDS: 2 g L cx<T>, then g of (int64, T)
+template <class T>
+__global__ void __launch_bounds__(256) k_rowspec(RowJob<T> a, RowJob<T> b, int nimg, int g, FftDesc d) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    cx<T> *C = reinterpret_cast<cx<T> *>(smem_raw);   // [G][PR]
-    __shared__ T rowmu[G];                             // the pair's image mean, subtracted on load when given
+    cx<T> *p = reinterpret_cast<cx<T> *>(smem_raw), *q = p + g * d.n;
+    int64_t *org = reinterpret_cast<int64_t *>(q + g * d.n);
+    T *mu = reinterpret_cast<T *>(org + g);
+    const bool first = int(blockIdx.x) < a.blocks;
+    const RowJob<T> &j = first ? a : b;
+    const int t0 = (blockIdx.x - (first ? 0 : a.blocks)) * g, nr = min(g, nimg * ((j.h + 1) / 2) - t0);
+    load_row_pairs(j, t0, nr, d.n, org, mu, [&](int k, int x, cx<T> v) { p[k * d.n + x] = v; });
+    const cx<T> *Z = fft_lds<T, -1>(p, q, d, nr, 1, d.n);
+    store_row_spectra(j, t0, nr, d.n, [&](int k, int bin) { return Z[k * d.n + bin]; });
+}
+
+// in-place transforms (fft_nat2dr, length L = R1 * R2, read back from digit-reversed
+// order), G row pairs per block of odd LDS pitch
+template <class T, int R1, int R2, int G, int NTH = 256>
+__global__ void __launch_bounds__(NTH) k_rowspec_f(RowJob<T> a, RowJob<T> b, int nimg, const cx<T> *tw) {
+    constexpr int L = R1 * R2, PR = L + 1;
+    __shared__ cx<T> C[G * PR];
+    __shared__ int64_t org[G];
+    __shared__ T mu[G];
     __shared__ cx<T> twl[L];                           // twiddles, read from LDS
     for (int i = threadIdx.x; i < L; i += NTH) twl[i] = tw[i];
-    const int np = (h + 1) / 2;
-    const int t0 = blockIdx.x * G;
-    const int nr = min(G, nimg * np - t0);
-    if (mean) {
-        if (threadIdx.x < nr) rowmu[threadIdx.x] = T(mean[(t0 + threadIdx.x) / np]);
-        __syncthreads();
-    }
-    for (int i = threadIdx.x; i < nr * L; i += NTH) {
-        const int k = i / L, x = i - k * L;
-        const int t = t0 + k, win = t / np, r = 2 * (t - win * np);
-        const T *im = img + size_t(win) * h * w;
-        cx<T> v = {x < w ? im[r * w + x] : T(0), (x < w && r + 1 < h) ? im[(r + 1) * w + x] : T(0)};
-        if (mean) {
-            const T mu = rowmu[k];
-            v = {x < w ? v.x - mu : T(0), (x < w && r + 1 < h) ? v.y - mu : T(0)};
-        }
-        C[k * PR + x] = v;
-    }
-    __syncthreads();
+    const bool first = int(blockIdx.x) < a.blocks;
+    const RowJob<T> &j = first ? a : b;
+    const int t0 = (blockIdx.x - (first ? 0 : a.blocks)) * G, nr = min(G, nimg * ((j.h + 1) / 2) - t0);
+    load_row_pairs(j, t0, nr, L, org, mu, [&](int k, int x, cx<T> v) { C[k * PR + x] = v; });
     fft_nat2dr<T, -1, R1, R2, NTH>(C, nr, PR, 1, twl);
-    for (int i = threadIdx.x; i < nr * H1; i += NTH) {
-        const int k = i / H1, kk = i - k * H1;
-        const int t = t0 + k, win = t / np, j = t - win * np;
-        const cx<T> za = C[k * PR + dr_pos<R1, R2>(kk)], bc = conj(C[k * PR + dr_pos<R1, R2>(kk ? L - kk : 0)]);
-        cx<T> *sp = spec + size_t(win) * h * H1;
-        sp[size_t(2 * j) * H1 + kk] = (za + bc) * T(0.5);
-        if (2 * j + 1 < h) {
-            const cx<T> dd = (za - bc) * T(0.5);
-            sp[size_t(2 * j + 1) * H1 + kk] = {dd.y, -dd.x};
-        }
-    }
+    store_row_spectra(j, t0, nr, L, [&](int k, int bin) { return C[k * PR + dr_pos<R1, R2>(bin)]; });
 }
 
 // the inverse row FFT of the lag rows and k_crop_real in one pass: rows t of
@@ -444,6 +583,209 @@ __global__ void __launch_bounds__(64 * NQ) k_mac_lags(const cx<T> *tspec, int th
     }
 }
 
+// ---------------------------------------------------------------------------
+// Window sums for the normalization (formula of cuCorrNormalization.cu:230-314 and
+// cuCorrNormalizationSAT.cu:237-240), FP64, by lag rows: the sums of s and s^2 over SUM_BLK
+// rows of every search column (k_block_sums) give a lag row's column sums from th / SUM_BLK
+// blocks and a few rows at the ends; the next lag rows slide down from it; a wave prefix
+// scan over the columns then leaves every horizontal window sum as a difference.
+// ---------------------------------------------------------------------------
+constexpr int SUM_BLK = 16;
+
+// sums[w][b][0 and 1][c]: s and s^2 over rows [SUM_BLK b, SUM_BLK (b + 1)) of column c of
+// [n][sh][sw] images; a wave per 64 columns and row block (task), 4 tasks a workgroup
+__host__ __device__ inline int block_sum_tasks(int sh, int sw) { return ((sh + SUM_BLK - 1) / SUM_BLK) * ((sw + 63) / 64); }
+
+template <class T>
+__device__ __forceinline__ void block_sums_task(const T *img, int sh, int sw, int task, int win, double *sums) {
+    const int cols = (sw + 63) / 64, b = task / cols, c = 64 * (task - b * cols) + (threadIdx.x & 63);
+    if (task >= block_sum_tasks(sh, sw) || c >= sw) return;
+    const int nblk = (sh + SUM_BLK - 1) / SUM_BLK, r0 = b * SUM_BLK;
+    const T *p = img + (size_t(win) * sh + r0) * sw + c;
+    T v[SUM_BLK];
+#pragma unroll
+    for (int r = 0; r < SUM_BLK; ++r) v[r] = r0 + r < sh ? p[size_t(r) * sw] : T(0);
+    double a = 0.0, q = 0.0;
+#pragma unroll
+    for (int r = 0; r < SUM_BLK; ++r) {
+        a += double(v[r]);
+        q += double(v[r]) * double(v[r]);
+    }
+    double *o = sums + ((size_t(win) * nblk + b) * 2) * sw + c;
+    o[0] = a;
+    o[sw] = q;
+}
+
+template <class T>
+__global__ void __launch_bounds__(256) k_block_sums(const T *img, int sh, int sw, double *sums) {
+    block_sums_task(img, sh, sw, blockIdx.x * 4 + (threadIdx.x >> 6), blockIdx.y, sums);
+}
+
+// prefix sums over the columns of the window sums of lag rows [u0, u0 + kl): V[2 j] of s,
+// V[2 j + 1] of s^2 (rows of sw doubles in LDS); every thread of the NTH calls it
+template <int NTH, class T>
+__device__ __forceinline__ void lag_row_prefixes(const T *im, const double *sums, int sh, int sw, int th, int u0, int kl,
+                                                 double *V) {
+    const int lo = min((u0 + SUM_BLK - 1) / SUM_BLK, (u0 + th) / SUM_BLK), hi = (u0 + th) / SUM_BLK;
+    for (int c = threadIdx.x; c < sw; c += NTH) {
+        double a = 0.0, b = 0.0;
+        auto row = [&](int r, double sign) {
+            const double v = double(im[size_t(r) * sw + c]);
+            a = fma(sign, v, a);
+            b = fma(sign * v, v, b);
+        };
+        #pragma unroll 4
+        for (int k = lo; k < hi; ++k) {
+            a += sums[size_t(2 * k) * sw + c];
+            b += sums[size_t(2 * k + 1) * sw + c];
+        }
+        #pragma unroll 4
+        for (int r = u0; r < min(lo * SUM_BLK, u0 + th); ++r) row(r, 1.0);
+        #pragma unroll 4
+        for (int r = max(hi * SUM_BLK, u0); r < u0 + th; ++r) row(r, 1.0);
+        for (int j = 0; j < kl; ++j) {
+            V[size_t(2 * j) * sw + c] = a;
+            V[size_t(2 * j + 1) * sw + c] = b;
+            if (j + 1 < kl) {
+                row(u0 + j + th, 1.0);
+                row(u0 + j, -1.0);
+            }
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    for (int i = threadIdx.x >> 6; i < 2 * kl; i += NTH / 64) {
+        double *v = V + size_t(i) * sw, carry = 0.0;
+        for (int c0 = 0; c0 < sw; c0 += 64) {
+            const double x = wave_scan_f64(c0 + lane < sw ? v[c0 + lane] : 0.0) + carry;
+            if (c0 + lane < sw) v[c0 + lane] = x;
+            carry = lane63_f64(x);
+        }
+    }
+    __syncthreads();
+}
+
+// 1 / the correlation's norm squared is norm2 + FLT_EPSILON at lag (row j of V, v)
+__device__ __forceinline__ double lag_norm2(const double *V, int j, int sw, int v, int tw, double inv, double t2) {
+    const double *p1 = V + size_t(2 * j) * sw, *p2 = p1 + sw;
+    const double s1 = p1[v + tw - 1] - (v ? p1[v - 1] : 0.0), s2 = p2[v + tw - 1] - (v ? p2[v - 1] : 0.0);
+    return (s2 - s1 * s1 * inv) * t2;
+}
+
+// corr[w][u][v] /= norm for K lag rows of one window per workgroup; LDS: 2 K sw doubles.
+// (841 windows of 128, half search 32, both correlations: 316 us with column sums of every
+// lag row through HBM, 252 us with the block sums' pass.)
+template <class T>
+__global__ void __launch_bounds__(256) k_norm_lags(T *corr, int nl, int nlw, int th, int tw, const T *sr, int sh, int sw,
+                                                   const double *sums, const double *ssd, int K) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    double *V = reinterpret_cast<double *>(smem_raw);
+    const int win = blockIdx.y, u0 = blockIdx.x * K, kl = min(K, nl - u0), nblk = (sh + SUM_BLK - 1) / SUM_BLK;
+    lag_row_prefixes<256>(sr + size_t(win) * sh * sw, sums + size_t(win) * nblk * 2 * sw, sh, sw, th, u0, kl, V);
+    const double t2 = ssd[win], inv = 1.0 / (double(th) * tw);
+    T *c = corr + (size_t(win) * nl + u0) * nlw;
+    for (int o = threadIdx.x; o < kl * nlw; o += 256) {
+        const int j = o / nlw, v = o - j * nlw;
+        c[o] = T(double(c[o]) / sqrt(lag_norm2(V, j, sw, v, tw, inv, t2) + double(FLT_EPSILON)));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Normalized correlation of few windows (the FP64 pipeline: re-runs of near ties, and
+// precision 2), from the row half spectra in two launches instead of four (k_mac_lags,
+// k_lagrows_real and the normalization). With few windows those are bound by latency (a
+// thread walks a quarter of the search rows, or a whole column), so here
+//   k_lag_parts: partial lag sums over template rows [t0, t0 + per): a wave per 64 bins,
+//     K lag rows and row part, a sliding window of K search rows in registers; and, in the
+//     same launch, the block sums of the search amplitudes;
+//   k_corr_lags: one lag row per workgroup (K when there are many windows) sums the parts,
+//     evaluates c[v] = (1/L) sum_k Q[k] e^{2 pi i k v / L} at the wanted lags only (8 threads
+//     a value) and divides by the norm.
+// Windows of 64, half search 20: both correlations of 64 windows 91 -> 62 us, the
+// oversampled one of a single window 40 -> 16 us.
+// ---------------------------------------------------------------------------
+// q[w][part][u][k] = sum over the part's template rows t of conj(T_t[k]) S_{t+u}[k]
+template <class T, int K>
+__global__ void __launch_bounds__(256) k_lag_parts(const cx<T> *tspec, int th, const cx<T> *sspec, int sh, int nl, int H1,
+                                                   int parts, cx<T> *q, int lag_blocks, const T *sr, int sw, double *sums) {
+    const int win = blockIdx.y, lane = threadIdx.x & 63;
+    if (int(blockIdx.x) >= lag_blocks) {
+        block_sums_task(sr, sh, sw, (blockIdx.x - lag_blocks) * 4 + (threadIdx.x >> 6), win, sums);
+        return;
+    }
+    const int bins = (H1 + 63) / 64, task = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int part = task % parts, g = task / parts, k = 64 * (g % bins) + lane, u0 = (g / bins) * K;
+    if (k >= H1 || u0 >= nl) return;
+    const int per = (th + parts - 1) / parts, t0 = part * per, t1 = min(th, t0 + per);
+    const cx<T> *ts = tspec + size_t(win) * th * H1 + k, *ss = sspec + (size_t(win) * sh + u0) * H1 + k;
+    const int last = sh - 1 - u0;               // search rows past the end meet only lags past nl
+    cx<T> acc[K], s[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) acc[j] = cx<T>{T(0), T(0)};
+#pragma unroll
+    for (int j = 0; j + 1 < K; ++j) s[j] = ss[size_t(min(t0 + j, last)) * H1];
+    #pragma unroll 4
+    for (int t = t0; t < t1; ++t) {
+        const cx<T> tv = ts[size_t(t) * H1];
+        s[K - 1] = ss[size_t(min(t + K - 1, last)) * H1];
+#pragma unroll
+        for (int j = 0; j < K; ++j) acc[j] = cmac_conj(acc[j], tv, s[j]);
+#pragma unroll
+        for (int j = 0; j + 1 < K; ++j) s[j] = s[j + 1];
+    }
+    cx<T> *o = q + ((size_t(win) * parts + part) * nl + u0) * H1 + k;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+        if (u0 + j < nl) o[size_t(j) * H1] = acc[j];
+}
+
+// bytes of LDS: Q [K][H1], V [K][2][sw], twiddles [L]
+template <class T>
+__host__ __device__ inline size_t corr_lags_lds(int K, int L, int sw) {
+    return (size_t(K) * (L / 2 + 1) + L) * sizeof(cx<T>) + size_t(2) * K * sw * sizeof(double);
+}
+
+template <class T>
+__global__ void __launch_bounds__(256) k_corr_lags(const cx<T> *q, int parts, int L, int nl, int nlw, int th, int tw,
+                                                   const T *sr, int sh, int sw, const double *sums, const double *ssd,
+                                                   const cx<T> *twid, T *out, int K) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int H1 = L / 2 + 1, win = blockIdx.y, u0 = blockIdx.x * K, kl = min(K, nl - u0);
+    const int nblk = (sh + SUM_BLK - 1) / SUM_BLK;
+    cx<T> *Q = reinterpret_cast<cx<T> *>(smem_raw), *twl = Q + size_t(K) * H1;
+    double *V = reinterpret_cast<double *>(twl + L);
+    for (int i = threadIdx.x; i < L; i += 256) twl[i] = twid[i];
+    const cx<T> *qw = q + (size_t(win) * parts * nl + u0) * H1;
+    for (int i = threadIdx.x; i < kl * H1; i += 256) {
+        cx<T> v = qw[i];
+        #pragma unroll 4
+        for (int p = 1; p < parts; ++p) v = v + qw[size_t(p) * nl * H1 + i];
+        Q[i] = v;
+    }
+    lag_row_prefixes<256>(sr + size_t(win) * sh * sw, sums + size_t(win) * nblk * 2 * sw, sh, sw, th, u0, kl, V);
+    const double t2 = ssd[win], inv = 1.0 / (double(th) * tw);
+    const int slice = threadIdx.x & 7, nyq = L % 2 ? -1 : L / 2;           // an even L's Nyquist bin counts once
+    for (int o = threadIdx.x >> 3; o < kl * nlw; o += 32) {
+        const int j = o / nlw, v = o - j * nlw;
+        const cx<T> *qj = Q + j * H1;
+        T acc = T(0);
+        int m = int((int64_t(slice) * v) % L);
+        const int step = int((int64_t(8) * v) % L);
+        for (int k = slice; k < H1; k += 8) {
+            const cx<T> w = twl[m];                                        // e^{-2 pi i k v / L}
+            const T re = fma(qj[k].x, w.x, qj[k].y * w.y);
+            acc += k == 0 || k == nyq ? re : T(2) * re;
+            m += step;
+            if (m >= L) m -= L;
+        }
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) acc += __shfl_xor(acc, d);
+        if (slice == 0)
+            out[(size_t(win) * nl + u0 + j) * nlw + v] =
+                T(double(acc) / double(L) / sqrt(lag_norm2(V, j, sw, v, tw, inv, t2) + double(FLT_EPSILON)));
+    }
+}
+
 // real part of the top-left oh x ow block
 template <class T>
 __global__ void k_crop_real(const cx<T> *z, int Lh, int Lw, T *out, int oh, int ow) {
@@ -461,7 +803,7 @@ __global__ void k_crop_real(const cx<T> *z, int Lh, int Lw, T *out, int oh, int 
 // per-column vertical sums over the template height, slid down one lag row at
 // a time, and horizontal window sums from a block prefix scan of them. One
 // 256-thread block per window; dynamic LDS 4*sw + 2 doubles. Used for search
-// chips wider than the two-pass path below handles.
+// chips wider than the lag-row form above handles (1024 columns).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void block_scan256(double &x1, double &x2, double *sh4) {
     // inclusive scan of (x1, x2) over the 256 threads; sh4 holds 8 doubles
@@ -538,94 +880,6 @@ __global__ void __launch_bounds__(256) k_normalize(T *corr, int ch, int cw, cons
 }
 
 // ---------------------------------------------------------------------------
-// normalization in two barrier-free passes (same formula and FP64 sums as
-// k_normalize): k_colsums slides the vertical window sums of s and s^2 down
-// every column (one thread per column) into V[w][u][c]; k_norm_rows takes one
-// lag row per wave, forms the horizontal window sums from a wave prefix scan of
-// V and scales the correlation row. ssd[w] is the template's sum of squared
-// deviations (k_sub_mean).
-// ---------------------------------------------------------------------------
-template <class T>
-__global__ void __launch_bounds__(64) k_colsums(const T *srch, int sh, int sw, int th, int nl, double *V1,
-                                                double *V2) {
-    const int w = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= sw) return;
-    const T *s = srch + size_t(w) * sh * sw + c;
-    double b1[4] = {0.0, 0.0, 0.0, 0.0}, b2[4] = {0.0, 0.0, 0.0, 0.0};
-    int r = 0;
-    for (; r + 4 <= th; r += 4) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const double v = double(s[size_t(r + k) * sw]);
-            b1[k] += v;
-            b2[k] += v * v;
-        }
-    }
-    for (; r < th; ++r) {
-        const double v = double(s[size_t(r) * sw]);
-        b1[0] += v;
-        b2[0] += v * v;
-    }
-    double a1 = (b1[0] + b1[1]) + (b1[2] + b1[3]), a2 = (b2[0] + b2[1]) + (b2[2] + b2[3]);
-    double *o1 = V1 + size_t(w) * nl * sw + c, *o2 = V2 + size_t(w) * nl * sw + c;
-    o1[0] = a1;
-    o2[0] = a2;
-    for (int u = 1; u < nl; ++u) {
-        const double vn = double(s[size_t(u + th - 1) * sw]), vo = double(s[size_t(u - 1) * sw]);
-        a1 += vn - vo;
-        a2 += vn * vn - vo * vo;
-        o1[size_t(u) * sw] = a1;
-        o2[size_t(u) * sw] = a2;
-    }
-}
-
-template <class T, int CPL>
-__global__ void __launch_bounds__(256) k_norm_rows(T *corr, int n, int ch, int cw, int th, int tw, const double *V1,
-                                                   const double *V2, int sw, const double *ssd) {
-    const int lane = threadIdx.x & 63;
-    const int g = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int w = g / ch, u = g - w * ch;
-    if (w >= n) return;
-    const double *v1 = V1 + (size_t(w) * ch + u) * sw, *v2 = V2 + (size_t(w) * ch + u) * sw;
-    // inclusive prefix over columns: p[m] at column lane + 64 m
-    double p1[CPL], p2[CPL];
-    double c1 = 0.0, c2 = 0.0;
-#pragma unroll
-    for (int m = 0; m < CPL; ++m) {
-        const int c = lane + 64 * m;
-        double x1 = c < sw ? v1[c] : 0.0, x2 = c < sw ? v2[c] : 0.0;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const double y1 = __shfl_up(x1, d), y2 = __shfl_up(x2, d);
-            if (lane >= d) { x1 += y1; x2 += y2; }
-        }
-        x1 += c1; x2 += c2;
-        p1[m] = x1; p2[m] = x2;
-        c1 = __shfl(x1, 63);
-        c2 = __shfl(x2, 63);
-    }
-    const double t2 = ssd[w], inv = 1.0 / double(th * tw);
-    T *cr = corr + (size_t(w) * ch + u) * cw;
-    for (int k = 0; k * 64 < cw; ++k) {
-        const int v = lane + 64 * k;
-        const int hi = min(v + tw - 1, sw - 1), lo = v - 1;
-        double ph1 = 0, ph2 = 0, pl1 = 0, pl2 = 0;
-#pragma unroll
-        for (int m = 0; m < CPL; ++m) {
-            const double a1 = __shfl(p1[m], hi & 63), a2 = __shfl(p2[m], hi & 63);
-            const double b1 = __shfl(p1[m], lo & 63), b2 = __shfl(p2[m], lo & 63);
-            if ((hi >> 6) == m) { ph1 = a1; ph2 = a2; }
-            if (lo >= 0 && (lo >> 6) == m) { pl1 = b1; pl2 = b2; }
-        }
-        if (v < cw) {
-            const double s1 = ph1 - pl1, s2 = ph2 - pl2;
-            const double norm2 = (s2 - s1 * s1 * inv) * t2;
-            cr[v] = T(double(cr[v]) / sqrt(norm2 + double(FLT_EPSILON)));
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // argmax with the reference tie rule (cuOffset.cu:23-84), one block per surface
 // ---------------------------------------------------------------------------
 template <class T>
@@ -658,6 +912,29 @@ __device__ __forceinline__ void adjust_axis(int maxloc, int old_range, int new_r
     else if (start > rbound) { shift = start - rbound; start = rbound; }
 }
 
+// covariance from the peak's curvature (cuEstimateStats.cu:49-110); g(dx, dy): the
+// normalized surface around the peak, read only when `inner` (the peak has neighbours)
+template <class G>
+__device__ __forceinline__ void peak_covariance(G g, bool inner, double peak, int template_size, float *cov3) {
+    double cxx = 99.0, cyy = 99.0, cxy = 0.0;
+    if (inner) {
+        double dxx = -(g(1, 0) + g(-1, 0) - 2.0 * g(0, 0)) * template_size;
+        double dyy = -(g(0, 1) + g(0, -1) - 2.0 * g(0, 0)) * template_size;
+        double dxy = (g(1, 1) + g(-1, -1) - g(1, -1) - g(-1, 1)) * 0.25 * template_size;
+        double n2 = fmax(1.0 - peak, 0.0);
+        const double n4 = n2 * n2 * 0.5 * template_size;
+        n2 *= 2.0;
+        const double u = dxy * dxy - dxx * dyy;
+        const double u2 = u * u;
+        if (fabs(u) >= 1e-2) {
+            cxx = (-n2 * u * dyy + n4 * (dyy * dyy + dxy * dxy)) / u2;
+            cyy = (-n2 * u * dxx + n4 * (dxx * dxx + dxy * dxy)) / u2;
+            cxy = (n2 * u * dxy - n4 * (dxx + dyy) * dxy) / u2;
+        }
+    }
+    cov3[0] = float(cxx); cov3[1] = float(cyy); cov3[2] = float(cxy);
+}
+
 // Covariance and SNR of one window's normalized surface, computed by one wave:
 // lanes share the SNR patch sum, lane 0 writes both results.
 template <class T>
@@ -682,40 +959,32 @@ __device__ void window_stats(const T *c, int nx, int ny, int px, int py, double 
         count += __shfl_xor(count, o);
     }
     if (lane != 0) return;
-    // covariance
-    double cxx = 99.0, cyy = 99.0, cxy = 0.0;
-    if (!(px - 1 < 0 || py - 1 < 0 || px + 1 >= nx || py + 1 >= ny)) {
-        auto g = [&](int dx, int dy) { return double(c[(px + dx) * ny + py + dy]); };
-        double dxx = -(g(1, 0) + g(-1, 0) - 2.0 * g(0, 0)) * template_size;
-        double dyy = -(g(0, 1) + g(0, -1) - 2.0 * g(0, 0)) * template_size;
-        double dxy = (g(1, 1) + g(-1, -1) - g(1, -1) - g(-1, 1)) * 0.25 * template_size;
-        double n2 = fmax(1.0 - peak, 0.0);
-        const double n4 = n2 * n2 * 0.5 * template_size;
-        n2 *= 2.0;
-        const double u = dxy * dxy - dxx * dyy;
-        const double u2 = u * u;
-        if (fabs(u) >= 1e-2) {
-            cxx = (-n2 * u * dyy + n4 * (dyy * dyy + dxy * dxy)) / u2;
-            cyy = (-n2 * u * dxx + n4 * (dxx * dxx + dxy * dxy)) / u2;
-            cxy = (n2 * u * dxy - n4 * (dxx + dyy) * dxy) / u2;
-        }
-    }
-    cov3[0] = float(cxx); cov3[1] = float(cyy); cov3[2] = float(cxy);
+    peak_covariance([&](int dx, int dy) { return double(c[(px + dx) * ny + py + dy]); },
+                    !(px - 1 < 0 || py - 1 < 0 || px + 1 >= nx || py + 1 >= ny), peak, template_size, cov3);
     const double mean = (sum - peak * peak) / double(count - 1);
     *snr = float(peak * peak / mean);
 }
 
-// one 64-thread block (one wave) per window
+// argmax (k_maxloc), then covariance, SNR and the zoom start/shift of one surface per
+// 256-thread block
 template <class T>
-__global__ void __launch_bounds__(64) k_stats(const T *corr, int nx, int ny, int n, const int32_t *loc, const T *val,
-                                              int template_size, int patch_h, int patch_w, int hs_down,
-                                              int hs_across, int hz, float *cov, float *snr, int32_t *start,
-                                              int32_t *shift) {
+__global__ void __launch_bounds__(256) k_peak(const T *corr, int nx, int ny, int template_size, int patch_h, int patch_w,
+                                              int hs_down, int hs_across, int hz, int32_t *loc, T *val, float *margin,
+                                              float *cov, float *snr, int32_t *start, int32_t *shift) {
+    __shared__ T shv[4], shv2[4];
+    __shared__ uint64_t shk[4];
     const int w = blockIdx.x;
-    const int px = loc[2 * w], py = loc[2 * w + 1];
-    window_stats(corr + size_t(w) * nx * ny, nx, ny, px, py, double(val[w]), template_size, patch_h, patch_w,
-                 cov + 3 * w, snr + w);
+    const T *s = corr + size_t(w) * nx * ny;
+    Top2<T> top;
+    for (int i = threadIdx.x; i < nx * ny; i += 256) top.add(s[i], maxloc_key(uint32_t(i)));
+    top.template reduce<256>(shv, shv2, shk);
+    if (threadIdx.x >= 64) return;
+    const int idx = top.index(), px = idx / ny, py = idx - px * ny;
+    window_stats(s, nx, ny, px, py, double(top.v1), template_size, patch_h, patch_w, cov + 3 * w, snr + w);
     if (threadIdx.x == 0) {
+        loc[2 * w] = px; loc[2 * w + 1] = py;
+        val[w] = top.v1;
+        if (margin) margin[w] = top.margin();
         int s0, h0, s1, h1;
         adjust_axis(px, hs_down, hz, s0, h0);
         adjust_axis(py, hs_across, hz, s1, h1);
@@ -738,38 +1007,63 @@ __device__ __forceinline__ const cx<T> *crop_origin(const cx<T> *src, int ih, in
     return start ? o + start[2 * win] * iw + start[2 * win + 1] : o;
 }
 
-template <class T>
-__global__ void __launch_bounds__(1024) k_deramp_phase(const cx<T> *src, int ih, int iw, const int32_t *start, int h,
-                                                       int w, cx<double> *tab) {
-    __shared__ double sh[16];
-    const cx<T> *z = crop_origin(src, ih, iw, start, blockIdx.x);
-    double ayr = 0, ayi = 0, axr = 0, axi = 0;
-    for (int i = threadIdx.x; i < h * w; i += blockDim.x) {
-        const int r = i / w, c = i - r * w;
-        const cx<T> v = z[r * iw + c];
-        const double zr = double(v.x), zi = double(v.y);
-        if (c < w - 1) {   // z * conj(z_right)
-            const cx<T> u = z[r * iw + c + 1];
-            const double br = double(u.x), bi = double(u.y);
-            ayr += zr * br + zi * bi;
-            ayi += zi * br - zr * bi;
-        }
-        if (r < h - 1) {   // z * conj(z_below)
-            const cx<T> u = z[(r + 1) * iw + c];
-            const double br = double(u.x), bi = double(u.y);
-            axr += zr * br + zi * bi;
-            axi += zi * br - zr * bi;
-        }
+// two kinds of chips in one launch: blockIdx.y picks the job
+struct PhaseJob {
+    ChipSrc chip;
+    int h, w;
+    cx<double> *tab;
+};
+
+static __global__ void __launch_bounds__(1024) k_deramp_phase(PhaseJob a, PhaseJob b) {
+    __shared__ double sh[4][16];
+    const PhaseJob &j = blockIdx.y ? b : a;
+    const int h = j.h, w = j.w, lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int64_t o0 = chip_origin(j.chip, blockIdx.x);
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    // pixels as stored: deramped chips are complex or real images (mode 1 is derampMethod 0)
+    constexpr int U = 4;
+    with_kind(j.chip, [&](auto real) {
+        constexpr bool R = decltype(real)::value;
+        chip_pixels<U>(h, w, [&](const int (&r)[U], const int (&c)[U], const bool (&ok)[U]) {
+            float2 z[U], x[U], y[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                // neighbours past the last column or row count as zero (the pixel itself is read instead)
+                const int64_t o = o0 + r[u] * j.chip.pitch + c[u];
+                z[u] = chip_raw<R>(j.chip, o);
+                x[u] = chip_raw<R>(j.chip, c[u] < w - 1 ? o + 1 : o);
+                y[u] = chip_raw<R>(j.chip, r[u] < h - 1 ? o + j.chip.pitch : o);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool right = ok[u] && c[u] < w - 1, below = ok[u] && r[u] < h - 1;
+                const double zr = z[u].x, zi = z[u].y;
+                const double xr = right ? x[u].x : 0.f, xi = right ? x[u].y : 0.f;
+                const double yr = below ? y[u].x : 0.f, yi = below ? y[u].y : 0.f;
+                t[0] += zr * xr + zi * xi;      // z * conj(z_right)
+                t[1] += zi * xr - zr * xi;
+                t[2] += zr * yr + zi * yi;      // z * conj(z_below)
+                t[3] += zi * yr - zr * yi;
+            }
+        });
+    });
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        t[k] = wave_scan_f64(t[k]);
+        if (lane == 63) sh[k][wv] = t[k];
     }
-    ayr = block_sum256(ayr, sh);
-    ayi = block_sum256(ayi, sh);
-    axr = block_sum256(axr, sh);
-    axi = block_sum256(axi, sh);
-    const double phy = atan2(ayi, ayr);
-    const double phx = atan2(axi, axr);
-    cx<double> *rowf = tab + size_t(blockIdx.x) * (h + w), *colf = rowf + h;
-    for (int r = threadIdx.x; r < h; r += blockDim.x) sincos(double(r) * phy, &rowf[r].y, &rowf[r].x);
-    for (int c = threadIdx.x; c < w; c += blockDim.x) sincos(double(c) * phx, &colf[c].y, &colf[c].x);
+    __syncthreads();
+    cx<double> *rowf = j.tab + size_t(blockIdx.x) * (h + w);
+    for (int i = threadIdx.x; i < h + w; i += blockDim.x) {
+        const bool row = i < h;
+        double re = 0.0, im = 0.0;
+        for (int k = 0; k < nw; ++k) {
+            re += sh[row ? 0 : 2][k];
+            im += sh[row ? 1 : 3][k];
+        }
+        const double phase = atan2(im, re);
+        sincos(double(row ? i : i - h) * phase, &rowf[i].y, &rowf[i].x);
+    }
 }
 
 template <class T>
@@ -832,10 +1126,12 @@ __device__ __forceinline__ cx<T> half_shift(int k, int n) {
     return {T(c / n), T(s / n)};
 }
 
-template <class T>
-__device__ __forceinline__ cx<T> chip_pixel(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                            const cx<double> *tab, int win, int h, int w, int r, int c) {
-    cx<T> v = crop_origin(src, ih, iw, start, win)[r * iw + c];
+// pixel (r, c) of window win's h x w chip, whose first pixel is at image offset `org`,
+// deramped with `tab` when given
+template <class T, bool REAL>
+__device__ __forceinline__ cx<T> chip_pixel(const ChipSrc &src, int64_t org, const cx<double> *tab, int win, int h, int w,
+                                            int r, int c) {
+    cx<T> v = chip_value<T>(src, chip_raw<REAL>(src, org + r * src.pitch + c));
     if (tab) {
         const cx<double> *rowf = tab + size_t(win) * (h + w);
         v = deramp_apply(v, rowf[r], rowf[h + c]);
@@ -846,18 +1142,22 @@ __device__ __forceinline__ cx<T> chip_pixel(const cx<T> *src, int ih, int iw, co
 // `cb` chip columns per block (blockIdx.x), one chip per blockIdx.y; d.n = h;
 // Y: [nimg][h][w]
 template <class T>
-__global__ void __launch_bounds__(256) k_os2_cols(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                                  const cx<double> *tab, int w, int cb, FftDesc d, cx<T> *Y) {
+__global__ void __launch_bounds__(256) k_os2_cols(ChipSrc src, const cx<double> *tab, int w, int cb, FftDesc d,
+                                                  cx<T> *Y) {
     extern __shared__ unsigned char smem_raw[];
     const int h = d.n;
     cx<T> *a = reinterpret_cast<cx<T> *>(smem_raw);
     cx<T> *b = a + cb * h;
     cx<T> *sh = b + cb * h;
     const int win = blockIdx.y, c0 = blockIdx.x * cb, nc = min(cb, w - c0);
-    for (int i = threadIdx.x; i < h * nc; i += blockDim.x) {
-        const int r = i / nc, c = i - r * nc;
-        a[r * cb + c] = chip_pixel(src, ih, iw, start, tab, win, h, w, r, c0 + c);
-    }
+    const int64_t org = chip_origin(src, win);
+    with_kind(src, [&](auto real) {
+        #pragma unroll 4
+        for (int i = threadIdx.x; i < h * nc; i += blockDim.x) {
+            const int r = i / nc, c = i - r * nc;
+            a[r * cb + c] = chip_pixel<T, decltype(real)::value>(src, org, tab, win, h, w, r, c0 + c);
+        }
+    });
     for (int k = threadIdx.x; k < h; k += blockDim.x) sh[k] = half_shift<T>(k, h);
     __syncthreads();
     cx<T> *X = fft_lds<T, +1>(a, b, d, nc, cb, 1);
@@ -876,10 +1176,13 @@ __global__ void __launch_bounds__(256) k_os2_cols(const cx<T> *src, int ih, int 
 }
 
 // `g` output rows per block over the nimg * 2h rows; d.n = w; out: [nimg][2h][2w]
-// real, |.| (OUT 1) of the oversampled chip
+// real, |.| (OUT 1) of the oversampled chip. LDS: os2_rows_lds
 template <class T>
-__global__ void __launch_bounds__(256) k_os2_rows(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                                  const cx<double> *tab, const cx<T> *Y, int nimg, int h, int g,
+__host__ __device__ inline size_t os2_rows_lds(int g, int w) {
+    return (2 * size_t(g) + 1) * w * sizeof(cx<T>) + size_t(g) * w * sizeof(T) + 8 + size_t(g) * sizeof(int64_t);
+}
+template <class T>
+__global__ void __launch_bounds__(256) k_os2_rows(ChipSrc src, const cx<double> *tab, const cx<T> *Y, int nimg, int h, int g,
                                                   FftDesc d, T *out) {
     extern __shared__ unsigned char smem_raw[];
     const int w = d.n;
@@ -887,15 +1190,21 @@ __global__ void __launch_bounds__(256) k_os2_rows(const cx<T> *src, int ih, int 
     cx<T> *b = a + g * w;
     cx<T> *sh = b + g * w;
     T *amp = reinterpret_cast<T *>(sh + w);
+    int64_t *org = reinterpret_cast<int64_t *>((reinterpret_cast<uintptr_t>(amp + size_t(g) * w) + 7) & ~uintptr_t(7));
     const int t0 = blockIdx.x * g;
     const int nr = min(g, nimg * 2 * h - t0);
-    for (int i = threadIdx.x; i < nr * w; i += blockDim.x) {
-        const int k = i / w, c = i - k * w;
-        const int t = t0 + k, win = t / (2 * h), tr = t - win * 2 * h, m = tr >> 1;
-        const cx<T> v = (tr & 1) ? Y[(size_t(win) * h + m) * w + c] : chip_pixel(src, ih, iw, start, tab, win, h, w, m, c);
-        a[i] = v;
-        amp[i] = amag(v);
-    }
+    for (int k = threadIdx.x; k < nr; k += blockDim.x) org[k] = chip_origin(src, (t0 + k) / (2 * h));
+    __syncthreads();
+    with_kind(src, [&](auto real) {
+        for (int i = threadIdx.x; i < nr * w; i += blockDim.x) {
+            const int k = i / w, c = i - k * w;
+            const int t = t0 + k, win = t / (2 * h), tr = t - win * 2 * h, m = tr >> 1;
+            const cx<T> v = (tr & 1) ? Y[(size_t(win) * h + m) * w + c]
+                                     : chip_pixel<T, decltype(real)::value>(src, org[k], tab, win, h, w, m, c);
+            a[i] = v;
+            amp[i] = amag(v);
+        }
+    });
     for (int k = threadIdx.x; k < w; k += blockDim.x) sh[k] = half_shift<T>(k, w);
     __syncthreads();
     cx<T> *X = fft_lds<T, +1>(a, b, d, nr, 1, w);
@@ -917,63 +1226,87 @@ __global__ void __launch_bounds__(256) k_os2_rows(const cx<T> *src, int ih, int 
 // (fft_half_sample: three LDS passes), one chip line per LDS row of odd pitch.
 // `tw`, `shift`: e^{-2 pi i k/N} and the half-sample shifts, copied into LDS.
 
-// CB chip columns per block (blockIdx.x), one chip per blockIdx.y; chip height
-// R1 * R2; Y: [nimg][R1 * R2][w]
-template <class T, int R1, int R2, int CB, int NTH = 256>
-__global__ void __launch_bounds__(NTH) k_os2_cols_f(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                                    const cx<double> *tab, int w, const cx<T> *tw, const cx<T> *shift,
-                                                    cx<T> *Y) {
+// One kind of chips: h x w pixels, Y [nimg][h][w] (odd rows), out [nimg][2h][2w]; twiddles
+// and shifts of the column (h) and the row (w) transforms. The first `blocks` workgroups (of a window in the column
+// pass, of the launch in the row pass) take the first job of a launch with two.
+template <class T>
+struct OsJob {
+    ChipSrc chip;
+    const cx<double> *tab;
+    int h, w;
+    const cx<T> *tw_h, *shift_h, *tw_w, *shift_w;
+    cx<T> *Y;
+    T *out;
+    double *part;
+    int blocks;
+};
+
+// CB chip columns of window win (block bx); chip height R1 * R2; LDS: os2_cols_lds
+template <class T>
+__host__ __device__ constexpr size_t os2_cols_lds(int N, int CB) { return (size_t(N) * (CB + 1) + 2 * N) * sizeof(cx<T>); }
+template <class T, int R1, int R2, int CB, int NTH>
+__device__ __forceinline__ void os2_cols_body(const OsJob<T> &j, int bx, int win, unsigned char *smem_raw) {
     constexpr int N = R1 * R2, PC = CB + 1;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *C = reinterpret_cast<cx<T> *>(smem_raw);   // [N][PC]: column c at C[c + r * PC]
-    __shared__ cx<T> twl[N], sh[N];
-    const int win = blockIdx.y, c0 = blockIdx.x * CB, nc = min(CB, w - c0);
-    for (int i = threadIdx.x; i < N * CB; i += NTH) {
-        const int r = i / CB, c = i - r * CB;
-        if (c < nc) C[r * PC + c] = chip_pixel(src, ih, iw, start, tab, win, N, w, r, c0 + c);
-    }
+    cx<T> *twl = C + N * PC, *sh = twl + N;
+    const int c0 = bx * CB, nc = min(CB, j.w - c0);
+    const int64_t org = chip_origin(j.chip, win);
+    with_kind(j.chip, [&](auto real) {
+        #pragma unroll 4
+        for (int i = threadIdx.x; i < N * CB; i += NTH) {
+            const int r = i / CB, c = i - r * CB;
+            if (c < nc) C[r * PC + c] = chip_pixel<T, decltype(real)::value>(j.chip, org, j.tab, win, N, j.w, r, c0 + c);
+        }
+    });
     for (int k = threadIdx.x; k < N; k += NTH) {
-        sh[k] = shift[k];
-        twl[k] = tw[k];
+        sh[k] = j.shift_h[k];
+        twl[k] = j.tw_h[k];
     }
     __syncthreads();
     // consecutive work items hold consecutive columns: the results go out as they are made
-    cx<T> *y = Y + size_t(win) * N * w + c0;
+    cx<T> *y = j.Y + size_t(win) * N * j.w + c0;
     fft_half_sample<T, R1, R2, NTH>(C, nc, 1, PC, twl, sh, [](int, int, cx<T>) {},
-                                    [&](int c, int r, cx<T> v) { y[size_t(r) * w + c] = v; });
+                                    [&](int c, int r, cx<T> v) { y[size_t(r) * j.w + c] = v; });
 }
 
-// G output rows per block over the nimg * 2h rows; chip width R1 * R2;
-// out: [nimg][2h][2 R1 R2] amplitudes. With `part` (G dividing 2h, so that a
-// block holds rows of one chip only), each block also writes the FP64 sums of
-// its amplitudes and of their squares to part[2 * block], part[2 * block + 1].
-template <class T, int R1, int R2, int G, int NTH = 256>
-__global__ void __launch_bounds__(NTH) k_os2_rows_f(const cx<T> *src, int ih, int iw, const int32_t *start,
-                                                    const cx<double> *tab, const cx<T> *Y, int nimg, int h,
-                                                    const cx<T> *tw, const cx<T> *shift, T *out, double *part) {
+// G output rows (block bx) over the nimg * 2h rows; chip width R1 * R2. With `part`
+// (G dividing 2h, so that a block holds rows of one chip only), the block also writes
+// the FP64 sums of its amplitudes and of their squares to part[2 bx], part[2 bx + 1].
+template <class T>
+__host__ __device__ constexpr size_t os2_rows_f_lds(int N, int G) {
+    return (size_t(G) * (N + 1) + 2 * N) * sizeof(cx<T>) + size_t(G) * N * sizeof(T);
+}
+template <class T, int R1, int R2, int G, int NTH>
+__device__ __forceinline__ void os2_rows_body(const OsJob<T> &j, int bx, int nimg, unsigned char *smem_raw, int64_t *org,
+                                              double *red) {
     constexpr int N = R1 * R2, PR = N + 1;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<T> *C = reinterpret_cast<cx<T> *>(smem_raw);   // [G][PR]
-    T *amp = reinterpret_cast<T *>(C + G * PR);        // [G][N]
-    __shared__ cx<T> twl[N], sh[N];
-    const int t0 = blockIdx.x * G;
+    cx<T> *twl = C + G * PR, *sh = twl + N;
+    T *amp = reinterpret_cast<T *>(sh + N);            // [G][N]
+    const int h = j.h, t0 = bx * G;
     const int nr = min(G, nimg * 2 * h - t0);
-    for (int i = threadIdx.x; i < nr * N; i += NTH) {
-        const int k = i / N, c = i - k * N;
-        const int t = t0 + k, win = t / (2 * h), tr = t - win * 2 * h, m = tr >> 1;
-        const cx<T> v = (tr & 1) ? Y[(size_t(win) * h + m) * N + c] : chip_pixel(src, ih, iw, start, tab, win, h, N, m, c);
-        C[k * PR + c] = v;
-        amp[i] = amag(v);
-    }
+    if (threadIdx.x < nr) org[threadIdx.x] = chip_origin(j.chip, (t0 + threadIdx.x) / (2 * h));
     for (int k = threadIdx.x; k < N; k += NTH) {
-        sh[k] = shift[k];
-        twl[k] = tw[k];
+        sh[k] = j.shift_w[k];
+        twl[k] = j.tw_w[k];
     }
+    __syncthreads();
+    with_kind(j.chip, [&](auto real) {
+        #pragma unroll 2
+        for (int i = threadIdx.x; i < nr * N; i += NTH) {
+            const int k = i / N, c = i - k * N;
+            const int t = t0 + k, win = t / (2 * h), tr = t - win * 2 * h, m = tr >> 1;
+            const cx<T> v = (tr & 1) ? j.Y[(size_t(win) * h + m) * N + c]
+                                     : chip_pixel<T, decltype(real)::value>(j.chip, org[k], j.tab, win, h, N, m, c);
+            C[k * PR + c] = v;
+            amp[i] = amag(v);
+        }
+    });
     __syncthreads();
     fft_half_sample<T, R1, R2, NTH>(C, nr, PR, 1, twl, sh, [](int, int, cx<T>) {},
                                     [&](int k, int c, cx<T> v) { C[k * PR + c] = v; });
     __syncthreads();
-    T *o = out + size_t(t0) * 2 * N;
+    T *o = j.out + size_t(t0) * 2 * N;
     double s1 = 0.0, s2 = 0.0;
     for (int i = threadIdx.x; i < nr * N; i += NTH) {
         const int k = i / N, c = i - k * N;
@@ -982,15 +1315,45 @@ __global__ void __launch_bounds__(NTH) k_os2_rows_f(const cx<T> *src, int ih, in
         s1 += double(a0) + double(a1);
         s2 += double(a0) * double(a0) + double(a1) * double(a1);
     }
-    if (part) {
-        __shared__ double red[16];
+    if (j.part) {
         s1 = block_sum256(s1, red);
         s2 = block_sum256(s2, red);
         if (threadIdx.x == 0) {
-            part[2 * blockIdx.x] = s1;
-            part[2 * blockIdx.x + 1] = s2;
+            j.part[2 * bx] = s1;
+            j.part[2 * bx + 1] = s2;
         }
     }
+}
+
+// one kind of chips per launch (many windows: each kind keeps its own registers and threads)
+template <class T, int R1, int R2, int CB, int NTH = 256>
+__global__ void __launch_bounds__(NTH) k_os2_cols_f(OsJob<T> j) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    os2_cols_body<T, R1, R2, CB, NTH>(j, blockIdx.x, blockIdx.y, smem_raw);
+}
+template <class T, int R1, int R2, int G, int NTH = 256>
+__global__ void __launch_bounds__(NTH) k_os2_rows_f(OsJob<T> j, int nimg) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ int64_t org[G];
+    __shared__ double red[16];
+    os2_rows_body<T, R1, R2, G, NTH>(j, blockIdx.x, nimg, smem_raw, org, red);
+}
+
+// reference and search chips in one launch (the FP64 pipeline's few windows, where a
+// launch more costs what a kernel does): sides A1 * A2 and B1 * B2
+template <class T, int A1, int A2, int B1, int B2, int CB>
+__global__ void __launch_bounds__(256) k_os2_cols_pair(OsJob<T> a, OsJob<T> b) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    if (int(blockIdx.x) < a.blocks) os2_cols_body<T, A1, A2, CB, 256>(a, blockIdx.x, blockIdx.y, smem_raw);
+    else os2_cols_body<T, B1, B2, CB, 256>(b, blockIdx.x - a.blocks, blockIdx.y, smem_raw);
+}
+template <class T, int A1, int A2, int B1, int B2, int G>
+__global__ void __launch_bounds__(256) k_os2_rows_pair(OsJob<T> a, OsJob<T> b, int nimg) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ int64_t org[G];
+    __shared__ double red[16];
+    if (int(blockIdx.x) < a.blocks) os2_rows_body<T, A1, A2, G, 256>(a, blockIdx.x, nimg, smem_raw, org, red);
+    else os2_rows_body<T, B1, B2, G, 256>(b, blockIdx.x - a.blocks, nimg, smem_raw, org, red);
 }
 
 // idx[0..cap) = the first cap windows (in order) whose margins are below the
@@ -1030,18 +1393,26 @@ static __global__ void __launch_bounds__(1024) k_select_near(const float *mc, co
 }
 
 // mean and sum of squared deviations of each [size] image from nb block sums
-// (k_os2_rows_f's `part`): the values k_sub_mean finds, for the consumer to
-// subtract the mean as it loads the image (k_rowspec_f's `mean`)
-static __global__ void k_mean_parts(const double *part, int nb, int size, int nimg, double *mean, double *ssd) {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
+// (os2_rows_body's `part`), for the consumer to subtract the mean as it loads the
+// image; one wave per image, four a block
+static __global__ void __launch_bounds__(256) k_mean_parts(const double *part, int nb, int size, int nimg, double *mean,
+                                                           double *ssd) {
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (w >= nimg) return;
     double s1 = 0.0, s2 = 0.0;
-    for (int j = 0; j < nb; ++j) {
+    for (int j = lane; j < nb; j += 64) {
         s1 += part[2 * (size_t(w) * nb + j)];
         s2 += part[2 * (size_t(w) * nb + j) + 1];
     }
-    mean[w] = s1 / size;
-    if (ssd) ssd[w] = fmax(s2 - s1 * s1 / size, 0.0);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        s1 += __shfl_xor(s1, o);
+        s2 += __shfl_xor(s2, o);
+    }
+    if (lane == 0) {
+        mean[w] = s1 / size;
+        ssd[w] = fmax(s2 - s1 * s1 / size, 0.0);
+    }
 }
 
 template <class T>
@@ -1261,7 +1632,14 @@ __global__ void __launch_bounds__(NTH) k_surface(const T *corr, int ch, int cw, 
 #pragma unroll
         for (int k1 = 0; k1 < 16; ++k1) {
             const cx<T> g = G[k1 * SO + threadIdx.x];
-            bq += ampcor::amag(g);
+            if constexpr (sizeof(T) == 8) {
+                // max + min / 2 is never below the modulus (and at most 12% above), and
+                // costs a tenth of an FP64 square root
+                const T x = fabs(g.x), y = fabs(g.y);
+                bq += fma(T(0.5), fmin(x, y), fmax(x, y));
+            } else {
+                bq += ampcor::amag(g);
+            }
         }
         keep = !(bq * T(1.0 + 0x1p-10) + T(0x1p-11) * amag < amax);
     }
