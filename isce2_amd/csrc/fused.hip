@@ -207,6 +207,110 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
 }
 
 // ---------------------------------------------------------------------------
+// Covariance of the coarse peak from the images: the normalized correlation at the peak
+// and its eight neighbours, as FP64 sums over the window (the formula divides second
+// differences of the surface, whose FP32 rounding it can magnify tenfold and more, by
+// another rounding in each pipeline). Run for the surfaces that reach the fused kernels
+// in automatic mode only, where the staged pipeline's rounding had been the result's.
+// One 128-thread workgroup per window; a thread keeps a column and walks its rows, three
+// columns and rows of the neighbourhood in registers, the next row's loads in flight.
+// Bound by its FP64 sums (17 a pixel; more waves a window would repeat the reductions).
+// ---------------------------------------------------------------------------
+constexpr int COV_NT = 128;
+template <int W>
+__global__ void __launch_bounds__(COV_NT) k_peak_cov(CoarseArgs a, int w0) {
+    constexpr int RP = W * W / COV_NT, NW = COV_NT / 64, NV = 29;   // rows per thread; t, t^2, then s, s^2, t s per lag
+    __shared__ double part[NW][NV];
+    const int win = w0 + blockIdx.x;
+    const int px = a.maxloc[2 * win], py = a.maxloc[2 * win + 1];
+    const int NLh = 2 * a.hs_d + 1, NLw = 2 * a.hs_a + 1;
+    if (px < 1 || py < 1 || px + 1 >= NLh || py + 1 >= NLw) return;     // the coarse kernel's sentinel stands
+    const int c = threadIdx.x % W, r0 = (threadIdx.x / W) * RP;
+    const int64_t t0 = (int64_t(a.ref_d[win]) + r0) * a.ref_pitch + a.ref_a[win] + c;
+    const int64_t s0 = (int64_t(a.sec_d[win]) + px - 1 + r0) * a.sec_pitch + a.sec_a[win] + py - 1 + c;
+    double st = 0.0, stt = 0.0, ts[3][3], s1[3], s2[3], s[3][3], head[2][3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        s1[j] = s2[j] = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) ts[i][j] = 0.0;
+    }
+    auto walk = [&](auto load) {
+        auto amp = [&](float2 z) { return double(raw_amp(z, a.mode)); };
+        float2 nt, ns[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            s[0][j] = head[0][j] = amp(load(a.sec, s0 + j));
+            s[1][j] = head[1][j] = amp(load(a.sec, s0 + a.sec_pitch + j));
+            ns[j] = load(a.sec, s0 + 2 * a.sec_pitch + j);
+        }
+        nt = load(a.ref, t0);
+        #pragma unroll 2
+        for (int r = 0; r < RP; ++r) {
+            const double t = amp(nt);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) s[2][j] = amp(ns[j]);
+            if (r + 1 < RP) {
+                nt = load(a.ref, t0 + (r + 1) * a.ref_pitch);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) ns[j] = load(a.sec, s0 + (r + 3) * a.sec_pitch + j);
+            }
+            st += t;
+            stt = fma(t, t, stt);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                s1[j] += s[0][j];
+                s2[j] = fma(s[0][j], s[0][j], s2[j]);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) ts[i][j] = fma(t, s[i][j], ts[i][j]);
+                s[0][j] = s[1][j];
+                s[1][j] = s[2][j];
+            }
+        }
+    };
+    if (a.mode == 2) walk([](const void *img, int64_t o) { return float2{static_cast<const float *>(img)[o], 0.f}; });
+    else walk([](const void *img, int64_t o) { return static_cast<const float2 *>(img)[o]; });
+    auto put = [&](int i, double v) {
+        v = wave_scan_f64(v);
+        if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6][i] = v;
+    };
+    put(0, st);
+    put(1, stt);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        // sums of the rows one and two further down, from the first two rows and the last
+        // two, which are left in s[0] and s[1]
+        double a1 = s1[j], a2 = s2[j];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            put(2 + 3 * (3 * i + j), a1);
+            put(3 + 3 * (3 * i + j), a2);
+            put(4 + 3 * (3 * i + j), ts[i][j]);
+            if (i < 2) {
+                a1 += s[i][j] - head[i][j];
+                a2 += s[i][j] * s[i][j] - head[i][j] * head[i][j];
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x >= 9) return;
+    auto total = [&](int i) {
+        double v = 0.0;
+        for (int w = 0; w < NW; ++w) v += part[w][i];
+        return v;
+    };
+    const int k = threadIdx.x;
+    const double n = double(W * W), tt = total(0), t2 = fmax(total(1) - tt * tt / n, 0.0);
+    const double q1 = total(2 + 3 * k), q2 = total(3 + 3 * k), qt = total(4 + 3 * k);
+    const double ncc = (qt - tt * q1 / n) / sqrt((q2 - q1 * q1 / n) * t2 + double(FLT_EPSILON));
+    double v[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) v[i] = __shfl(ncc, i);
+    if (k == 0)
+        peak_covariance([&](int dx, int dy) { return v[3 * (dx + 1) + dy + 1]; }, true, v[4], W * W, a.cov + 3 * win);
+}
+
+// ---------------------------------------------------------------------------
 // x2 chip oversampling (cuOverSampler.cpp:72-78, cuArraysPadding.cu:59-103,
 // cuDeramp.cu:67-148): per axis, odd samples = (1/N) FFT_-(FFT_+(x) e^{-i pi k_s/N}),
 // even samples = x. Output pixel (2r+p, 2c+q) comes from:
@@ -972,6 +1076,10 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
             else if (L1 == 128) launch_coarse<32, 8, 16>(K1, ca, tw1, n, w0, lds_c, st);
             else launch_coarse<32, 8, 8>(K1, ca, tw1, n, w0, lds_c, st);
         });
+        if (surf != 16) {
+            if (W == 64) hipLaunchKernelGGL(k_peak_cov<64>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
+            else hipLaunchKernelGGL(k_peak_cov<32>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
+        }
         OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, tw_ref, shift_ref, tamp, tmean};
         OsArgs osec{c.sec, c.sec_pitch, mode, c.sec_d, c.sec_a, c.start, p.deramp, tw_zoom, shift_zoom, samp, nullptr};
         FineArgs fa{tamp, tmean, samp, c.start, p.hs_down, p.hs_across, 1.0f / float(p.surf_ovs * p.raw_ovs),
