@@ -796,7 +796,14 @@ __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) 
 // LDS (TC + NL - 1 rows; the last NL - 1 carry over to the next chunk), so a
 // workgroup needs ~68 KB of LDS and two share a CU. The window sums of the
 // normalization come from FP64 column sums accumulated as the search rows
-// arrive, with the first and last NL - 1 rows kept for the slides.
+// arrive, with the first and last NL - 1 rows kept for the slides. The lag sums run on
+// the matrix cores from the transforms of packed row pairs (lag_sums), without the pass
+// that splits the pairs.
+// Bound by vector and matrix issue (about 29.7k + 2.9k instructions a window, 70% of its
+// time) and, with two workgroups a CU, by the waits between its short phases: of 3.1 ms
+// for 31,248 windows the chip loads take 0.8, the row transforms 0.5, the lag sums 0.6,
+// the normalization 0.25, the inverse 0.1 and the surface 0.45 ms. With split spectra and
+// v_fma_f32 sums (40.8k instructions, 1.0 ms for split and sums): 3.4 ms.
 // ---------------------------------------------------------------------------
 struct Fine2Lds {
     int sr, tb, save, nrm, corr, red, tw, total;   // bytes
@@ -816,8 +823,8 @@ struct Fine2Lds {
     }
 };
 
-template <int T, int R1, int R2, int K, int NTH, int TC, int SURF>
-__global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, int w0) {
+template <int T, int R1, int R2, int NTH, int TC, int SURF>
+__global__ void __launch_bounds__(NTH, 4) k_fine2(FineArgs a, const cf *tw_g, int w0) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int P = R1 * R2, L = P, PP = L + 1, H = L / 2;
     constexpr int NL = P - T + 1;            // lags per axis (17)
@@ -830,8 +837,7 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
     constexpr int Q = P / 2, TQ = T / 2;     // polyphase plane sides
     static_assert(T % TC == 0 && TC % 2 == 0 && NS % 2 == 0 && NS == 16, "even chunks, 16x16 zoom surface");
     static_assert(NCH > 1 && NS <= 2 * SRP && TC + NS <= 2 * SRP, "the kept rows lie in the first and last chunks");
-    // mac_rows reads up to K - 2 rows past a chunk's search rows; the template pairs follow them
-    static_assert(TCP >= K / 2 + 1, "the template chunk follows the search rows");
+    static_assert(R2 == 16 && R1 == NTH / 64 + 1 && TC == 32 && NL <= 17, "LagLane's and lag_sums' shapes");
     static_assert(3 * P <= NTH, "one thread per column and row-pair phase");
     static_assert(6 * P * 8 <= (TC / 2) * (P + 1) * 8, "column-sum partials fit the template chunk region");
     const Fine2Lds lay(P, NL, TC, SURF > 0 ? 16 * SURF : 16 * a.ovs);
@@ -849,68 +855,52 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
     const float *tp = a.tamp + size_t(win) * T * T;
     const float *sg = a.samp + size_t(win) * P * P;
     const double mean = a.tmean[2 * win], t2 = a.tmean[2 * win + 1];
-    // planar oversampled chips: pixel (2j + p, 2c + q) sits in plane 2p + q at (j, c)
-    auto sval = [&](int r, int x) -> float {
-        return sg[size_t(2 * (r & 1) + (x & 1)) * Q * Q + (r >> 1) * Q + (x >> 1)];
-    };
-    auto tval = [&](int r, int x) -> float {
-        return tp[size_t(2 * (r & 1) + (x & 1)) * TQ * TQ + (r >> 1) * TQ + (x >> 1)];
-    };
     // FP64 column sums of s and s^2 over rows [0, T): thread (column, phase)
     // takes the row pairs whose index is phase mod 3, both rows of a pair from
     // one load; the three partials are added in phase order by the window sums
     const int cs_c = threadIdx.x % P, cs_ph = threadIdx.x / P;
     double cs1 = 0.0, cs2 = 0.0;
 
-    const int f = threadIdx.x % H, blk = threadIdx.x / H, u0 = blk * K;
-    const bool active = (blk < NTH / H) && (u0 < NL);
-    cf q[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) q[k] = {0.f, 0.f};
-    // the MAC lanes all take the complex form; slot 0's (DC, Nyquist) lag sums come
-    // from one thread per lag and component in a wave the MAC leaves idle
-    constexpr int HB = ((NL + K - 1) / K * H + 63) / 64 * 64;
-    static_assert(NTH - HB >= 2 * NL, "an idle wave holds the slot-0 sums");
-    const int hid = int(threadIdx.x) - HB;
-    float dcn = 0.f;
+    // bins by wave (LagLane): wave 0 keeps two groups of 8 over all the chunk's template rows, the
+    // other waves one group over each half of them; the last wave adds the Nyquist sums
+    LagSums lag;
+    float nyq = 0.f;
 
+    // Chip loads: search rows [c0 + 2 first, c0 + SROWS) and template rows [c0, c0 + TC) of
+    // the planar chips (pixel (2j + p, 2c + q) in plane 2p + q at (j, c)), four columns of
+    // one parity per work item, from 16-byte loads of both rows of a pair, all of a chunk's
+    // in flight at once. Neighbouring lanes take the even and the odd columns, which halves
+    // the LDS bank conflicts of the stores against eight columns a lane. (Asked for a chunk
+    // ahead, the values spill: 3.5 ms, and 3.2 ms between the lag sums and the next chunk,
+    // against 3.1 ms for 31,248 windows.)
+    constexpr int LI = L / 4, TI = T / 4;    // work items a row pair
+    static_assert(TCP * TI == NTH && (SRP - KEEP) * LI >= NTH && SRP * LI <= 2 * NTH, "items of a chunk by thread");
+    struct Quad { float4 e0, e1; };
+    auto fetch = [&](const float *plane, int side, int row, int x) {
+        const float *b = plane + (x & 1) * side * side + row * side + 2 * (x & ~1);
+        return Quad{*reinterpret_cast<const float4 *>(b), *reinterpret_cast<const float4 *>(b + 2 * side * side)};
+    };
+    auto put = [&](cf *pair, int x, const Quad &v) {
+        cf *d = pair + 4 * (x & ~1) + (x & 1);
+        d[0] = {v.e0.x, v.e1.x}; d[2] = {v.e0.y, v.e1.y}; d[4] = {v.e0.z, v.e1.z}; d[6] = {v.e0.w, v.e1.w};
+    };
     #pragma unroll 1
     for (int ch = 0; ch < NCH; ++ch) {
         const int c0 = ch * TC;
         const int first = ch ? KEEP : 0;     // first pair slot loaded in this chunk
-        // search rows [c0 + 2 first, c0 + SROWS) into pair slots [first, SRP), eight
-        // columns per work item: four 16-byte loads (even and odd columns of both rows)
-        for (int i = threadIdx.x; i < (SRP - first) * (L / 8); i += NTH) {
-            const int jj = first + i / (L / 8), x0 = 8 * (i - (i / (L / 8)) * (L / 8));
-            const int r = c0 + 2 * jj;      // even: planes 0/1 hold row r, planes 2/3 row r + 1
-            const float *b = sg + (r >> 1) * Q + (x0 >> 1);
-            const float4 e0 = *reinterpret_cast<const float4 *>(b);
-            const float4 o0 = *reinterpret_cast<const float4 *>(b + Q * Q);
-            const float4 e1 = *reinterpret_cast<const float4 *>(b + 2 * Q * Q);
-            const float4 o1 = *reinterpret_cast<const float4 *>(b + 3 * Q * Q);
-            cf *d = SR + jj * PP + x0;
-            d[0] = {e0.x, e1.x}; d[1] = {o0.x, o1.x}; d[2] = {e0.y, e1.y}; d[3] = {o0.y, o1.y};
-            d[4] = {e0.z, e1.z}; d[5] = {o0.z, o1.z}; d[6] = {e0.w, e1.w}; d[7] = {o0.w, o1.w};
-        }
-        // template rows [c0, c0 + TC) minus the FP64 mean, zero beyond column T
-        for (int i = threadIdx.x; i < TCP * (L / 8); i += NTH) {
-            const int j = i / (L / 8), x0 = 8 * (i - j * (L / 8));
-            cf *d = TB + j * PP + x0;
-            if (x0 < T) {
-                const float *b = tp + ((c0 >> 1) + j) * TQ + (x0 >> 1);
-                const float4 e0 = *reinterpret_cast<const float4 *>(b);
-                const float4 o0 = *reinterpret_cast<const float4 *>(b + TQ * TQ);
-                const float4 e1 = *reinterpret_cast<const float4 *>(b + 2 * TQ * TQ);
-                const float4 o1 = *reinterpret_cast<const float4 *>(b + 3 * TQ * TQ);
-                auto m = [&](float v) { return float(double(v) - mean); };
-                d[0] = {m(e0.x), m(e1.x)}; d[1] = {m(o0.x), m(o1.x)}; d[2] = {m(e0.y), m(e1.y)};
-                d[3] = {m(o0.y), m(o1.y)}; d[4] = {m(e0.z), m(e1.z)}; d[5] = {m(o0.z), m(o1.z)};
-                d[6] = {m(e0.w), m(e1.w)}; d[7] = {m(o0.w), m(o1.w)};
-            } else {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) d[k] = cf{0.f, 0.f};
-            }
-        }
+        // positions worked out in place: kept over the loop, they would be spilled
+        const int tid = opaque(threadIdx.x), si1 = tid + NTH, row = ch * TCP + first;
+        Quad qs1 = {};
+        const Quad qs0 = fetch(sg, Q, row + tid / LI, tid % LI);
+        if (si1 < (SRP - first) * LI) qs1 = fetch(sg, Q, row + si1 / LI, si1 % LI);
+        const Quad qt = fetch(tp, TQ, ch * TCP + tid / TI, tid % TI);
+        put(SR + (first + tid / LI) * PP, tid % LI, qs0);
+        if (si1 < (SRP - first) * LI) put(SR + (first + si1 / LI) * PP, si1 % LI, qs1);
+        // template rows minus the FP64 mean, zero beyond column T
+        auto m = [&](float v) { return float(double(v) - mean); };
+        put(TB + tid / TI * PP, tid % TI, Quad{{m(qt.e0.x), m(qt.e0.y), m(qt.e0.z), m(qt.e0.w)},
+                                   {m(qt.e1.x), m(qt.e1.y), m(qt.e1.z), m(qt.e1.w)}});
+        for (int i = threadIdx.x; i < TCP * (L - T); i += NTH) TB[i / (L - T) * PP + T + i % (L - T)] = cf{0.f, 0.f};
         __syncthreads();
         // column sums of the new row pairs below T (T is even: no pair straddles it)
         if (cs_ph < 3) {
@@ -939,9 +929,10 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
         __syncthreads();
         // row spectra of the new search pairs and the template pairs (contiguous in LDS)
         fft_nat2dr<float, -1, R1, R2, NTH>(SR + first * PP, SRP - first + TCP, PP, 1, tw);
-        split_pairs_inplace<R1, R2, NTH>(SR + first * PP, SRP - first + TCP, PP);
-        if (active) mac_rows<H, K, false>(q, SR, PP, TB, PP, 0, 0, TC, u0, SROWS, f);
-        else if (hid >= 0 && hid < 2 * NL) dcn = dc_lag_sum<H>(dcn, SR, PP, TB, PP, TC, 0, hid >> 1, SROWS, hid & 1);
+        const LagLane<R1> ll(tid >> 6, tid & 63);
+        // half `part` of the chunk is template rows [16 part, 16 part + 16)
+        lag_sums(lag, SR + (8 * ll.part + ll.pair) * PP, TB + (8 * ll.part + ll.pair) * PP, PP, 4 * ll.halves, ll);
+        if (ll.wave == NTH / 64 - 1) nyq = nyquist_sums<TC, NL>(nyq, SR + R2 / 2, TB + R2 / 2, PP, tid & 63);
         __syncthreads();
         if (ch + 1 < NCH) {
             // the last KEEP pairs are the next chunk's first
@@ -956,12 +947,8 @@ __global__ void __launch_bounds__(NTH, 2) k_fine2(FineArgs a, const cf *tw_g, in
         part[(3 + cs_ph) * P + cs_c] = cs2;
     }
     cf *Qs = SR;
-    if (active && f != 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-            if (u0 + k < NL) Qs[(u0 + k) * H + f] = q[k];
-    }
-    if (hid >= 0 && hid < 2 * NL) reinterpret_cast<float *>(Qs + (hid >> 1) * H)[hid & 1] = dcn;
+    const LagLane<R1> ll(threadIdx.x >> 6, threadIdx.x & 63);
+    store_lag_sums<H, NL>(lag, nyq, Qs, ll, ll.wave == NTH / 64 - 1);
     __syncthreads();
     window_norms_rows<(P + 63) / 64, NTH, T % 64 == 0 ? T / 64 : 0>(
         [&](int r, int c) -> double { return double(r < NS ? save[r * P + c] : save[(NS + r - T) * P + c]); },
@@ -995,8 +982,8 @@ void launch_coarse(int K, const CoarseArgs &a, const cf *tw, int n, int w0, size
 
 // k_fine2 for the surfaces other than factor 16 by the FFT
 void launch_fine2(int surf, const FineArgs &a, const cf *tw, int n, int w0, size_t lds, hipStream_t st) {
-    if (surf == 0) hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, 0>), dim3(n), dim3(NT), lds, st, a, tw, w0);
-    else hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, -1>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+    if (surf == 0) hipLaunchKernelGGL((k_fine2<128, 9, 16, NT, 32, 0>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+    else hipLaunchKernelGGL((k_fine2<128, 9, 16, NT, 32, -1>), dim3(n), dim3(NT), lds, st, a, tw, w0);
 }
 
 }  // namespace fused
@@ -1097,7 +1084,7 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                 if (surf != 16)
                     launch_fine2(surf, fa, tw2, n, w0, lds_f2, st);
                 else if (fine_kernel == 2)
-                    hipLaunchKernelGGL((k_fine2<128, 9, 16, 3, NT, 32, 16>), dim3(n), dim3(NT), lds_f2, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine2<128, 9, 16, NT, 32, 16>), dim3(n), dim3(NT), lds_f2, st, fa, tw2, w0);
                 else if (fine_threads == 1024)
                     hipLaunchKernelGGL((k_fine<128, 9, 16, 2, 1024, 16>), dim3(n), dim3(1024), lds_f, st, fa, tw2, w0);
                 else

@@ -317,9 +317,7 @@ __device__ __forceinline__ int row_slot(int r, int P) { return (r >> 1) * P + (r
 
 // ---------------------------------------------------------------------------
 // MAC over template rows [i_beg, i_end): q[k] += conj(T_i[f]) S_{i+u0+k}[f]
-// (slot 0 packs two real bins: (DC, Nyquist) multiply component-wise; with
-// DC = false every lane takes the complex form and the caller computes slot 0's
-// sums elsewhere: dc_lag_sum). Rows sit in pairs (row r at slot (r >> 1) P +
+// (slot 0 packs two real bins: (DC, Nyquist) multiply component-wise). Rows sit in pairs (row r at slot (r >> 1) P +
 // (r & 1) H); i_beg and t_off are even and the range a multiple of 8, so a
 // thread's search rows keep the parity of u0 and every load of a block is a
 // fixed offset from one of two addresses. Template row i meets search row
@@ -328,10 +326,10 @@ __device__ __forceinline__ int row_slot(int r, int P) { return (r >> 1) * P + (r
 // lags), and the callers' LDS continues past their search rows: such rows are
 // read without a bound check and only reach sums that are discarded.
 // ---------------------------------------------------------------------------
-template <int H, int K, bool DC = true>
+template <int H, int K>
 __device__ __forceinline__ void mac_rows(cf (&q)[K], const cf *S, int Sp, const cf *Tsp, int Tp, int t_off,
                                          int i_beg, int i_end, int u0, int SH, int f) {
-    const bool dc = DC && f == 0;
+    const bool dc = f == 0;
     const int p = u0 & 1;
     const int e0 = p ? H : 0, e1 = p ? Sp : H;      // slot offset of even / odd block rows
     (void)SH;
@@ -359,22 +357,166 @@ __device__ __forceinline__ void mac_rows(cf (&q)[K], const cf *S, int Sp, const 
     }
 }
 
-// Slot 0 of mac_rows for one lag u and one component (0: DC, 1: Nyquist):
-// acc += T_i[0].comp * S_{s_off+i+u}[0].comp over template rows i in [0, n) of Tsp,
-// in mac_rows' order, so for the lags a caller keeps (whose search rows all lie
-// below SH; rows at or past it read as zero here) the sums agree bit for bit
-// with mac_rows' slot-0 lane
-template <int H, int UNROLL = 8>
-__device__ __forceinline__ float dc_lag_sum(float acc, const cf *S, int Sp, const cf *Tsp, int Tp, int n, int s_off,
-                                            int u, int SH, int comp) {
-    const float *s = reinterpret_cast<const float *>(S) + comp, *t = reinterpret_cast<const float *>(Tsp) + comp;
-    #pragma unroll UNROLL
-    for (int i = 0; i < n; ++i) {
-        const int r = s_off + i + u;
-        const float sv = (r < SH) ? s[2 * row_slot<H>(r, Sp)] : 0.f;
-        acc = fmaf(t[2 * row_slot<H>(i, Tp)], sv, acc);
+// ---------------------------------------------------------------------------
+// Lag sums on the matrix cores, for up to 17 lags and row transforms of R1 x 16 points:
+// Q[u][f] = sum_i conj(T_i[f]) S_{i+u}[f]. v_mfma_f32_4x4x1_16b multiplies, in each of 16
+// blocks of 4 lanes, a column of 4 values by a row of 4: here a block is one bin f, the
+// column 4 template rows 4 m + a, the row 4 search rows 4 (m + d) + b, so accumulator d
+// holds, for a in its registers and b in its lanes, sums for the lag 4 d + b - a. All 16
+// products of a block are wanted (17 of the 20 lags of d = 0..4 for each a), a lane loads
+// one template row and one search row for 20 instructions, and each of those does four
+// times the work of a v_fma_f32 in 2.1 times its issue time.
+// The spectra come straight from the transform of packed row pairs, Z = FFT(row 2j + i
+// row 2j+1) in digit-reversed order: row 2j + p enters as w = Z_k +- conj(Z_{L-k}), which
+// is 2 A for the even row and 2i B for the odd one; the factors (1/4, and +-i where the
+// two rows' parities differ) are applied to the finished sums.
+// ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int LAG_D = 5;                    // blocks of 4 lags met by 4 template rows: 17 + 3 <= 20
+
+struct LagSums {
+    f32x4 re[LAG_D], im[LAG_D];
+    __device__ LagSums() {
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) re[d] = im[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+};
+
+// v, of which the compiler knows nothing: what is computed from it is computed in place
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// What a lane of R1 - 1 waves works on. Bins R1 q + c, q < 8, sit next to each other in
+// digit-reversed order (storage 16 c + q; their mirrors L - k also, reversed), so a group
+// of 8 bins shares c: waves 1.. take group c = wave over the two halves of a chunk's
+// template rows, wave 0 the groups 0 and R1 - 1, each over both halves.
+template <int R1>
+struct LagLane {
+    int wave, bin, pk, pc, part, halves, pair;
+    float sign;
+    __device__ LagLane(int w, int lane) {
+        wave = __builtin_amdgcn_readfirstlane(w);
+        const int blk = lane >> 2, q = blk & 7, hi = blk >> 3;
+        const int c = wave ? wave : hi * (R1 - 1);
+        bin = R1 * q + c;
+        pk = 16 * c + q;
+        pc = c ? 16 * (R1 - c) + 15 - q : (16 - q) & 15;
+        part = wave ? hi : 0;
+        halves = wave ? 1 : 2;
+        pair = (lane >> 1) & 1;             // row a = lane & 3 of a group of 4: its pair and parity
+        sign = (lane & 1) ? -1.f : 1.f;
+    }
+};
+
+// acc += 4 M template rows (T; M > 0) against 4 (M + 4) search rows (S), both at the lane's first pair
+template <int R1>
+__device__ __forceinline__ void lag_sums(LagSums &acc, const cf *S, const cf *T, int P, int M, const LagLane<R1> &ll) {
+    // pointers to bins k and L - k; the next group's values are loaded ahead of the products
+    const cf *sk = S + ll.pk, *sc = S + ll.pc, *tk = T + ll.pk, *tc = T + ll.pc;
+    auto row = [&](cf zk, cf zc) { return cf{fmaf(ll.sign, zc.x, zk.x), fmaf(-ll.sign, zc.y, zk.y)}; };
+    cf s[LAG_D];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) s[g] = row(sk[2 * g * P], sc[2 * g * P]);
+    cf ak = sk[8 * P], ac = sc[8 * P], bk = *tk, bc = *tc;
+    #pragma unroll 4
+    for (int m = 0; m < M; ++m) {
+        s[4] = row(ak, ac);
+        const cf t = row(bk, bc);
+        const float nty = -t.y;
+        sk += 2 * P; sc += 2 * P; tk += 2 * P; tc += 2 * P;
+        if (m + 1 < M) {
+            ak = sk[8 * P]; ac = sc[8 * P]; bk = *tk; bc = *tc;
+        }
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            acc.re[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(t.x, s[d].x, acc.re[d], 0, 0, 0);
+            acc.im[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(t.x, s[d].y, acc.im[d], 0, 0, 0);
+        }
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            acc.re[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(t.y, s[d].y, acc.re[d], 0, 0, 0);
+            acc.im[d] = __builtin_amdgcn_mfma_f32_4x4x1f32(nty, s[d].x, acc.im[d], 0, 0, 0);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) s[d] = s[d + 1];
+    }
+}
+
+// Nyquist bin (real, row 2j + p in component p of S/T's pair j) of TC template rows: lane
+// u + NL k sums lag u over the k-th third of the rows
+template <int TC, int NL>
+__device__ __forceinline__ float nyquist_sums(float acc, const cf *S, const cf *T, int P, int lane) {
+    static_assert(3 * NL <= 64, "three lanes a lag");
+    constexpr int TH = (TC + 2) / 3;
+    auto at = [&](const cf *z, int r) { return reinterpret_cast<const float *>(z + (r >> 1) * P)[r & 1]; };
+    const int k = lane / NL, u = lane - k * NL;
+    if (k < 3) {
+#pragma unroll
+        for (int i = 0; i < TH; ++i) {
+            const int r = k * TH + i;
+            if (r < TC) acc = fmaf(at(T, r), at(S, r + u), acc);
+        }
     }
     return acc;
+}
+
+template <int CTRL>
+__device__ __forceinline__ float quad_perm(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// finished sums -> Qs[u][f] (slot 0: DC and Nyquist): lag 4 d + b of a bin sits in lane b
+// of its four after the sums of template row a have moved a lanes down
+template <int H, int NL, int R1>
+__device__ __forceinline__ void store_lag_sums(const LagSums &acc, float nyq, cf *Qs, const LagLane<R1> &ll, bool nyquist) {
+    const int lane = threadIdx.x & 63, b = lane & 3;
+    cf out[LAG_D];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        cf v[LAG_D + 1];
+        const bool mixed = ((a ^ b) & 1) != 0;           // rows of different parity: times i or -i
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            const float re = acc.re[d][a], im = acc.im[d][a];
+            v[d] = {mixed ? ((a & 1) ? -im : im) : re, mixed ? ((a & 1) ? re : -re) : im};
+        }
+        v[LAG_D] = {0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            if (a == 0) {
+                out[d] = v[d];
+                continue;
+            }
+            const cf s = b >= a ? v[d] : v[d + 1];
+            constexpr int rot[4] = {0xe4, 0x39, 0x4e, 0x93};
+            out[d].x += a == 1 ? quad_perm<rot[1]>(s.x) : a == 2 ? quad_perm<rot[2]>(s.x) : quad_perm<rot[3]>(s.x);
+            out[d].y += a == 1 ? quad_perm<rot[1]>(s.y) : a == 2 ? quad_perm<rot[2]>(s.y) : quad_perm<rot[3]>(s.y);
+        }
+    }
+    if (ll.halves == 1) {                                // the other half of the rows, 32 lanes up
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            out[d].x += __shfl_xor(out[d].x, 32);
+            out[d].y += __shfl_xor(out[d].y, 32);
+        }
+    }
+    if (ll.part == 0) {
+#pragma unroll
+        for (int d = 0; d < LAG_D; ++d) {
+            const int u = 4 * d + b;
+            if (u < NL) {
+                cf *q = Qs + u * H + ll.bin;
+                q->x = 0.25f * out[d].x;
+                if (ll.bin) q->y = 0.25f * out[d].y;
+            }
+        }
+    }
+    if (nyquist) {
+        const float sum = nyq + __shfl(nyq, lane + NL) + __shfl(nyq, lane + 2 * NL);
+        if (lane < NL) Qs[lane * H].y = sum;
+    }
 }
 
 // Inverse of the accumulated Q[u][f] (Qs: [NLh][H]) into corr[u][v] * nrm[u][v]
