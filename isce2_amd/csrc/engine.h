@@ -183,6 +183,7 @@ struct Engine {
     int precision = 1;
     float tau_coarse = 2e-6f, tau_fine = 2e-6f;
     long long prec_checked = 0, prec_rerun = 0;
+    int32_t *host_counts = nullptr;    // [3] page-locked: a call's windows to re-run and its first bad one
     void run(const RunArgs &a);
     void run_staged(const RunArgs &a);
     template <class T> void run_staged_t(const RunArgs &a);

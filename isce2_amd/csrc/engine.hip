@@ -56,6 +56,7 @@ void Engine::prof_collect() {
 Engine::~Engine() {
     for (auto &r : prof_pending) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto e : event_pool) (void)hipEventDestroy(e);
+    if (host_counts) (void)hipHostFree(host_counts);
 }
 
 // FP64 rows are few (re-runs of near ties): radices of at most 4 spread a row over more
@@ -907,10 +908,12 @@ __global__ void k_take_starts(const int32_t *rd, const int32_t *ra, const int32_
 // Windows to re-run in FP64, in order: first every window whose coarse margin
 // is below tc (or whose fine margin is below tf when no zoom starts are given:
 // has_start 0), then every other window whose fine margin is below tf (NaN
-// counts as below). cnt[0] = first kind, cnt[1] = both kinds. Two launches over
+// counts as below). cnt[0] = first kind, cnt[1] = both kinds, cnt[2] = the first
+// window whose chips leave their images (n if none). Two launches over
 // blocks of SEL_WIN windows (four consecutive ones per thread): the per-block
 // counts of both kinds, then each block's slots from the counts of the blocks
-// before it and a block prefix sum of the per-thread counts.
+// before it and a block prefix sum of the per-thread counts. A single block needs
+// no counts of others and is one launch (bcnt null).
 constexpr int SEL_NT = 256, SEL_WIN = 4 * SEL_NT;
 
 __device__ __forceinline__ void rerun_flags(const float *mc, const float *mf, int n, float tc, float tf,
@@ -941,6 +944,24 @@ __device__ __forceinline__ int sel_block_sum(int v, int *sh) {
     return t;
 }
 
+constexpr int CHK_NT = 256;               // windows per block of the bounds check
+static_assert(SEL_NT == 256 && CHK_NT == 256, "block_min takes four waves");
+
+// smallest v of the workgroup (256 threads) in every thread
+__device__ __forceinline__ int block_min(int v, int *sh) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return min(min(sh[0], sh[1]), min(sh[2], sh[3]));
+}
+
+__device__ __forceinline__ bool chips_inside(int64_t r, int64_t c, int64_t s, int64_t t, int64_t ref_h, int64_t ref_w,
+                                             int64_t sec_h, int64_t sec_w, int wh, int ww, int sh, int sw) {
+    return r >= 0 && c >= 0 && r + wh <= ref_h && c + ww <= ref_w && s >= 0 && t >= 0 && s + sh <= sec_h && t + sw <= sec_w;
+}
+
 __global__ void __launch_bounds__(SEL_NT) k_select_count(const float *mc, const float *mf, int n, float tc, float tf,
                                                          int has_start, int32_t *bcnt) {
     __shared__ int sh[SEL_NT / 64];
@@ -954,22 +975,26 @@ __global__ void __launch_bounds__(SEL_NT) k_select_count(const float *mc, const 
 }
 
 __global__ void __launch_bounds__(SEL_NT) k_select_write(const float *mc, const float *mf, int n, float tc, float tf,
-                                                         int has_start, const int32_t *bcnt, int nb, int32_t *idx,
-                                                         int32_t *cnt) {
+                                                         int has_start, const int32_t *bcnt, int nb,
+                                                         const int32_t *first_bad, int32_t *idx, int32_t *cnt) {
     __shared__ int sh[SEL_NT / 64], wf[SEL_NT / 64], wq[SEL_NT / 64];
     // slots of this block: first kind after the earlier blocks' first kind, second
     // kind after every first-kind window and the earlier blocks' second kind
-    int pf = 0, pq = 0, tf_ = 0, tq = 0;
-    for (int j = threadIdx.x; j < nb; j += SEL_NT) {
-        const int a = bcnt[2 * j], b = bcnt[2 * j + 1];
-        tf_ += a; tq += b;
-        if (j < int(blockIdx.x)) { pf += a; pq += b; }
-    }
-    pf = sel_block_sum(pf, sh); pq = sel_block_sum(pq, sh);
-    tf_ = sel_block_sum(tf_, sh); tq = sel_block_sum(tq, sh);
     const int i0 = blockIdx.x * SEL_WIN + 4 * threadIdx.x;
     unsigned full, fine;
     rerun_flags(mc, mf, n, tc, tf, has_start, i0, full, fine);
+    int pf = 0, pq = 0, tf_ = 0, tq = 0;
+    if (bcnt) {
+        for (int j = threadIdx.x; j < nb; j += SEL_NT) {
+            const int a = bcnt[2 * j], b = bcnt[2 * j + 1];
+            tf_ += a; tq += b;
+            if (j < int(blockIdx.x)) { pf += a; pq += b; }
+        }
+        pf = sel_block_sum(pf, sh); pq = sel_block_sum(pq, sh);
+    } else {
+        tf_ = __popc(full); tq = __popc(fine);
+    }
+    tf_ = sel_block_sum(tf_, sh); tq = sel_block_sum(tq, sh);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int mf_ = __popc(full), mq = __popc(fine);
     int xf = mf_, xq = mq;                 // inclusive prefix sums over the wave
@@ -990,10 +1015,39 @@ __global__ void __launch_bounds__(SEL_NT) k_select_write(const float *mc, const 
         if (full & (1u << j)) idx[sf++] = i0 + j;
         if (fine & (1u << j)) idx[sq++] = i0 + j;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (blockIdx.x > 0 || !cnt) return;
+    int bad = n;
+    for (int j = threadIdx.x; j < (n + CHK_NT - 1) / CHK_NT; j += SEL_NT) bad = min(bad, first_bad[j]);
+    bad = block_min(bad, sh);
+    if (threadIdx.x == 0) {
         cnt[0] = tf_;
         cnt[1] = tf_ + tq;
+        cnt[2] = bad;
+        __threadfence_system();            // cnt is in host memory
     }
+}
+
+// Bounds check of a call whose FP64 re-run reports it: sanitized starts as
+// k_sanitize_starts writes them, and each block's first window whose chips leave their
+// images (n if none) into first[block]
+__global__ void __launch_bounds__(CHK_NT) k_check_starts(const int32_t *rd, const int32_t *ra, const int32_t *sd,
+                                                         const int32_t *sa, int n, int64_t ref_h, int64_t ref_w,
+                                                         int64_t sec_h, int64_t sec_w, int wh, int ww, int sh, int sw,
+                                                         int32_t *out, int32_t *first) {
+    __shared__ int mins[CHK_NT / 64];
+    const int i = blockIdx.x * CHK_NT + threadIdx.x;
+    int bad = n;
+    if (i < n) {
+        const int32_t r = rd[i], c = ra[i], s = sd[i], t = sa[i];
+        const bool ok = chips_inside(r, c, s, t, ref_h, ref_w, sec_h, sec_w, wh, ww, sh, sw);
+        out[i] = ok ? r : 0;
+        out[n + i] = ok ? c : 0;
+        out[2 * n + i] = ok ? s : 0;
+        out[3 * n + i] = ok ? t : 0;
+        if (!ok) bad = i;
+    }
+    bad = block_min(bad, mins);
+    if (threadIdx.x == 0) first[blockIdx.x] = bad;
 }
 
 // the first window (lowest index) whose chips leave their images, or n, into *first
@@ -1003,9 +1057,7 @@ __global__ void k_first_bad(const int32_t *rd, const int32_t *ra, const int32_t 
                             int sw, int32_t *first) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const int64_t r = rd[i], c = ra[i], s = sd[i], t = sa[i];
-    if (r < 0 || c < 0 || r + wh > ref_h || c + ww > ref_w || s < 0 || t < 0 || s + sh > sec_h || t + sw > sec_w)
-        atomicMin(first, i);
+    if (!chips_inside(rd[i], ra[i], sd[i], sa[i], ref_h, ref_w, sec_h, sec_w, wh, ww, sh, sw)) atomicMin(first, i);
 }
 
 __global__ void k_set_i32(int32_t *p, int v) { *p = v; }
@@ -1025,20 +1077,32 @@ void Engine::rerun_fp64(const RunArgs &a, const float *mc, const float *mf, cons
     // the windows to re-run, selected on the device: those needing the whole
     // pipeline first, then those re-run from the zoom stage on (their coarse
     // results, SNR and covariance stay the FP32 ones); only the two counts
-    // come back to the host
-    // p_count[2]: the first window whose chips leave their images (a.n if none),
-    // set by Engine::run's bounds check
+    // come back to the host, with the first window whose chips leave its images
+    // (Engine::run's bounds check), in page-locked memory that the kernel writes:
+    // a copy of twelve bytes is a command of its own, about 10 us a call
     int32_t *d_idx = buf<int32_t>("p_idx", a.n);
-    int32_t *d_cnt = buf<int32_t>("p_count", 3);
+    if (!host_counts) {
+        void *q = nullptr;
+        if (hipHostMalloc(&q, 4 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            throw Error(AMPCOR_E_NOMEM, "page-locked allocation of 16 bytes failed");
+        }
+        host_counts = static_cast<int32_t *>(q);
+    }
+    int32_t *d_cnt = nullptr;
+    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void **>(&d_cnt), host_counts, 0));
     const int nb = idivup(a.n, SEL_WIN);
-    int32_t *d_bcnt = buf<int32_t>("p_bcount", 2 * size_t(nb));
-    hipLaunchKernelGGL(k_select_count, dim3(nb), dim3(SEL_NT), 0, a.stream, mc, mf, a.n, tau_coarse, tau_fine,
-                       start32 != nullptr, d_bcnt);
+    int32_t *d_bcnt = nullptr;
+    if (nb > 1) {
+        d_bcnt = buf<int32_t>("p_bcount", 2 * size_t(nb));
+        hipLaunchKernelGGL(k_select_count, dim3(nb), dim3(SEL_NT), 0, a.stream, mc, mf, a.n, tau_coarse, tau_fine,
+                           start32 != nullptr, d_bcnt);
+    }
     hipLaunchKernelGGL(k_select_write, dim3(nb), dim3(SEL_NT), 0, a.stream, mc, mf, a.n, tau_coarse, tau_fine,
-                       start32 != nullptr, d_bcnt, nb, d_idx, d_cnt);
-    int32_t cnt[3];
-    HIP_OK(hipMemcpyAsync(cnt, d_cnt, sizeof(cnt), hipMemcpyDeviceToHost, a.stream));
+                       start32 != nullptr, d_bcnt, nb, buf<int32_t>("p_first_bad", idivup(a.n, CHK_NT)), d_idx, d_cnt);
+    HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(a.stream));
+    const int32_t cnt[3] = {host_counts[0], host_counts[1], host_counts[2]};
     if (cnt[2] < a.n) throw Error(AMPCOR_E_RANGE, "window " + std::to_string(cnt[2]) + " reads outside its image");
     const int m_full = cnt[0], m = cnt[1];
     prec_checked += a.n;
@@ -1109,16 +1173,11 @@ void Engine::run(const RunArgs &in) {
         // bounds checked on the device and reported with the FP64 re-run's counts
         // (one host synchronization per call): out-of-image windows read window
         // (0, 0) meanwhile, and the call fails with AMPCOR_E_RANGE before the re-run
-        int32_t *cnt = buf<int32_t>("p_count", 3);
         int32_t *st4 = buf<int32_t>("ns_starts", 4 * size_t(a.n));
-        int32_t *flags = buf<int32_t>("ns_bad", a.n);
-        hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(1), 0, a.stream, cnt + 2, int(a.n));
-        hipLaunchKernelGGL(k_first_bad, dim3(idivup(a.n, 256)), dim3(256), 0, a.stream, a.ref_d, a.ref_a, a.sec_d,
-                           a.sec_a, int(a.n), a.ref_h, a.ref_w, a.sec_h, a.sec_w, p.window_h, p.window_w,
-                           sz.search_h, sz.search_w, cnt + 2);
-        hipLaunchKernelGGL(k_sanitize_starts<int32_t>, dim3(idivup(a.n, 256)), dim3(256), 0, a.stream, a.ref_d, a.ref_a,
-                           a.sec_d, a.sec_a, a.n, a.ref_h, a.ref_w, a.sec_h, a.sec_w, p.window_h, p.window_w,
-                           sz.search_h, sz.search_w, st4, flags);
+        const int nb = idivup(a.n, CHK_NT);
+        hipLaunchKernelGGL(k_check_starts, dim3(nb), dim3(CHK_NT), 0, a.stream, a.ref_d, a.ref_a, a.sec_d, a.sec_a,
+                           int(a.n), a.ref_h, a.ref_w, a.sec_h, a.sec_w, p.window_h, p.window_w, sz.search_h,
+                           sz.search_w, st4, buf<int32_t>("p_first_bad", nb));
         a.ref_d = st4; a.ref_a = st4 + a.n; a.sec_d = st4 + 2 * size_t(a.n); a.sec_a = st4 + 3 * size_t(a.n);
     } else {
         // bounds: every chip must lie inside its image, checked on the device (the
