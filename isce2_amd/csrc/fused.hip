@@ -6,6 +6,7 @@
 #include <cmath>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 #include "engine.h"
 #include "fused_kernels.h"
@@ -52,8 +53,22 @@ struct CoarseArgs {
     float *margin;                 // [n] top-1 minus top-2 of the normalized surface, or null
 };
 
-template <int W, int R1, int R2, int K>
-__global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, const cf *tw_g, int w0) {
+struct OsArgs;
+template <int R1, int R2, bool MEAN, int NTH>
+__device__ __forceinline__ void oversample_window(const OsArgs &a, int win);
+
+// With an OsArgs as `os` the launch has a second workgroup a window (from n = gridDim.x / 2
+// on) that oversamples its reference chip: neither reads what the other writes. For calls
+// of few windows, where each stage's latency is the other's idle chip (MERGE_MAX).
+template <int W, int R1, int R2, int K, class... Os>
+__global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, const cf *tw_g, int w0, Os... os) {
+    if constexpr (sizeof...(Os) > 0) {
+        const int n = int(gridDim.x >> 1);
+        if (int(blockIdx.x) >= n) {
+            oversample_window<8, W / 8, true, NT>(os..., w0 + int(blockIdx.x) - n);
+            return;
+        }
+    }
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int L = R1 * R2, H = L / 2, P = L + 1, TC = coarse_tc(W), nTc = TC / 2;
     static_assert(W % TC == 0, "template chunks cover the window");
@@ -70,7 +85,7 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
     float *nrm = reinterpret_cast<float *>(smem + lay.nrm);
     float *corr = reinterpret_cast<float *>(S + lay.corr_off);
     double *red = reinterpret_cast<double *>(smem + lay.red);
-    const int win = w0 + xcd_window(blockIdx.x, gridDim.x);
+    const int win = w0 + (sizeof...(Os) > 0 ? int(blockIdx.x) : xcd_window(blockIdx.x, gridDim.x));
     // twiddles read from LDS (the transforms' table loads wait one at a time)
     cf *twl = reinterpret_cast<cf *>(smem + lay.tw);
     for (int i = threadIdx.x; i < L; i += NT) twl[i] = tw_g[i];
@@ -344,8 +359,8 @@ __host__ __device__ inline int os_lds_bytes(int N) { return al16(N * (N + 1) * 8
 // of the workgroups that share a CU leaves room for (four of N = 64, three of N = 72)
 __host__ __device__ constexpr int os_threads(int N) { return N >= 64 ? 512 : N == 40 ? 320 : 256; }
 
-template <int R1, int R2, bool MEAN, int NTH = os_threads(R1 * R2)>
-__global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArgs a, int w0) {
+template <int R1, int R2, bool MEAN, int NTH>
+__device__ __forceinline__ void oversample_window(const OsArgs &a, int win) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int N = R1 * R2, PC = N + 1, NW = NTH / 64;
     static_assert(2 * N <= NTH, "one thread per deramp row and column factor");
@@ -359,7 +374,6 @@ __global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArg
         twl[threadIdx.x] = a.tw[threadIdx.x];
         shl[threadIdx.x] = a.shift[threadIdx.x];
     }
-    const int win = w0 + xcd_window(blockIdx.x, gridDim.x);
     int64_t r0 = a.sd[win], c0 = a.sa[win];
     if (a.start) { r0 += a.start[2 * win]; c0 += a.start[2 * win + 1]; }
     // a thread keeps one chip column and RP consecutive rows of it in registers; where the
@@ -486,6 +500,11 @@ __global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArg
             a.mean[2 * win + 1] = fmax(sum2 - sum * sum / cnt, 0.0);
         }
     }
+}
+
+template <int R1, int R2, bool MEAN, int NTH = os_threads(R1 * R2)>
+__global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArgs a, int w0) {
+    oversample_window<R1, R2, MEAN, NTH>(a, w0 + xcd_window(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------------------
@@ -969,14 +988,25 @@ int pick_k(int nl, int blocks) {
     return 0;
 }
 
+// Windows up to which the reference chips' oversampling shares the coarse stage's launch:
+// one window of either stage a CU. One window of 64: 121 -> 109 us a call; 14 x 14
+// windows: 272 -> 255 us. (Past it the coarse stage alone fills the chip.)
+constexpr int MERGE_MAX = 256;
+
+// o: the reference chips' oversampling in the same launch, or null
 template <int W, int R1, int R2>
-void launch_coarse(int K, const CoarseArgs &a, const cf *tw, int n, int w0, size_t lds, hipStream_t st) {
+void launch_coarse(int K, const CoarseArgs &a, const cf *tw, const OsArgs *o, int n, int w0, size_t lds, hipStream_t st) {
+    auto go = [&](auto k) {
+        constexpr int KK = decltype(k)::value;
+        if (o) hipLaunchKernelGGL((k_coarse<W, R1, R2, KK, OsArgs>), dim3(2 * n), dim3(NT), lds, st, a, tw, w0, *o);
+        else hipLaunchKernelGGL((k_coarse<W, R1, R2, KK>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+    };
     switch (K) {
-        case 2: hipLaunchKernelGGL((k_coarse<W, R1, R2, 2>), dim3(n), dim3(NT), lds, st, a, tw, w0); break;
-        case 3: hipLaunchKernelGGL((k_coarse<W, R1, R2, 3>), dim3(n), dim3(NT), lds, st, a, tw, w0); break;
-        case 5: hipLaunchKernelGGL((k_coarse<W, R1, R2, 5>), dim3(n), dim3(NT), lds, st, a, tw, w0); break;
-        case 6: hipLaunchKernelGGL((k_coarse<W, R1, R2, 6>), dim3(n), dim3(NT), lds, st, a, tw, w0); break;
-        default: hipLaunchKernelGGL((k_coarse<W, R1, R2, 9>), dim3(n), dim3(NT), lds, st, a, tw, w0); break;
+        case 2: go(std::integral_constant<int, 2>()); break;
+        case 3: go(std::integral_constant<int, 3>()); break;
+        case 5: go(std::integral_constant<int, 5>()); break;
+        case 6: go(std::integral_constant<int, 6>()); break;
+        default: go(std::integral_constant<int, 9>()); break;
     }
 }
 
@@ -1058,22 +1088,26 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
     const size_t lds_f = FineLds(P, P - T2 + 1, T2, sz.surf_out).total;
     const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32, sz.surf_out).total;
     {
+        OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, tw_ref, shift_ref, tamp, tmean};
+        // (a profile times the stages one by one)
+        const bool merged = n <= MERGE_MAX && !profiling;
+        const OsArgs *o = merged ? &oref : nullptr;
+        const size_t lds_m = merged ? std::max(lds_c, lds_or) : lds_c;
         timed("k_coarse", n, st, [&] {
-            if (W == 64) launch_coarse<64, 8, 16>(K1, ca, tw1, n, w0, lds_c, st);
-            else if (L1 == 128) launch_coarse<32, 8, 16>(K1, ca, tw1, n, w0, lds_c, st);
-            else launch_coarse<32, 8, 8>(K1, ca, tw1, n, w0, lds_c, st);
+            if (W == 64) launch_coarse<64, 8, 16>(K1, ca, tw1, o, n, w0, lds_m, st);
+            else if (L1 == 128) launch_coarse<32, 8, 16>(K1, ca, tw1, o, n, w0, lds_m, st);
+            else launch_coarse<32, 8, 8>(K1, ca, tw1, o, n, w0, lds_m, st);
         });
         if (surf != 16) {
             if (W == 64) hipLaunchKernelGGL(k_peak_cov<64>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
             else hipLaunchKernelGGL(k_peak_cov<32>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
         }
-        OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, tw_ref, shift_ref, tamp, tmean};
         OsArgs osec{c.sec, c.sec_pitch, mode, c.sec_d, c.sec_a, c.start, p.deramp, tw_zoom, shift_zoom, samp, nullptr};
         FineArgs fa{tamp, tmean, samp, c.start, p.hs_down, p.hs_across, 1.0f / float(p.surf_ovs * p.raw_ovs),
                     p.surf_ovs, static_cast<const cf *>(tb.tws), SincTable{sinc_table.as<float>(), sinc_dec}, c.shift,
                     c.zidx, c.offset, c.mf, c.surf ? c.surf - size_t(w0) * 256 : nullptr};
         if (W == 64) {
-            timed("k_oversample_ref", n, st, [&] {
+            if (!merged) timed("k_oversample_ref", n, st, [&] {
                 hipLaunchKernelGGL((k_oversample<8, 8, true>), dim3(n), dim3(os_threads(64)), lds_or, st, oref, w0);
             });
             timed("k_oversample_search", n, st, [&] {
@@ -1091,7 +1125,7 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                     hipLaunchKernelGGL((k_fine<128, 16, 9, 3, NT, 16>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
             });
         } else {
-            timed("k_oversample_ref", n, st, [&] {
+            if (!merged) timed("k_oversample_ref", n, st, [&] {
                 hipLaunchKernelGGL((k_oversample<8, 4, true>), dim3(n), dim3(os_threads(32)), lds_or, st, oref, w0);
             });
             timed("k_oversample_search", n, st, [&] {
