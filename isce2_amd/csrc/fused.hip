@@ -681,16 +681,14 @@ __device__ __forceinline__ void fine_surface(const FineArgs &a, const float *cor
     #pragma unroll 1
     for (int t = threadIdx.x; t < M * ncols; t += NTH) {
         const int b = t / ncols, qq = cols[t - b * ncols];
-        // e^{-2 pi i b k/SO} for k = 1..8 (negative bins use the conjugate)
-        cf w[9];
-#pragma unroll
-        for (int k = 1; k <= 8; ++k) w[k] = tws[b * k];
+        // times e^{-2 pi i b k/SO} for k = 1..8, its conjugate for the negative bins
         cf x[16];
         x[0] = G[qq];
 #pragma unroll
-        for (int k1 = 1; k1 < 16; ++k1) {
-            const cf tk = k1 < 8 ? w[k1] : conj(w[16 - k1]);
-            x[k1] = cmul(G[k1 * SO + qq], tk);
+        for (int k = 1; k <= 8; ++k) {
+            const cf w = tws[b * k];
+            if (k < 8) x[k] = cmul(G[k * SO + qq], w);
+            x[16 - k] = cmul(G[(16 - k) * SO + qq], conj(w));
         }
         dft16<float, -1>(x);
 #pragma unroll
@@ -722,8 +720,12 @@ __device__ __forceinline__ void fine_finish(const FineArgs &a, const float *corr
     else fine_surface<NTH, SURF>(a, corr, NL, work, work + 256 * (SURF ? SURF : a.ovs), cols, red, win);
 }
 
+// Windows of 32 (T = 64): 49.5 KB of LDS lets three workgroups share a CU, so registers
+// are held to 84 (about 20 spilled around the surface's evaluation); the radix-16 pass is
+// the one without twiddles, and a split round takes 36 of the 72 signals (U = 3). 15,625
+// windows: 780 -> 680 us against two workgroups a CU and radices 16, 5.
 template <int T, int R1, int R2, int K, int NTH, int SURF>
-__global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) {
+__global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const cf *tw, int w0) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int P = R1 * R2, L = P, PP = L + 1, H = L / 2, nS = P / 2;
     constexpr int NL = P - T + 1;      // 17
@@ -731,6 +733,7 @@ __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) 
     static_assert(Z == 16, "fused surface stage assumes a 16x16 zoom surface");
     // mac_rows reads up to K - 2 rows past the search; the template spectra follow it
     static_assert(T / 2 >= K / 2 + 1, "the template region follows the search rows");
+    constexpr int U = T == 64 ? 3 : 4;      // signals a thread splits at a time: two rounds either way
     const FineLds lay(P, NL, T, SURF > 0 ? 16 * SURF : 16 * a.ovs);
     cf *S = reinterpret_cast<cf *>(smem + lay.spec);
     cf *Tb = reinterpret_cast<cf *>(smem + lay.tchunk);
@@ -782,7 +785,7 @@ __global__ void __launch_bounds__(NTH) k_fine(FineArgs a, const cf *tw, int w0) 
     if (lay.tchunk == nS * PP * 8) {
         // search and template spectra are one evenly spaced set of signals
         fft_nat2dr<float, -1, R1, R2, NTH>(S, nS + T / 2, PP, 1, tw);
-        split_pairs_inplace<R1, R2, NTH>(S, nS + T / 2, PP);
+        split_pairs_inplace<R1, R2, NTH, U>(S, nS + T / 2, PP);
     } else {
         fft_nat2dr<float, -1, R1, R2, NTH>(S, nS, PP, 1, tw);
         fft_nat2dr<float, -1, R1, R2, NTH>(Tb, T / 2, PP, 1, tw);
@@ -1133,11 +1136,11 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
             });
             timed("k_fine", n, st, [&] {
                 if (surf == 16)
-                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, 16>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine<64, 5, 16, 2, NT, 16>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
                 else if (surf == 0)
-                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, 0>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine<64, 5, 16, 2, NT, 0>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
                 else
-                    hipLaunchKernelGGL((k_fine<64, 16, 5, 2, NT, -1>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
+                    hipLaunchKernelGGL((k_fine<64, 5, 16, 2, NT, -1>), dim3(n), dim3(NT), lds_f, st, fa, tw2, w0);
             });
         }
         if (c.refined)

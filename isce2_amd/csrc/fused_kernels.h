@@ -264,9 +264,9 @@ __device__ __forceinline__ void window_norms(Amp amp, int SW, int TH, int TW, in
 // slot 0 = (DC, Nyquist) of that row. A round covers whole signals only: the
 // reads of signal j (bins k and L-k) must all happen before any write to j.
 // ---------------------------------------------------------------------------
-template <int R1, int R2, int NTH = NT>
+template <int R1, int R2, int NTH = NT, int U = 4>
 __device__ __forceinline__ void split_pairs_inplace(cf *buf, int nsig, int P) {
-    constexpr int L = R1 * R2, H = L / 2, U = 4;
+    constexpr int L = R1 * R2, H = L / 2;
     // each thread keeps one bin for the whole call (its storage indices computed
     // once): bins 1..H-1 on the first SPR (H-1) threads, bin 0 on the next SPR,
     // so only the wave that holds the bin-0 threads takes both paths; a round
