@@ -62,13 +62,13 @@ typedef struct ampcor_sizes {
     int32_t os_corr_h, os_corr_w;        /* oversampled correlation surface (before trim) */
     int32_t surf_out;                    /* oversampled surface side */
     int32_t corr_raw_zoom_h, corr_raw_zoom_w; /* SNR patch */
-    int32_t fused;                       /* 1 if the fused per-window kernels cover this config */
+    int32_t fused;                       /* 1 if AMPCOR_MODE_FUSED covers this config */
     int32_t fft_corr_raw_h, fft_corr_raw_w; /* staged correlation transform sizes (>= search chip, */
     int32_t fft_corr_os_h, fft_corr_os_w;   /* smallest 2^a 3^b 5^c: any length >= the chip gives the same lags) */
 } ampcor_sizes;
 
 /* Execution modes of ampcor_run_windows. */
-#define AMPCOR_MODE_AUTO    0   /* fused when supported, else staged */
+#define AMPCOR_MODE_AUTO    0   /* fused kernels where they fit (surface factors 2..32, sinc too), else staged */
 #define AMPCOR_MODE_STAGED  1   /* one batched kernel per pipeline stage (any size) */
 #define AMPCOR_MODE_FUSED   2   /* per-window fused kernels (window <= 64 class) */
 /* Flag OR-ed into the mode: no host synchronization inside the call. Chip
