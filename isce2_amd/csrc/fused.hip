@@ -1,7 +1,8 @@
 // Fused per-window pipeline: the fast path for square windows of 32 or 64
 // pixels with 2x raw oversampling, a 16x16 zoom surface (the reference's
-// defaults) and surface oversampling by 2 to 32, by the FFT or the windowed sinc. Three kernels per chunk of windows:
-// k_coarse -> k_oversample (reference chip; search zoom chip) -> k_fine.
+// defaults) and surface oversampling by 2 to 32, by the FFT or the windowed sinc.
+// Three kernels per chunk of windows: k_coarse -> k_oversample (reference chip; search
+// zoom chip) -> k_fine.
 #include <algorithm>
 #include <cmath>
 #include <map>
