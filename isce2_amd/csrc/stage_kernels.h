@@ -409,13 +409,14 @@ struct RowJob {
 };
 
 // row pairs [t0, t0 + nr) of the job into z(k, x); org and mu hold a value per pair in LDS
+// (short rows come by more pairs than the workgroup has threads)
 template <class T, class Z>
 __device__ __forceinline__ void load_row_pairs(const RowJob<T> &j, int t0, int nr, int L, int64_t *org, T *mu, Z z) {
     const int np = (j.h + 1) / 2;
-    if (threadIdx.x < nr) {
-        const int t = t0 + threadIdx.x, win = t / np, r = 2 * (t - win * np);
-        org[threadIdx.x] = j.img ? (int64_t(win) * j.h + r) * j.w : chip_origin(j.chip, win) + r * j.chip.pitch;
-        mu[threadIdx.x] = j.mean ? T(j.mean[win]) : T(0);
+    for (int k = threadIdx.x; k < nr; k += blockDim.x) {
+        const int t = t0 + k, win = t / np, r = 2 * (t - win * np);
+        org[k] = j.img ? (int64_t(win) * j.h + r) * j.w : chip_origin(j.chip, win) + r * j.chip.pitch;
+        mu[k] = j.mean ? T(j.mean[win]) : T(0);
     }
     __syncthreads();
     auto rows = [&](auto pixels) {
