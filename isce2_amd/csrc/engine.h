@@ -32,7 +32,9 @@ struct DevBuf {
     template <class U> U *as() const { return static_cast<U *>(ptr); }
 };
 
-// FFT plan: radix schedule + FP32 and FP64 twiddle tables on the device.
+// FFT plan: radix schedule + FP32 and FP64 tables on the device, of n values each: the
+// twiddles e^{-2 pi i k/n}, then the half-sample shifts e^{-i pi k_s/n}/n, k_s = k below
+// n/2 and k - n from there on. A plan enters the engine's map once its tables are uploaded.
 struct FftPlan {
     int n = 0;
     FftDesc desc32{}, desc64{};
@@ -114,16 +116,9 @@ struct Engine {
                                           "; run the same call once before capturing it");
     }
     const FftPlan &plan(int n);
-    // [n] half-sample shifts e^{-i pi k_s/n}/n, k_s = k below n/2 and k - n from there on, in device memory
     template <class T> const cx<T> *half_shifts(int n) {
-        const std::string key = (sizeof(T) == 8 ? "d_hsh" : "f_hsh") + std::to_string(n);
-        const bool have = bufs.count(key) != 0;
-        cx<T> *dst = buf<cx<T>>(key, n);
-        if (!have) put_half_shifts(dst, n);
-        return dst;
+        return static_cast<const cx<T> *>(plan(n).tw(T())) + n;
     }
-    void put_half_shifts(cx<float> *dst, int n);
-    void put_half_shifts(cx<double> *dst, int n);
     void set_fft_radices(int n, const int32_t *radices, int count);
     template <class U> U *buf(const std::string &name, size_t count) {
         auto &b = bufs[name];
