@@ -1448,7 +1448,8 @@ __device__ __forceinline__ void sinc_patch_peak(A a, int nin, int nout, int shif
     const int rng = 2 * covs;
     const int x0 = nout / 2 - rng + shift0 * factor, y0 = nout / 2 - rng + shift1 * factor;
     const int size = min(2 * rng + 1, nout);           // distinct positions per axis
-    auto wrap = [&](int o) { return o >= nout ? o - nout : o; };
+    // from [-nout, 2 nout): the patch of the smallest surface (nin = 2) starts before it
+    auto wrap = [&](int o) { return o < 0 ? o + nout : o >= nout ? o - nout : o; };
     // integer part and phase of an output position, as the reference computes them
     auto split = [&](int o, int &i, int &f) {
         i = o / covs;
@@ -1456,6 +1457,7 @@ __device__ __forceinline__ void sinc_patch_peak(A a, int nin, int nout, int shif
     };
     auto tap = [&](int i, int p) {
         int x = i - p + TAPS / 2;
+        if (nin == 2) return x & 1;                    // fewer samples than half the taps wrap twice
         if (x < 0) x += nin;
         if (x >= nin) x -= nin;
         return x;
