@@ -27,7 +27,8 @@ __host__ __device__ constexpr int coarse_tc(int W) { return W > 32 ? 32 : W; }
 
 struct CoarseLds {
     int spec, nrm, red, tw, total, y_off, corr_off;   // bytes (spec, nrm, red, tw, total); cf units (y_off, corr_off)
-    __host__ __device__ CoarseLds(int W, int L, int SH, int NLh, int NLw) {
+    // nb: bytes of a normalization factor
+    __host__ __device__ CoarseLds(int W, int L, int SH, int NLh, int NLw, int nb) {
         const int P = L + 1, H = L / 2;
         const int nS = (SH + 1) / 2, nTc = coarse_tc(W) / 2;
         y_off = (NLh * H + 1) & ~1;                   // lag spectra Q, then the inverse pairs Y
@@ -38,7 +39,7 @@ struct CoarseLds {
         if (need > cf_units) cf_units = need;
         spec = 0;
         nrm = al16(spec + cf_units * 8);
-        red = al16(nrm + NLh * NLw * 4);
+        red = al16(nrm + NLh * NLw * nb);
         tw = red + 32 * 8;                            // the row transform's twiddles
         total = tw + L * 8;
     }
@@ -61,7 +62,7 @@ __device__ __forceinline__ void oversample_window(const OsArgs &a, int win);
 // With an OsArgs as `os` the launch has a second workgroup a window (from n = gridDim.x / 2
 // on) that oversamples its reference chip: neither reads what the other writes. For calls
 // of few windows, where each stage's latency is the other's idle chip (MERGE_MAX).
-template <int W, int R1, int R2, int K, class... Os>
+template <int W, int R1, int R2, int K, class Norms, class... Os>
 __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, const cf *tw_g, int w0, Os... os) {
     if constexpr (sizeof...(Os) > 0) {
         const int n = int(gridDim.x >> 1);
@@ -80,10 +81,10 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
     const int SH = W + 2 * a.hs_d, SW = W + 2 * a.hs_a;
     const int NLh = SH - W + 1, NLw = SW - W + 1;
     const int nS = (SH + 1) / 2;
-    const CoarseLds lay(W, L, SH, NLh, NLw);
+    const CoarseLds lay(W, L, SH, NLh, NLw, Norms::BYTES);
     cf *S = reinterpret_cast<cf *>(smem + lay.spec);
     cf *Tb = S + nS * P;
-    float *nrm = reinterpret_cast<float *>(smem + lay.nrm);
+    const Norms nrm(smem + lay.nrm, NLh * NLw);
     float *corr = reinterpret_cast<float *>(S + lay.corr_off);
     double *red = reinterpret_cast<double *>(smem + lay.red);
     const int win = w0 + (sizeof...(Os) > 0 ? int(blockIdx.x) : xcd_window(blockIdx.x, gridDim.x));
@@ -517,13 +518,18 @@ __global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArg
 // split together and the per-bin sums run over all template rows in one pass.
 // ---------------------------------------------------------------------------
 
+// normalization factors by surface stage (fine_finish)
+template <int SURF> using NormsOf = std::conditional_t<SURF == 16, Norms32, Norms48>;
+// bytes of the factors of NL x NL lags, whose place the surface's column list of SO ints takes after them
+__host__ __device__ constexpr int norm_bytes(int NL, int SO, int nb) { return NL * NL * nb > SO * 4 ? NL * NL * nb : SO * 4; }
+
 // complex values the surface stage holds: G[16][SO], the 16 x 16 spectrum, e^{-2 pi i k/SO}
 __host__ __device__ constexpr int surface_units(int SO) { return 16 * SO + 256 + SO; }
 
 struct FineLds {
     int spec, tchunk, nrm, corr, red, total, y_off;
-    // SO: surface side (16 x the surface oversampling factor)
-    __host__ __device__ FineLds(int P, int NL, int T, int SO) {
+    // SO: surface side (16 x the surface oversampling factor); nb: bytes of a normalization factor
+    __host__ __device__ FineLds(int P, int NL, int T, int SO, int nb) {
         const int L = P, PP = L + 1, H = L / 2;
         const int nS = P / 2;
         y_off = (NL * H + 1) & ~1;
@@ -536,7 +542,7 @@ struct FineLds {
         // the surface's G[16][SO], 16x16 spectrum and twiddles reuse both regions
         const int chips = tchunk + t_units * 8, surf = surface_units(SO) * 8;
         nrm = al16(chips > surf ? chips : surf);
-        corr = al16(nrm + (NL * NL > SO ? NL * NL : SO) * 4);   // the column list of the surface reuses nrm
+        corr = al16(nrm + norm_bytes(NL, SO, nb));
         red = al16(corr + NL * NL * 4);
         total = red + 64 * 8;          // block sums + workgroup argmax scratch (up to 1024 threads)
     }
@@ -735,10 +741,10 @@ __global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const
     // mac_rows reads up to K - 2 rows past the search; the template spectra follow it
     static_assert(T / 2 >= K / 2 + 1, "the template region follows the search rows");
     constexpr int U = T == 64 ? 3 : 4;      // signals a thread splits at a time: two rounds either way
-    const FineLds lay(P, NL, T, SURF > 0 ? 16 * SURF : 16 * a.ovs);
+    const FineLds lay(P, NL, T, SURF > 0 ? 16 * SURF : 16 * a.ovs, NormsOf<SURF>::BYTES);
     cf *S = reinterpret_cast<cf *>(smem + lay.spec);
     cf *Tb = reinterpret_cast<cf *>(smem + lay.tchunk);
-    float *nrm = reinterpret_cast<float *>(smem + lay.nrm);
+    const NormsOf<SURF> nrm(smem + lay.nrm, NL * NL);
     float *corr = reinterpret_cast<float *>(smem + lay.corr);
     double *red = reinterpret_cast<double *>(smem + lay.red);
     const int win = w0 + xcd_window(blockIdx.x, gridDim.x);
@@ -810,7 +816,7 @@ __global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const
     __syncthreads();
     inverse_lags<R1, R2, NTH>(Qs, NL, NL, S + lay.y_off, PP, tw, nrm, corr);
 
-    fine_finish<NTH, SURF>(a, corr, NL, S, reinterpret_cast<int *>(nrm), red, win);
+    fine_finish<NTH, SURF>(a, corr, NL, S, reinterpret_cast<int *>(smem + lay.nrm), red, win);
 }
 
 // ---------------------------------------------------------------------------
@@ -830,7 +836,7 @@ __global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const
 // ---------------------------------------------------------------------------
 struct Fine2Lds {
     int sr, tb, save, nrm, corr, red, tw, total;   // bytes
-    __host__ __device__ Fine2Lds(int P, int NL, int TC, int SO) {
+    __host__ __device__ Fine2Lds(int P, int NL, int TC, int SO, int nb) {
         const int PP = P + 1;
         const int srp = (TC + NL - 1 + 1) / 2, tcp = TC / 2;
         sr = 0;
@@ -839,7 +845,7 @@ struct Fine2Lds {
         // the surface stage reuses everything below nrm, and its column list nrm itself
         const int chips = save + 2 * (NL - 1) * P * 4, surf = surface_units(SO) * 8;
         nrm = al16(chips > surf ? chips : surf);
-        corr = al16(nrm + (NL * NL > SO ? NL * NL : SO) * 4);
+        corr = al16(nrm + norm_bytes(NL, SO, nb));
         red = al16(corr + NL * NL * 4);
         tw = red + 64 * 8;                         // the row transform's twiddles
         total = tw + P * 8;
@@ -863,11 +869,11 @@ __global__ void __launch_bounds__(NTH, 4) k_fine2(FineArgs a, const cf *tw_g, in
     static_assert(R2 == 16 && R1 == NTH / 64 + 1 && TC == 32 && NL <= 17, "LagLane's and lag_sums' shapes");
     static_assert(3 * P <= NTH, "one thread per column and row-pair phase");
     static_assert(6 * P * 8 <= (TC / 2) * (P + 1) * 8, "column-sum partials fit the template chunk region");
-    const Fine2Lds lay(P, NL, TC, SURF > 0 ? 16 * SURF : 16 * a.ovs);
+    const Fine2Lds lay(P, NL, TC, SURF > 0 ? 16 * SURF : 16 * a.ovs, NormsOf<SURF>::BYTES);
     cf *SR = reinterpret_cast<cf *>(smem + lay.sr);
     cf *TB = reinterpret_cast<cf *>(smem + lay.tb);
     float *save = reinterpret_cast<float *>(smem + lay.save);   // rows [0, NS) then [T, T + NS), pitch P
-    float *nrm = reinterpret_cast<float *>(smem + lay.nrm);
+    const NormsOf<SURF> nrm(smem + lay.nrm, NL * NL);
     float *corr = reinterpret_cast<float *>(smem + lay.corr);
     double *red = reinterpret_cast<double *>(smem + lay.red);
     // twiddles read from LDS (the transforms' table loads wait one at a time)
@@ -977,7 +983,7 @@ __global__ void __launch_bounds__(NTH, 4) k_fine2(FineArgs a, const cf *tw_g, in
         [&](int r, int c) -> double { return double(r < NS ? save[r * P + c] : save[(NS + r - T) * P + c]); },
         part, 3, P, T, T, NL, NL, t2, nrm);
     inverse_lags<R1, R2, NTH>(Qs, NL, NL, SR + ((NL * H + 1) & ~1), PP, tw, nrm, corr);
-    fine_finish<NTH, SURF>(a, corr, NL, SR, reinterpret_cast<int *>(nrm), red, win);
+    fine_finish<NTH, SURF>(a, corr, NL, SR, reinterpret_cast<int *>(smem + lay.nrm), red, win);
 }
 
 // ---------------------------------------------------------------------------
@@ -998,12 +1004,12 @@ int pick_k(int nl, int blocks) {
 constexpr int MERGE_MAX = 256;
 
 // o: the reference chips' oversampling in the same launch, or null
-template <int W, int R1, int R2>
+template <int W, int R1, int R2, class Norms>
 void launch_coarse(int K, const CoarseArgs &a, const cf *tw, const OsArgs *o, int n, int w0, size_t lds, hipStream_t st) {
     auto go = [&](auto k) {
         constexpr int KK = decltype(k)::value;
-        if (o) hipLaunchKernelGGL((k_coarse<W, R1, R2, KK, OsArgs>), dim3(2 * n), dim3(NT), lds, st, a, tw, w0, *o);
-        else hipLaunchKernelGGL((k_coarse<W, R1, R2, KK>), dim3(n), dim3(NT), lds, st, a, tw, w0);
+        if (o) hipLaunchKernelGGL((k_coarse<W, R1, R2, KK, Norms, OsArgs>), dim3(2 * n), dim3(NT), lds, st, a, tw, w0, *o);
+        else hipLaunchKernelGGL((k_coarse<W, R1, R2, KK, Norms>), dim3(n), dim3(NT), lds, st, a, tw, w0);
     };
     switch (K) {
         case 2: go(std::integral_constant<int, 2>()); break;
@@ -1013,6 +1019,17 @@ void launch_coarse(int K, const CoarseArgs &a, const cf *tw, const OsArgs *o, in
         default: go(std::integral_constant<int, 9>()); break;
     }
 }
+
+template <class Norms>
+void launch_coarse(int W, int L, int K, const CoarseArgs &a, const cf *tw, const OsArgs *o, int n, int w0, size_t lds,
+                   hipStream_t st) {
+    if (W == 64) launch_coarse<64, 8, 16, Norms>(K, a, tw, o, n, w0, lds, st);
+    else if (L == 128) launch_coarse<32, 8, 16, Norms>(K, a, tw, o, n, w0, lds, st);
+    else launch_coarse<32, 8, 8, Norms>(K, a, tw, o, n, w0, lds, st);
+}
+
+// bytes of a normalization factor (NormsOf)
+int norm_size(const ampcor_params &p) { return p.surf_ovs == 16 && p.surf_method == 0 ? Norms32::BYTES : Norms48::BYTES; }
 
 // k_fine2 for the surfaces other than factor 16 by the FFT
 void launch_fine2(int surf, const FineArgs &a, const cf *tw, int n, int w0, size_t lds, hipStream_t st) {
@@ -1034,11 +1051,12 @@ bool fused_fits(const ampcor_params &p, const ampcor_sizes &s) {
     const int L = coarse_L(s.search_w);
     if (L == 0) return false;
     if (pick_k(s.raw_corr_h, NT / (L / 2)) == 0) return false;
-    if (CoarseLds(p.window_w, L, s.search_h, s.raw_corr_h, s.raw_corr_w).total > 160 * 1024) return false;
+    const int nb = norm_size(p);
+    if (CoarseLds(p.window_w, L, s.search_h, s.raw_corr_h, s.raw_corr_w, nb).total > 160 * 1024) return false;
     // the window sums' block sums (doubles) live in the template chunk's region (cf)
     if (2 * ((s.search_h + NORM_BLK - 1) / NORM_BLK) * s.search_w > coarse_tc(p.window_w) / 2 * (L + 1)) return false;
     const int P = 2 * s.zoom_in_w;
-    if (FineLds(P, P - 2 * p.window_w + 1, 2 * p.window_w, s.surf_out).total > 160 * 1024) return false;
+    if (FineLds(P, P - 2 * p.window_w + 1, 2 * p.window_w, s.surf_out, nb).total > 160 * 1024) return false;
     return true;
 }
 
@@ -1087,10 +1105,11 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
     CoarseArgs ca{c.ref, c.ref_pitch, c.sec, c.sec_pitch, mode, c.ref_d, c.ref_a, c.sec_d, c.sec_a,
                   p.hs_down, p.hs_across, sz.half_zoom, sz.corr_raw_zoom_h, sz.corr_raw_zoom_w,
                   c.loc, c.val, c.start, c.shift, c.snr, c.cov, c.mc};
-    const size_t lds_c = CoarseLds(W, L1, sz.search_h, sz.raw_corr_h, sz.raw_corr_w).total;
+    const int nb = norm_size(p);
+    const size_t lds_c = CoarseLds(W, L1, sz.search_h, sz.raw_corr_h, sz.raw_corr_w, nb).total;
     const size_t lds_or = os_lds_bytes(W), lds_oz = os_lds_bytes(Zc);
-    const size_t lds_f = FineLds(P, P - T2 + 1, T2, sz.surf_out).total;
-    const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32, sz.surf_out).total;
+    const size_t lds_f = FineLds(P, P - T2 + 1, T2, sz.surf_out, nb).total;
+    const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32, sz.surf_out, nb).total;
     {
         OsArgs oref{c.ref, c.ref_pitch, mode, c.ref_d, c.ref_a, nullptr, p.deramp, tw_ref, shift_ref, tamp, tmean};
         // (a profile times the stages one by one)
@@ -1098,9 +1117,8 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
         const OsArgs *o = merged ? &oref : nullptr;
         const size_t lds_m = merged ? std::max(lds_c, lds_or) : lds_c;
         timed("k_coarse", n, st, [&] {
-            if (W == 64) launch_coarse<64, 8, 16>(K1, ca, tw1, o, n, w0, lds_m, st);
-            else if (L1 == 128) launch_coarse<32, 8, 16>(K1, ca, tw1, o, n, w0, lds_m, st);
-            else launch_coarse<32, 8, 8>(K1, ca, tw1, o, n, w0, lds_m, st);
+            if (surf == 16) launch_coarse<Norms32>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
+            else launch_coarse<Norms48>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
         });
         if (surf != 16) {
             if (W == 64) hipLaunchKernelGGL(k_peak_cov<64>, dim3(n), dim3(COV_NT), 0, st, ca, w0);

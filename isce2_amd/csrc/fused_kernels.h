@@ -67,6 +67,42 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 }
 
 // ---------------------------------------------------------------------------
+// Normalization factors 1/sqrt(x) of n lags in LDS, and the normalized value of a lag sum
+// c / L. The cancellation in x is resolved in FP64 either way.
+// Norms32: the hardware's reciprocal square root (within 1 ulp) of the FP32 value.
+// Norms48: the FP64 one, held as a float and the upper half of the float that is left over
+// (2^-32 of the factor), and one rounding of an FP64 product, for the surfaces whose calls
+// in automatic mode had been the staged pipeline's, which divides in FP64: x, two sums of
+// squares multiplied, leaves FP32's range where amplitudes reach about 1e7. Six bytes a
+// factor keep two workgroups a CU at window 64, half search 20 (81.6 KB each, with FP64
+// factors 84.9): command-line defaults (3,844 windows) 1.37 ms with FP64 factors.
+// ---------------------------------------------------------------------------
+struct Norms32 {
+    static constexpr int BYTES = 4;
+    float *p;
+    __device__ Norms32(void *lds, int) : p(static_cast<float *>(lds)) {}
+    __device__ __forceinline__ void put(int i, double x) const { p[i] = __builtin_amdgcn_rsqf(float(x)); }
+    template <int L> __device__ __forceinline__ float normalized(float c, int i) const { return c * (1.0f / float(L)) * p[i]; }
+};
+struct Norms48 {
+    static constexpr int BYTES = 6;
+    float *hi;
+    uint16_t *lo;
+    __device__ Norms48(void *lds, int n) : hi(static_cast<float *>(lds)), lo(reinterpret_cast<uint16_t *>(hi + n)) {}
+    __device__ __forceinline__ void put(int i, double x) const {
+        double r = __builtin_amdgcn_rsq(x);              // one Newton step to FP64
+        r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+        const float h = float(r);
+        hi[i] = h;
+        lo[i] = uint16_t(__float_as_uint(float(r - double(h))) >> 16);
+    }
+    template <int L> __device__ __forceinline__ float normalized(float c, int i) const {
+        const double r = double(hi[i]) + double(__uint_as_float(uint32_t(lo[i]) << 16));
+        return float(double(c) * r * (1.0 / L));
+    }
+};
+
+// ---------------------------------------------------------------------------
 // FP64 window sums -> nrm[u][v] = 1/sqrt((s2 - s1^2/n) t2 + FLT_EPSILON)
 // (cuCorrNormalization.cu:230-314, cuCorrNormalizationSAT.cu:237-240).
 // Vertical sums of s and s^2 over the first TH rows of every column come from
@@ -93,9 +129,9 @@ constexpr int NORM_BLOCKS = 4;
 //   and column j + TW sits in the same lane as column j, so each 64-column
 //   block of lag columns costs one wave scan of the differences plus one wave
 //   sum of the first TW columns per lag row, with no value read across lanes.
-template <int CPL, int NTH, int TWB = 0, class Amp>
+template <int CPL, int NTH, int TWB = 0, class Amp, class Norms>
 __device__ __forceinline__ void window_norms_rows(Amp amp, const double *part, int NB, int SW, int TH, int TW,
-                                                  int NLh, int NLw, double t2, float *nrm, int blk = 0) {
+                                                  int NLh, int NLw, double t2, Norms nrm, int blk = 0) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int NW = NTH / 64;
     const int per = (NLh + NW - 1) / NW;
@@ -149,7 +185,7 @@ __device__ __forceinline__ void window_norms_rows(Amp amp, const double *part, i
                 if (v < NLw) {
                     const double s1 = c1 + (x1 - d1), s2 = c2 + (x2 - d2);
                     const double norm2 = (s2 - s1 * s1 * inv_n) * t2;
-                    nrm[u * NLw + v] = __builtin_amdgcn_rsqf(float(norm2 + double(FLT_EPSILON)));
+                    nrm.put(u * NLw + v, norm2 + double(FLT_EPSILON));
                 }
                 c1 += lane63_f64(x1);
                 c2 += lane63_f64(x2);
@@ -179,9 +215,7 @@ __device__ __forceinline__ void window_norms_rows(Amp amp, const double *part, i
             if (v < NLw) {
                 const double s1 = ph1 - pl1, s2 = ph2 - pl2;
                 const double norm2 = (s2 - s1 * s1 * inv_n) * t2;
-                // the cancellation is resolved in FP64; the reciprocal square root of
-                // the FP32 result is the hardware one (within 1 ulp)
-                nrm[u * NLw + v] = __builtin_amdgcn_rsqf(float(norm2 + double(FLT_EPSILON)));
+                nrm.put(u * NLw + v, norm2 + double(FLT_EPSILON));
             }
         }
         }
@@ -204,9 +238,9 @@ __device__ __forceinline__ void window_norms_rows(Amp amp, const double *part, i
 // doubles), so that no wave slides far to its first lag row. TH must be a
 // multiple of NORM_BLK.
 constexpr int NORM_BLK = 16;
-template <int CPL, int NTH = NT, int TWB = 0, class Amp>
+template <int CPL, int NTH = NT, int TWB = 0, class Amp, class Norms>
 __device__ __forceinline__ void window_norms_blk(Amp amp, int SH, int SW, int TH, int TW, int NLh, int NLw,
-                                                 double t2, float *nrm, double *part) {
+                                                 double t2, Norms nrm, double *part) {
     const int NB = (SH + NORM_BLK - 1) / NORM_BLK;
     #pragma unroll 1
     for (int t = threadIdx.x; t < NB * SW; t += NTH) {
@@ -230,8 +264,8 @@ __device__ __forceinline__ void window_norms_blk(Amp amp, int SH, int SW, int TH
     window_norms_rows<CPL, NTH, TWB>(amp, part, NB, SW, TH, TW, NLh, NLw, t2, nrm, NORM_BLK);
 }
 
-template <int CPL, int NTH = NT, int TWB = 0, class Amp>
-__device__ __forceinline__ void window_norms(Amp amp, int SW, int TH, int TW, int NLh, int NLw, double t2, float *nrm,
+template <int CPL, int NTH = NT, int TWB = 0, class Amp, class Norms>
+__device__ __forceinline__ void window_norms(Amp amp, int SW, int TH, int TW, int NLh, int NLw, double t2, Norms nrm,
                              double *part) {
     constexpr int NB = NORM_BLOCKS;
     const int rows_per = (TH + NB - 1) / NB;
@@ -519,11 +553,11 @@ __device__ __forceinline__ void store_lag_sums(const LagSums &acc, float nyq, cf
     }
 }
 
-// Inverse of the accumulated Q[u][f] (Qs: [NLh][H]) into corr[u][v] * nrm[u][v]
+// Inverse of the accumulated Q[u][f] (Qs: [NLh][H]), times nrm[u][v], into corr[u][v]
 // for v < NLw: lag pairs (2p, 2p+1) share one complex transform placed in Y
 // (npair signals, pitch P, digit-reversed input order).
-template <int R1, int R2, int NTH = NT>
-__device__ __forceinline__ void inverse_lags(const cf *Qs, int NLh, int NLw, cf *Y, int P, const cx<float> *tw, const float *nrm,
+template <int R1, int R2, int NTH = NT, class Norms>
+__device__ __forceinline__ void inverse_lags(const cf *Qs, int NLh, int NLw, cf *Y, int P, const cx<float> *tw, Norms nrm,
                              float *corr) {
     constexpr int L = R1 * R2, H = L / 2;
     const int npair = (NLh + 1) / 2;
@@ -547,11 +581,10 @@ __device__ __forceinline__ void inverse_lags(const cf *Qs, int NLh, int NLw, cf 
     }
     __syncthreads();
     fft_dr2nat<float, +1, R1, R2, NTH>(Y, npair, P, 1, tw);
-    const float invL = 1.0f / float(L);
     for (int i = threadIdx.x; i < NLh * NLw; i += NTH) {
         const int u = i / NLw, v = i - u * NLw;
         const cf y = Y[(u >> 1) * P + v];
-        corr[i] = ((u & 1) ? y.y : y.x) * invL * nrm[i];
+        corr[i] = nrm.template normalized<L>((u & 1) ? y.y : y.x, i);
     }
     __syncthreads();
 }
