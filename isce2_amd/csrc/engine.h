@@ -32,9 +32,7 @@ struct DevBuf {
     template <class U> U *as() const { return static_cast<U *>(ptr); }
 };
 
-// FFT plan: radix schedule + FP32 and FP64 tables on the device, of n values each: the
-// twiddles e^{-2 pi i k/n}, then the half-sample shifts e^{-i pi k_s/n}/n, k_s = k below
-// n/2 and k - n from there on. A plan enters the engine's map once its tables are uploaded.
+// FFT plan: radix schedule + FP32 and FP64 twiddle tables on the device.
 struct FftPlan {
     int n = 0;
     FftDesc desc32{}, desc64{};
@@ -116,9 +114,10 @@ struct Engine {
                                           "; run the same call once before capturing it");
     }
     const FftPlan &plan(int n);
-    template <class T> const cx<T> *half_shifts(int n) {
-        return static_cast<const cx<T> *>(plan(n).tw(T())) + n;
-    }
+    // [n] half-sample shifts e^{-i pi k_s/n}/n, k_s = k below n/2 and k - n from there on, in
+    // device memory; a table enters the map once it is uploaded
+    std::map<int, std::unique_ptr<DevBuf>> shifts32, shifts64;
+    template <class T> const cx<T> *half_shifts(int n);
     void set_fft_radices(int n, const int32_t *radices, int count);
     template <class U> U *buf(const std::string &name, size_t count) {
         auto &b = bufs[name];

@@ -86,27 +86,44 @@ const FftPlan &Engine::plan(int n) {
     p->n = n;
     p->desc32 = make_schedule(n, false);
     p->desc64 = make_schedule(n, true);
-    std::vector<cx<float>> t32(2 * n);
-    std::vector<cx<double>> t64(2 * n);
+    std::vector<float> t32(2 * n);
+    std::vector<double> t64(2 * n);
     for (int k = 0; k < n; ++k) {
-        // in FP64; sin/cos of reduced angles for accuracy
-        const long double pi = 3.14159265358979323846264338327950288L;
-        const long double a = -2.0L * pi * k / n, b = -pi * (k < n / 2 ? k : k - n) / n;
-        t64[k] = {double(cosl(a)), double(sinl(a))};
-        t32[k] = {float(t64[k].x), float(t64[k].y)};
-        t64[n + k] = {double(cosl(b) / n), double(sinl(b) / n)};
-        t32[n + k] = {float(cosl(b) / n), float(sinl(b) / n)};
+        // e^{-2 pi i k/n} in FP64; sin/cos of reduced angles for accuracy
+        const long double a = -2.0L * 3.14159265358979323846264338327950288L * k / n;
+        const double c = double(cosl(a)), s = double(sinl(a));
+        t64[2 * k] = c; t64[2 * k + 1] = s;
+        t32[2 * k] = float(c); t32[2 * k + 1] = float(s);
     }
-    p->tw32.reserve(t32.size() * sizeof(t32[0]));
-    p->tw64.reserve(t64.size() * sizeof(t64[0]));
-    HIP_OK(hipMemcpy(p->tw32.ptr, t32.data(), t32.size() * sizeof(t32[0]), hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(p->tw64.ptr, t64.data(), t64.size() * sizeof(t64[0]), hipMemcpyHostToDevice));
+    p->tw32.reserve(t32.size() * sizeof(float));
+    p->tw64.reserve(t64.size() * sizeof(double));
+    HIP_OK(hipMemcpy(p->tw32.ptr, t32.data(), t32.size() * sizeof(float), hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(p->tw64.ptr, t64.data(), t64.size() * sizeof(double), hipMemcpyHostToDevice));
     p->desc32.tw = p->tw32.ptr;
     p->desc64.tw = p->tw64.ptr;
     auto &ref = *p;
     plans[n] = std::move(p);
     return ref;
 }
+
+template <class T>
+const cx<T> *Engine::half_shifts(int n) {
+    auto &tables = sizeof(T) == 8 ? shifts64 : shifts32;
+    auto it = tables.find(n);
+    if (it != tables.end()) return it->second->as<cx<T>>();
+    forbid_in_nosync("build a shift table");
+    std::vector<cx<T>> h(n);
+    for (int k = 0; k < n; ++k) {
+        const long double t = -3.14159265358979323846264338327950288L * (k < n / 2 ? k : k - n) / n;
+        h[k] = {T(cosl(t) / n), T(sinl(t) / n)};
+    }
+    std::unique_ptr<DevBuf> d(new DevBuf());
+    d->reserve(n * sizeof(cx<T>));
+    HIP_OK(hipMemcpy(d->ptr, h.data(), n * sizeof(cx<T>), hipMemcpyHostToDevice));
+    return (tables[n] = std::move(d))->template as<cx<T>>();
+}
+template const cx<float> *Engine::half_shifts(int n);
+template const cx<double> *Engine::half_shifts(int n);
 
 // cuAmpcorParameter::setupParameters (cuAmpcorParameter.cpp:70-98), with each
 // axis sized by its own half search range (the reference swaps them, :90-91).
