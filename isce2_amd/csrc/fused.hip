@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
             fft_nat2dr<float, -1, R1, R2, NT>(Tb, nTc, P, 1, tw);
             split_pairs_inplace<R1, R2>(Tb, nTc, P);
         }
-        if (active) mac_rows<H, K>(q, S, P, Tb, P, c0, c0, c0 + TC, u0, SH, f);
+        if (active) mac_row_parts<H, K, Norms::BYTES != 4>(q, S, P, Tb, P, c0, c0, c0 + TC, u0, SH, f);
         __syncthreads();
     }
     cf *Qs = S;
@@ -805,7 +805,7 @@ __global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const
     cf q[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) q[k] = {0.f, 0.f};
-    if (active) mac_rows<H, K>(q, S, PP, Tb, PP, 0, 0, T, u0, P, f);
+    if (active) mac_row_parts<H, K, SURF != 16>(q, S, PP, Tb, PP, 0, 0, T, u0, P, f);
     __syncthreads();
     cf *Qs = S;
     if (active) {

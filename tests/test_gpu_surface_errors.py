@@ -1,0 +1,47 @@
+"""FP32 errors of the fused kernels at the surfaces that automatic mode runs through them
+(factors other than 16 by the FFT): no larger than the staged pipeline's, whose calls these had
+been, in SNR, covariance, raw peak, both argmax leads and the refined offset.
+
+rms over 2,000 windows against the FP64 pipeline. Such an rms has a relative standard error of
+1.1% (Gaussian errors) to about 1.6% (their tails), the ratio of two 2.3%: bound 1.07, three of them.
+"""
+import numpy as np
+import pytest
+import torch
+
+from isce2_amd.engine import MODE_AUTO, MODE_STAGED, Engine, WindowParams
+from isce2_amd.synth import speckle_pair_shift
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("W,hs", [(64, 20), (32, 9)])
+@pytest.mark.parametrize("deramp", [0, 1])
+def test_errors_against_staged(W, hs, deramp):
+    ref, sec = speckle_pair_shift(1200, 1200, shift=(2.37, -3.21), snr_db=12.0, seed=6)
+    y, x = np.mgrid[0:1200, 0:1200]
+    ramp = np.exp(1j * (0.11 * y - 0.07 * x)).astype(np.complex64)
+    dev = torch.device("cuda", 0)
+    ref, sec = (torch.from_numpy(z * ramp).to(dev) for z in (ref, sec))
+    rng = np.random.default_rng(3)
+    d, a = rng.integers(hs, 1200 - W - hs, (2, 2000)).astype(np.int32)
+    st = [torch.as_tensor(v).to(dev) for v in (d, a, d - hs, a - hs)]
+    eng = Engine(0)
+    eng.setup(WindowParams(window_h=W, window_w=W, hs_down=hs, hs_across=hs, deramp=deramp, surf_ovs=8))
+
+    def run(precision, mode):
+        eng.set_precision(precision)
+        g = eng.run_windows(ref, sec, *st, mode=mode, debug=True, refine=True)
+        return {k: v.double().cpu().numpy() for k, v in g.items()}
+    exact, fused, staged = run(2, MODE_AUTO), run(0, MODE_AUTO), run(0, MODE_STAGED)
+    eng.close()
+    same = np.ones(2000, bool)
+    for g in (fused, staged):
+        same &= (g["start"] == exact["start"]).all(1) & (g["zoom_idx"] == exact["zoom_idx"]).all(1)
+    assert same.sum() > 1980
+    for k in ("snr", "cov", "maxval", "margin_coarse", "margin_fine", "offset_fp64"):
+        scale = np.abs(exact[k][same]).reshape(same.sum(), -1).max(1) if k in ("snr", "cov", "maxval") else 1.0
+        e, s = (np.sqrt(np.mean((np.abs(g[k][same] - exact[k][same]).reshape(same.sum(), -1).max(1) / scale) ** 2))
+                for g in (fused, staged))
+        print(f"[errors W={W} deramp={deramp}] {k}: fused {e:.3g} staged {s:.3g}")
+        assert e <= 1.07 * s, k
