@@ -56,7 +56,7 @@ struct CoarseArgs {
 };
 
 struct OsArgs;
-template <int R1, int R2, bool MEAN, int NTH>
+template <int R1, int R2, bool MEAN, int NTH, bool WIDE>
 __device__ __forceinline__ void oversample_window(const OsArgs &a, int win);
 
 // With an OsArgs as `os` the launch has a second workgroup a window (from n = gridDim.x / 2
@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
     if constexpr (sizeof...(Os) > 0) {
         const int n = int(gridDim.x >> 1);
         if (int(blockIdx.x) >= n) {
-            oversample_window<8, W / 8, true, NT>(os..., w0 + int(blockIdx.x) - n);
+            oversample_window<8, W / 8, true, NT, Norms::WIDE>(os..., w0 + int(blockIdx.x) - n);
             return;
         }
     }
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(NT, (K >= 9 ? 2 : 4)) k_coarse(CoarseArgs a, c
             fft_nat2dr<float, -1, R1, R2, NT>(Tb, nTc, P, 1, tw);
             split_pairs_inplace<R1, R2>(Tb, nTc, P);
         }
-        if (active) mac_row_parts<H, K, Norms::BYTES != 4>(q, S, P, Tb, P, c0, c0, c0 + TC, u0, SH, f);
+        if (active) mac_row_parts<H, K, Norms::WIDE>(q, S, P, Tb, P, c0, c0, c0 + TC, u0, SH, f);
         __syncthreads();
     }
     cf *Qs = S;
@@ -355,21 +355,26 @@ struct OsArgs {
 };
 
 // chip (pitch N+1), deramp row/column rotation factors, reduction scratch, twiddles, shifts
-__host__ __device__ inline int os_lds_bytes(int N) { return al16(N * (N + 1) * 8) + 4 * N * 8 + 32 * 8; }
+__host__ __device__ inline int os_lds_bytes(int N, bool wide) {
+    return al16(N * (N + 1) * 8) + 2 * N * (wide ? 16 : 8) + 32 * 8 + 2 * N * 8;
+}
 
 // threads per workgroup, and waves per SIMD to fit its registers to: as many as the LDS
 // of the workgroups that share a CU leaves room for (four of N = 64, three of N = 72)
 __host__ __device__ constexpr int os_threads(int N) { return N >= 64 ? 512 : N == 40 ? 320 : 256; }
 
-template <int R1, int R2, bool MEAN, int NTH>
+// WIDE: the deramp's factors and rotation in FP64 (deramp_apply), as the staged pipeline has
+// them, for the surfaces whose calls in automatic mode had been its (Norms48)
+template <int R1, int R2, bool MEAN, int NTH, bool WIDE>
 __device__ __forceinline__ void oversample_window(const OsArgs &a, int win) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int N = R1 * R2, PC = N + 1, NW = NTH / 64;
     static_assert(2 * N <= NTH, "one thread per deramp row and column factor");
     static_assert(4 * NW <= 32, "wave sums fit the reduction scratch");
     cf *C = reinterpret_cast<cf *>(smem);
-    cf *rowf = reinterpret_cast<cf *>(smem + al16(N * PC * 8));           // e^{i r phy}
-    cf *colf = rowf + N;                                                  // e^{i c phx}
+    using F = std::conditional_t<WIDE, double, float>;
+    cx<F> *rowf = reinterpret_cast<cx<F> *>(smem + al16(N * PC * 8));     // e^{i r phy}
+    cx<F> *colf = rowf + N;                                               // e^{i c phx}
     double *red = reinterpret_cast<double *>(colf + N);
     cf *twl = reinterpret_cast<cf *>(red + 32), *shl = twl + N;           // twiddles and shifts, read from LDS
     if (threadIdx.x < N) {
@@ -450,20 +455,24 @@ __device__ __forceinline__ void oversample_window(const OsArgs &a, int win) {
             const int k = row ? threadIdx.x : threadIdx.x - N;
             double sn, cs;
             sincos(double(k) * atan2(ai, ar), &sn, &cs);
-            (row ? rowf : colf)[k] = {float(cs), float(sn)};
+            (row ? rowf : colf)[k] = {F(cs), F(sn)};
         }
         __syncthreads();
         // rotation through float2's operator*= (float2.h:71-75: the imaginary part uses the new
         // real part); the phases and their sines and cosines are FP64, the factors and the
-        // rotation FP32
-        const cf fc = colf[c];
+        // rotation FP32 unless WIDE
+        const cx<F> fc = colf[c];
 #pragma unroll
         for (int k = 0; k < RP; ++k) {
             // read again from LDS: held through the FP64 sines, the pixels spill
             z[k] = own[k * PC];
-            const cf f = cmul(fc, rowf[rb + k]);
-            const float nx = z[k].x * f.x - z[k].y * f.y;
-            z[k] = {nx, z[k].y * f.x + nx * f.y};
+            if constexpr (WIDE) {
+                z[k] = deramp_apply(z[k], rowf[rb + k], fc);
+            } else {
+                const cf f = cmul(fc, rowf[rb + k]);
+                const float nx = z[k].x * f.x - z[k].y * f.y;
+                z[k] = {nx, z[k].y * f.x + nx * f.y};
+            }
         }
     }
     // X: even rows, even columns
@@ -504,9 +513,9 @@ __device__ __forceinline__ void oversample_window(const OsArgs &a, int win) {
     }
 }
 
-template <int R1, int R2, bool MEAN, int NTH = os_threads(R1 * R2)>
+template <int R1, int R2, bool MEAN, bool WIDE, int NTH = os_threads(R1 * R2)>
 __global__ void __launch_bounds__(NTH, R1 * R2 == 72 ? 6 : 8) k_oversample(OsArgs a, int w0) {
-    oversample_window<R1, R2, MEAN, NTH>(a, w0 + xcd_window(blockIdx.x, gridDim.x));
+    oversample_window<R1, R2, MEAN, NTH, WIDE>(a, w0 + xcd_window(blockIdx.x, gridDim.x));
 }
 
 // ---------------------------------------------------------------------------
@@ -1028,6 +1037,15 @@ void launch_coarse(int W, int L, int K, const CoarseArgs &a, const cf *tw, const
     else launch_coarse<32, 8, 8, Norms>(K, a, tw, o, n, w0, lds, st);
 }
 
+// N x N chips of n windows
+template <int R1, int R2, bool MEAN>
+void launch_oversample(bool wide, const OsArgs &a, int n, int w0, hipStream_t st) {
+    constexpr int N = R1 * R2;
+    const int lds = os_lds_bytes(N, wide);
+    if (wide) hipLaunchKernelGGL((k_oversample<R1, R2, MEAN, true>), dim3(n), dim3(os_threads(N)), lds, st, a, w0);
+    else hipLaunchKernelGGL((k_oversample<R1, R2, MEAN, false>), dim3(n), dim3(os_threads(N)), lds, st, a, w0);
+}
+
 // bytes of a normalization factor (NormsOf)
 int norm_size(const ampcor_params &p) { return p.surf_ovs == 16 && p.surf_method == 0 ? Norms32::BYTES : Norms48::BYTES; }
 
@@ -1107,7 +1125,8 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                   c.loc, c.val, c.start, c.shift, c.snr, c.cov, c.mc};
     const int nb = norm_size(p);
     const size_t lds_c = CoarseLds(W, L1, sz.search_h, sz.raw_corr_h, sz.raw_corr_w, nb).total;
-    const size_t lds_or = os_lds_bytes(W), lds_oz = os_lds_bytes(Zc);
+    const bool wide = surf != 16;
+    const size_t lds_or = os_lds_bytes(W, wide);
     const size_t lds_f = FineLds(P, P - T2 + 1, T2, sz.surf_out, nb).total;
     const size_t lds_f2 = Fine2Lds(P, P - T2 + 1, 32, sz.surf_out, nb).total;
     {
@@ -1117,10 +1136,10 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
         const OsArgs *o = merged ? &oref : nullptr;
         const size_t lds_m = merged ? std::max(lds_c, lds_or) : lds_c;
         timed("k_coarse", n, st, [&] {
-            if (surf == 16) launch_coarse<Norms32>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
-            else launch_coarse<Norms48>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
+            if (wide) launch_coarse<Norms48>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
+            else launch_coarse<Norms32>(W, L1, K1, ca, tw1, o, n, w0, lds_m, st);
         });
-        if (surf != 16) {
+        if (wide) {
             if (W == 64) hipLaunchKernelGGL(k_peak_cov<64>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
             else hipLaunchKernelGGL(k_peak_cov<32>, dim3(n), dim3(COV_NT), 0, st, ca, w0);
         }
@@ -1130,10 +1149,10 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
                     c.zidx, c.offset, c.mf, c.surf ? c.surf - size_t(w0) * 256 : nullptr};
         if (W == 64) {
             if (!merged) timed("k_oversample_ref", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 8, true>), dim3(n), dim3(os_threads(64)), lds_or, st, oref, w0);
+                launch_oversample<8, 8, true>(wide, oref, n, w0, st);
             });
             timed("k_oversample_search", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<9, 8, false>), dim3(n), dim3(os_threads(72)), lds_oz, st, osec, w0);
+                launch_oversample<9, 8, false>(wide, osec, n, w0, st);
             });
             timed("k_fine", n, st, [&] {
                 // the whole-template kernel is built for the surfaces AMPCOR_MODE_FUSED accepts
@@ -1148,10 +1167,10 @@ void Engine::launch_fused(const FusedTables &tb, const FusedLaunch &c, int n, in
             });
         } else {
             if (!merged) timed("k_oversample_ref", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<8, 4, true>), dim3(n), dim3(os_threads(32)), lds_or, st, oref, w0);
+                launch_oversample<8, 4, true>(wide, oref, n, w0, st);
             });
             timed("k_oversample_search", n, st, [&] {
-                hipLaunchKernelGGL((k_oversample<5, 8, false>), dim3(n), dim3(os_threads(40)), lds_oz, st, osec, w0);
+                launch_oversample<5, 8, false>(wide, osec, n, w0, st);
             });
             timed("k_fine", n, st, [&] {
                 if (surf == 16)

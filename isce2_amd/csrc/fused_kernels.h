@@ -79,6 +79,7 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 // ---------------------------------------------------------------------------
 struct Norms32 {
     static constexpr int BYTES = 4;
+    static constexpr bool WIDE = false;
     float *p;
     __device__ Norms32(void *lds, int) : p(static_cast<float *>(lds)) {}
     __device__ __forceinline__ void put(int i, double x) const { p[i] = __builtin_amdgcn_rsqf(float(x)); }
@@ -86,6 +87,7 @@ struct Norms32 {
 };
 struct Norms48 {
     static constexpr int BYTES = 6;
+    static constexpr bool WIDE = true;       // the kernel's other FP64 steps come with it
     float *hi;
     uint16_t *lo;
     __device__ Norms48(void *lds, int n) : hi(static_cast<float *>(lds)), lo(reinterpret_cast<uint16_t *>(hi + n)) {}

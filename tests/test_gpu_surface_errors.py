@@ -45,3 +45,32 @@ def test_errors_against_staged(W, hs, deramp):
                 for g in (fused, staged))
         print(f"[errors W={W} deramp={deramp}] {k}: fused {e:.3g} staged {s:.3g}")
         assert e <= 1.07 * s, k
+
+
+def test_refined_offset_with_deramp():
+    """Window 32 with a phase ramp: as accurate as the staged pipeline, whose deramp factors are FP64.
+    With FP32 factors the error was 1.0045 times its, with FP64 ones 0.9998 (40,000 windows; most of
+    the error is the same in both and cancels from that difference)."""
+    hs, n = 9, 40000
+    ref, sec = speckle_pair_shift(2400, 2400, shift=(2.37, -3.21), snr_db=12.0, seed=6)
+    y, x = np.mgrid[0:2400, 0:2400]
+    ramp = np.exp(1j * (0.11 * y - 0.07 * x)).astype(np.complex64)
+    dev = torch.device("cuda", 0)
+    ref, sec = (torch.from_numpy(z * ramp).to(dev) for z in (ref, sec))
+    d, a = np.random.default_rng(3).integers(hs, 2400 - 32 - hs, (2, n)).astype(np.int32)
+    st = [torch.as_tensor(v).to(dev) for v in (d, a, d - hs, a - hs)]
+    eng = Engine(0)
+    eng.setup(WindowParams(window_h=32, window_w=32, hs_down=hs, hs_across=hs, deramp=1, surf_ovs=8))
+    g = []
+    for precision, mode in ((2, MODE_AUTO), (0, MODE_AUTO), (0, MODE_STAGED)):
+        eng.set_precision(precision)
+        o = eng.run_windows(ref, sec, *st, mode=mode, debug=True, refine=True)
+        g.append({k: v.cpu().numpy() for k, v in o.items()})
+    eng.close()
+    same = np.ones(n, bool)
+    for o in g[1:]:
+        same &= (o["start"] == g[0]["start"]).all(1) & (o["zoom_idx"] == g[0]["zoom_idx"]).all(1)
+    assert same.mean() > 0.99
+    e, s = (np.sqrt(np.mean((o["offset_fp64"] - g[0]["offset_fp64"])[same] ** 2)) for o in g[1:])
+    print(f"[refined offset W=32 deramp=1] fused {e:.4g} staged {s:.4g}")
+    assert e <= 1.002 * s
