@@ -534,6 +534,16 @@ __global__ void k_given_starts(const int32_t *gs, const int32_t *gh, int f0, int
     shift[2 * i + 1] = gh[2 * i + 1];
 }
 
+// Whether an FP64 correlation's lags are summed one by one over the bins (k_lag_parts and
+// k_corr_lags: two launches, for few windows) or transformed by lag rows as the FP32 ones are.
+// The line is drawn on the direct sums' products, below which the launches decide: precision 2,
+// direct and transformed, ms: windows of 64, half search 20, n = 64 (6e6 products) 0.21 / 0.22,
+// n = 256 (2e7) 0.40 / 0.39, n = 1024 (9e7) 1.43 / 1.14; half search 50, n = 16 (1.4e7)
+// 0.20 / 0.21, n = 64 (6e7) 0.31 / 0.27; half search 200, n = 64 (2.5e9) 2.66 / 1.10.
+bool direct_lags(int windows, int NL, int NLw, int L) {
+    return double(windows) * NL * NLw * (L / 2 + 1) <= 1.5e7;
+}
+
 inline dim3 grid2(int per_img, int nimg) { return dim3(std::min(idivup(per_img, 256), 64), nimg); }
 }  // namespace
 
@@ -641,18 +651,22 @@ void Engine::run_staged_t(const RunArgs &a) {
     auto part_windows = [&](int th, int NL, int H1) {
         return std::min(size_t(nb) * idivup(th, 16), size_t(nb) + 4096 / (idivup(H1, 64) * idivup(NL, KLAG)) + 1);
     };
+    // FP64 lag rows by k_lag_parts and k_corr_lags, or transformed as the FP32 ones are
+    auto direct = [&](bool lean, int NL, int NLw, int L) {
+        return !f32 && lean && direct_lags(nb, NL, NLw, L);
+    };
     size_t spec_elems = 0, q_total = 0;
-    auto lag_rows = [&](bool lean, int th, int NL, int L) {
+    auto lag_rows = [&](bool lean, int th, int NL, int NLw, int L) {
         const int H1 = L / 2 + 1;
-        q_total = std::max(q_total, f32 || !lean ? size_t(nb) * NL * L : part_windows(th, NL, H1) * NL * H1);
+        q_total = std::max(q_total, direct(lean, NL, NLw, L) ? part_windows(th, NL, H1) * NL * H1 : size_t(nb) * NL * L);
     };
     if (row_raw) {
         spec_elems = std::max(spec_elems, size_t(W_h + S_h) * (R1w / 2 + 1));
-        lag_rows(lean_raw, W_h, sz.raw_corr_h, R1w);
+        lag_rows(lean_raw, W_h, sz.raw_corr_h, sz.raw_corr_w, R1w);
     }
     if (row_os) {
         spec_elems = std::max(spec_elems, size_t(sz.os_win_h + OSh) * (R2w / 2 + 1));
-        lag_rows(lean_os, sz.os_win_h, sz.os_corr_h, R2w);
+        lag_rows(lean_os, sz.os_win_h, sz.os_corr_h, sz.os_corr_w, R2w);
     }
     cx<T> *rspec = spec_elems ? buf<cx<T>>(tn + "rspec", size_t(nb) * spec_elems) : nullptr;
     cx<T> *rq = q_total ? buf<cx<T>>(tn + "rq", q_total) : nullptr;
@@ -695,7 +709,7 @@ void Engine::run_staged_t(const RunArgs &a) {
                        T *out, bool lean, int n) {
         row_spectra(t, s, L, n);
         if constexpr (sizeof(T) == 8) {
-            if (lean) {
+            if (direct(lean, NL, NLw, L)) {
                 const int H1 = L / 2 + 1, parts = lag_parts(t.h, NL, H1, n);
                 const int lag_blocks = idivup(parts * idivup(H1, 64) * idivup(NL, KLAG), 4);
                 hipLaunchKernelGGL((k_lag_parts<T, KLAG>), dim3(lag_blocks + idivup(block_sum_tasks(s.h, s.w), 4), n), dim3(256),

@@ -693,7 +693,7 @@ __global__ void __launch_bounds__(256) k_norm_lags(T *corr, int nl, int nlw, int
 
 // ---------------------------------------------------------------------------
 // Normalized correlation of few windows (the FP64 pipeline: re-runs of near ties, and
-// precision 2), from the row half spectra in two launches instead of four (k_mac_lags,
+// precision 2 up to direct_lags' line), from the row half spectra in two launches instead of four (k_mac_lags,
 // k_lagrows_real and the normalization). With few windows those are bound by latency (a
 // thread walks a quarter of the search rows, or a whole column), so here
 //   k_lag_parts: partial lag sums over template rows [t0, t0 + per): a wave per 64 bins,
