@@ -18,10 +18,6 @@ template <class T> __host__ __device__ __forceinline__ cx<T> operator*(cx<T> a, 
 template <class T> __host__ __device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
     return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
-// conj(a) * b
-template <class T> __host__ __device__ __forceinline__ cx<T> cmulc(cx<T> a, cx<T> b) {
-    return {a.x * b.x + a.y * b.y, a.x * b.y - a.y * b.x};
-}
 template <class T> __host__ __device__ __forceinline__ cx<T> conj(cx<T> a) { return {a.x, -a.y}; }
 // acc + conj(a) * b as two chained FMAs per component (the accumulator is the addend)
 template <class T> __device__ __forceinline__ cx<T> cmac_conj(cx<T> acc, cx<T> a, cx<T> b) {

@@ -267,16 +267,6 @@ void fft_cols(const FftPlan &pl, cx<T> *data, int nimg, int w, int elems, hipStr
     hipLaunchKernelGGL((k_fft_cols<T, DIR>), dim3(idivup(w, c), nimg), dim3(threads), lds, st, data, w, c, d);
 }
 
-template <class T, int DIR>
-void fft_rows_sel(const FftPlan &pl, cx<T> *data, int nimg, int H, int sel, int split, int off1, int elems,
-                  hipStream_t st) {
-    const FftDesc &d = std::is_same<T, float>::value ? pl.desc32 : pl.desc64;
-    const int g = std::max(1, elems / pl.n);
-    const size_t lds = 2 * size_t(g) * pl.n * sizeof(cx<T>);
-    hipLaunchKernelGGL((k_fft_rows_sel<T, DIR>), dim3(idivup(nimg * sel, g)), dim3(256), lds, st, data, nimg, H, sel,
-                       split, off1, g, d);
-}
-
 template <class T>
 int fft_elems(const Engine &e) { return sizeof(T) == 8 ? std::max(1024, e.fft_block_elems / 2) : e.fft_block_elems; }
 
@@ -300,14 +290,6 @@ void fft2_quad(Engine &e, const cx<T> *in, int nimg, int h, int w, cx<T> *work, 
     const int c = cols_per_block<T>(pc, W, elems, cols_width<T>(e));
     hipLaunchKernelGGL((k_fft_cols_quad<T, DIR, OUT>), dim3(idivup(W, c), nimg), dim3(c >= 16 ? 512 : 256),
                        2 * size_t(c) * H * sizeof(cx<T>), st, work, W, c, h / 2, f32 ? pc.desc32 : pc.desc64, out);
-}
-
-// 2D FFT of which only rows [0, keep) of the result are used: columns first,
-// then only those rows
-template <class T, int DIR>
-void fft2_rows_kept(Engine &e, cx<T> *data, int nimg, int h, int w, int keep, hipStream_t st) {
-    fft_cols<T, DIR>(e.plan(h), data, nimg, w, fft_elems<T>(e), st, cols_width<T>(e));
-    fft_rows_sel<T, DIR>(e.plan(w), data, nimg, h, keep, keep, 0, fft_elems<T>(e), st);
 }
 
 // 2D FFT of nimg images h x w (rows then columns), in place
@@ -557,8 +539,8 @@ void Engine::run_staged_t(const RunArgs &a) {
     const int S_h = sz.search_h, S_w = sz.search_w;
     const int chunk = std::min(a.chunk > 0 ? a.chunk : 1024, 65535);
     const int mode = p.image_complex ? (p.deramp == 0 ? 1 : 0) : 2;
-    // correlation transform sizes (5-smooth, >= the search chips)
-    const int L1h = sz.fft_corr_raw_h, L1w = sz.fft_corr_raw_w, L2h = sz.fft_corr_os_h, L2w = sz.fft_corr_os_w;
+    // correlation row transform sizes (5-smooth, >= the search chips)
+    const int L1w = sz.fft_corr_raw_w, L2w = sz.fft_corr_os_w;
     const int Z = sz.zoom, So = sz.surf_out;
     const int OSh = sz.os_search_h, OSw = sz.os_search_w;   // oversampled zoom chip (fixed by the interpolation)
     const int nb = std::min(chunk, a.n);
@@ -569,14 +551,10 @@ void Engine::run_staged_t(const RunArgs &a) {
 
     // Correlations through row spectra (k_rowspec, k_mac_lags, k_lagrows_real): row
     // FFTs of the template and search rows, per-bin sums over template rows for each
-    // lag row, and row IFFTs of the lag rows only. The padded 2-D FFT route remains
-    // for shapes whose row pairs outnumber the transform rows.
-    auto fits_rows = [&](int th, int sh, int Lh) { return (th + 1) / 2 + (sh + 1) / 2 <= Lh; };
-    const bool row_raw = fits_rows(W_h, S_h, L1h), row_os = fits_rows(sz.os_win_h, OSh, L2h);
-    // with them and the two-pass normalization (up to 1024 search columns) no mean-free
-    // template image is needed: the mean is subtracted as the template rows load, and the
-    // raw stage's rows are the amplitudes of chips read in place
-    const bool lean_raw = row_raw && S_w <= 1024, lean_os = row_os && OSw <= 1024;
+    // lag row, and row IFFTs of the lag rows only. With the two-pass normalization (up to
+    // 1024 search columns) no mean-free template image is needed: the mean is subtracted as
+    // the template rows load, and the raw stage's rows are the amplitudes of chips read in place
+    const bool lean_raw = S_w <= 1024, lean_os = OSw <= 1024;
     // the separable oversampler covers the x2 interpolation of even-sided chips (an
     // odd side loses its middle spectrum line to the quadrant padding, which does
     // not factor into the half-sample form)
@@ -636,10 +614,6 @@ void Engine::run_staged_t(const RunArgs &a) {
     T *corr_os = buf<T>(tn + "corr_os", size_t(nb) * sz.os_corr_h * sz.os_corr_w);
     const int nparts = sz.os_win_h / os2_rows_per_block<T>(W_w);
     double *os_part = part_mean ? buf<double>(tn + "os_part", size_t(nb) * 2 * nparts) : nullptr;
-    size_t zmax = 0;
-    if (!row_raw) zmax = size_t(L1h) * L1w;
-    if (!row_os) zmax = std::max(zmax, size_t(L2h) * L2w);
-    cx<T> *zc = zmax ? buf<cx<T>>(tn + "zc", size_t(nb) * zmax) : nullptr;
     // few windows (FP64): parts of the template rows whose lag sums are taken apart (k_lag_parts),
     // enough of 16 rows or more to leave about 4096 waves
     constexpr int KLAG = 9;
@@ -655,21 +629,16 @@ void Engine::run_staged_t(const RunArgs &a) {
     auto direct = [&](bool lean, int NL, int NLw, int L) {
         return !f32 && lean && direct_lags(nb, NL, NLw, L);
     };
-    size_t spec_elems = 0, q_total = 0;
+    size_t q_total = 0;
     auto lag_rows = [&](bool lean, int th, int NL, int NLw, int L) {
         const int H1 = L / 2 + 1;
         q_total = std::max(q_total, direct(lean, NL, NLw, L) ? part_windows(th, NL, H1) * NL * H1 : size_t(nb) * NL * L);
     };
-    if (row_raw) {
-        spec_elems = std::max(spec_elems, size_t(W_h + S_h) * (R1w / 2 + 1));
-        lag_rows(lean_raw, W_h, sz.raw_corr_h, sz.raw_corr_w, R1w);
-    }
-    if (row_os) {
-        spec_elems = std::max(spec_elems, size_t(sz.os_win_h + OSh) * (R2w / 2 + 1));
-        lag_rows(lean_os, sz.os_win_h, sz.os_corr_h, sz.os_corr_w, R2w);
-    }
-    cx<T> *rspec = spec_elems ? buf<cx<T>>(tn + "rspec", size_t(nb) * spec_elems) : nullptr;
-    cx<T> *rq = q_total ? buf<cx<T>>(tn + "rq", q_total) : nullptr;
+    lag_rows(lean_raw, W_h, sz.raw_corr_h, sz.raw_corr_w, R1w);
+    lag_rows(lean_os, sz.os_win_h, sz.os_corr_h, sz.os_corr_w, R2w);
+    const size_t spec_elems = std::max(size_t(W_h + S_h) * (R1w / 2 + 1), size_t(sz.os_win_h + OSh) * (R2w / 2 + 1));
+    cx<T> *rspec = buf<cx<T>>(tn + "rspec", size_t(nb) * spec_elems);
+    cx<T> *rq = buf<cx<T>>(tn + "rq", q_total);
     // row half spectra of the template (mean subtracted on load when given) and the search
     auto row_spectra = [&](RowJob<T> t, RowJob<T> s, int L, int n) {
         t.spec = rspec;
@@ -725,16 +694,6 @@ void Engine::run_staged_t(const RunArgs &a) {
         row_correlate(t.h, s.h, L, NL, NLw, out, n);
         normalize(out, NL, NLw, tm, t.h, t.w, sr, s.h, s.w, ssd, n);
     };
-    // ... through the padded 2-D FFT of two packed real images
-    auto fft_ncc = [&](const T *tm, int th, int tw, const T *sr, int sh, int sw, int Lh, int Lw, int NL, int NLw, const double *ssd,
-                       T *out, int n) {
-        hipLaunchKernelGGL(k_pack_corr<T>, grid2(Lh * Lw, n), dim3(256), 0, st, tm, th, tw, sr, sh, sw, zc, Lh, Lw);
-        fft2<T, -1>(*this, zc, n, Lh, Lw, st);
-        hipLaunchKernelGGL(k_spec_product<T>, grid2(Lh * Lw, n), dim3(256), 0, st, zc, Lh, Lw, T(1.0 / (double(Lh) * Lw)));
-        fft2_rows_kept<T, +1>(*this, zc, n, Lh, Lw, NL, st);
-        hipLaunchKernelGGL(k_crop_real<T>, grid2(NL * NLw, n), dim3(256), 0, st, zc, Lh, Lw, out, NL, NLw);
-        normalize(out, NL, NLw, tm, th, tw, sr, sh, sw, ssd, n);
-    };
     // the 16-sparse surface kernel and the sinc patch kernel keep no surface in HBM
     // (190 windows of 256 at factor 32: 3.10 ms with 512 x 512 surfaces transformed and
     // searched in HBM, 2.04 ms without; an FP64 G[16][SO] fits a workgroup's LDS up to
@@ -779,12 +738,9 @@ void Engine::run_staged_t(const RunArgs &a) {
             } else {
                 hipLaunchKernelGGL(k_sub_mean<T>, dim3(nraw), dim3(per_window), 0, st, r_ref, W_h * W_w,
                                    ssd_raw);
-                if (row_raw)
-                    row_ncc(RowJob<T>{r_ref, {}, W_h, W_w, nullptr, nullptr, nullptr, 0},
-                            RowJob<T>{r_sec, {}, S_h, S_w, nullptr, nullptr, nullptr, 0}, r_ref, r_sec, R1w, sz.raw_corr_h,
-                            sz.raw_corr_w, ssd_raw, corr, false, nraw);
-                else
-                    fft_ncc(r_ref, W_h, W_w, r_sec, S_h, S_w, L1h, L1w, sz.raw_corr_h, sz.raw_corr_w, ssd_raw, corr, nraw);
+                row_ncc(RowJob<T>{r_ref, {}, W_h, W_w, nullptr, nullptr, nullptr, 0},
+                        RowJob<T>{r_sec, {}, S_h, S_w, nullptr, nullptr, nullptr, 0}, r_ref, r_sec, R1w, sz.raw_corr_h,
+                        sz.raw_corr_w, ssd_raw, corr, false, nraw);
             }
             // argmax, covariance, SNR, zoom start/shift (cuAmpcorChunk.cpp:69-106)
             hipLaunchKernelGGL(k_peak<T>, dim3(nraw), dim3(256), 0, st, corr, sz.raw_corr_h, sz.raw_corr_w, W_h * W_w,
@@ -836,13 +792,9 @@ void Engine::run_staged_t(const RunArgs &a) {
         } else {
             hipLaunchKernelGGL(k_sub_mean<T>, dim3(n), dim3(per_window), 0, st, r_ref_os,
                                sz.os_win_h * sz.os_win_w, ssd_os);
-            if (row_os)
-                row_ncc(RowJob<T>{r_ref_os, {}, sz.os_win_h, sz.os_win_w, nullptr, nullptr, nullptr, 0},
-                        RowJob<T>{r_sec_os, {}, OSh, OSw, nullptr, nullptr, nullptr, 0}, r_ref_os, r_sec_os, R2w, sz.os_corr_h,
-                        sz.os_corr_w, ssd_os, corr_os, false, n);
-            else
-                fft_ncc(r_ref_os, sz.os_win_h, sz.os_win_w, r_sec_os, OSh, OSw, L2h, L2w, sz.os_corr_h, sz.os_corr_w, ssd_os,
-                        corr_os, n);
+            row_ncc(RowJob<T>{r_ref_os, {}, sz.os_win_h, sz.os_win_w, nullptr, nullptr, nullptr, 0},
+                    RowJob<T>{r_sec_os, {}, OSh, OSw, nullptr, nullptr, nullptr, 0}, r_ref_os, r_sec_os, R2w, sz.os_corr_h,
+                    sz.os_corr_w, ssd_os, corr_os, false, n);
         }
         // trim + surface oversampling + argmax + sub-pixel offset (cuAmpcorChunk.cpp:169-207)
         float *mf = a.margin_fine ? a.margin_fine + w0 : nullptr;

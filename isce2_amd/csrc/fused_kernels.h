@@ -19,13 +19,7 @@ constexpr int NT = 512;   // threads per workgroup (8 wave64)
 
 using cf = cx<float>;
 
-__device__ __forceinline__ float pixel_amp(const void *img, int mode, int64_t off) {
-    if (mode == 2) return fabsf(static_cast<const float *>(img)[off]);
-    const float2 z = static_cast<const float2 *>(img)[off];
-    return fast_sqrt(z.x * z.x + z.y * z.y);
-}
-
-// one pixel as loaded (real images: (value, 0)); raw_amp gives what pixel_amp gives
+// one pixel as loaded (real images: (value, 0)), and its amplitude
 __device__ __forceinline__ float2 pixel_raw(const void *img, int mode, int64_t off) {
     if (mode == 2) return {static_cast<const float *>(img)[off], 0.f};
     return static_cast<const float2 *>(img)[off];
@@ -33,13 +27,6 @@ __device__ __forceinline__ float2 pixel_raw(const void *img, int mode, int64_t o
 
 __device__ __forceinline__ float raw_amp(float2 z, int mode) {
     return mode == 2 ? fabsf(z.x) : fast_sqrt(z.x * z.x + z.y * z.y);
-}
-
-__device__ __forceinline__ cf pixel_cx(const void *img, int mode, int64_t off) {
-    if (mode == 2) return {static_cast<const float *>(img)[off], 0.f};
-    const float2 z = static_cast<const float2 *>(img)[off];
-    if (mode == 1) return {fast_sqrt(z.x * z.x + z.y * z.y), 0.f};
-    return {z.x, z.y};
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
@@ -346,10 +333,6 @@ __device__ __forceinline__ void split_pairs_inplace(cf *buf, int nsig, int P) {
         __syncthreads();
     }
 }
-
-// address of row r's half spectrum after split_pairs_inplace
-template <int H>
-__device__ __forceinline__ int row_slot(int r, int P) { return (r >> 1) * P + (r & 1) * H; }
 
 // ---------------------------------------------------------------------------
 // MAC over template rows [i_beg, i_end): q[k] += conj(T_i[f]) S_{i+u0+k}[f]

@@ -29,35 +29,6 @@ __global__ void __launch_bounds__(256) k_fft_rows(cx<T> *data, int nrows, int g,
     for (int i = threadIdx.x; i < tot; i += blockDim.x) base[i] = res[i];
 }
 
-// rows of length d.n selected per image: of the `sel` selected rows of each
-// [H][d.n] image, rows s < split are row s and the others row off1 + s - split
-// (the non-zero rows of a quadrant-padded spectrum, or the leading rows an
-// inverse correlation keeps); `g` selected rows per block
-template <class T, int DIR>
-__global__ void __launch_bounds__(256) k_fft_rows_sel(cx<T> *data, int nimg, int H, int sel, int split, int off1,
-                                                      int g, FftDesc d) {
-    extern __shared__ unsigned char smem_raw[];
-    cx<T> *a = reinterpret_cast<cx<T> *>(smem_raw);
-    cx<T> *b = a + g * d.n;
-    const int t0 = blockIdx.x * g;
-    const int nr = min(g, nimg * sel - t0);
-    auto row = [&](int k) {
-        const int t = t0 + k, img = t / sel, sr = t - img * sel;
-        const int r = sr < split ? sr : off1 + (sr - split);
-        return data + (size_t(img) * H + r) * d.n;
-    };
-    for (int i = threadIdx.x; i < nr * d.n; i += blockDim.x) {
-        const int k = i / d.n, c = i - k * d.n;
-        a[i] = row(k)[c];
-    }
-    __syncthreads();
-    cx<T> *res = fft_lds<T, DIR>(a, b, d, nr, 1, d.n);
-    for (int i = threadIdx.x; i < nr * d.n; i += blockDim.x) {
-        const int k = i / d.n, c = i - k * d.n;
-        row(k)[c] = res[i];
-    }
-}
-
 // columns: images [nimg][h][w] with h = d.n; `c` columns per block
 template <class T, int DIR>
 __global__ void __launch_bounds__(512) k_fft_cols(cx<T> *data, int w, int c, FftDesc d) {
@@ -341,47 +312,6 @@ __global__ void __launch_bounds__(256) k_chip_sums(ChipSrc src, int h, int w, do
 }
 
 // ---------------------------------------------------------------------------
-// correlation via one complex 2D FFT of z = t_pad + i*s (cuCorrFrequency.cu:63-111)
-// ---------------------------------------------------------------------------
-template <class T>
-__global__ void k_pack_corr(const T *tmpl, int th, int tw, const T *srch, int sh, int sw,
-                            cx<T> *z, int Lh, int Lw) {
-    const int win = blockIdx.y;
-    const int tot = Lh * Lw;
-    const T *t = tmpl + size_t(win) * th * tw;
-    const T *s = srch + size_t(win) * sh * sw;
-    cx<T> *o = z + size_t(win) * tot;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
-        const int r = i / Lw, c = i - r * Lw;
-        const T a = (r < th && c < tw) ? t[r * tw + c] : T(0);
-        const T b = (r < sh && c < sw) ? s[r * sw + c] : T(0);
-        o[i] = {a, b};
-    }
-}
-
-// P[k] = conj(T[k]) S[k] / L^2 with T = (Z[k] + conj Z[-k])/2, S = (Z[k] - conj Z[-k])/(2i);
-// P[-k] = conj(P[k]). One thread per (k, -k) pair.
-template <class T>
-__global__ void k_spec_product(cx<T> *z, int Lh, int Lw, T scale) {
-    const int win = blockIdx.y;
-    cx<T> *Z = z + size_t(win) * Lh * Lw;
-    const int tot = Lh * Lw;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
-        const int r = i / Lw, c = i - r * Lw;
-        const int rn = r ? Lh - r : 0, cn = c ? Lw - c : 0;
-        const int j = rn * Lw + cn;
-        if (j < i) continue;   // pair handled by the smaller index
-        const cx<T> a = Z[i], bc = conj(Z[j]);
-        const cx<T> tk = (a + bc) * T(0.5);
-        const cx<T> d = (a - bc) * T(0.5);
-        const cx<T> sk = {d.y, -d.x};   // d / i
-        const cx<T> p = cmulc(tk, sk) * scale;
-        Z[i] = p;
-        if (j != i) Z[j] = conj(p);
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Row-spectrum correlation over NL lag rows:
 //   c[u][v] = (1/L) IFFT_L( sum_t conj(T_t) S_{t+u} )[v],   0 <= u < NL,
 // equal to the zero-padded 2-D correlation (cuCorrFrequency.cu:63-79) at every
@@ -505,7 +435,7 @@ __global__ void __launch_bounds__(NTH) k_rowspec_f(RowJob<T> a, RowJob<T> b, int
     store_row_spectra(j, t0, nr, L, [&](int k, int bin) { return C[k * PR + dr_pos<R1, R2>(bin)]; });
 }
 
-// the inverse row FFT of the lag rows and k_crop_real in one pass: rows t of
+// the inverse row FFT of the lag rows and its real part: rows t of
 // length d.n (t = window * nl + lag) -> out[t][v] = Re, v < nlw; `g` rows per block
 template <class T>
 __global__ void __launch_bounds__(256) k_lagrows_real(const cx<T> *q, int nrows, int g, FftDesc d, int nlw, T *out) {
@@ -784,17 +714,6 @@ __global__ void __launch_bounds__(256) k_corr_lags(const cx<T> *q, int parts, in
         if (slice == 0)
             out[(size_t(win) * nl + u0 + j) * nlw + v] =
                 T(double(acc) / double(L) / sqrt(lag_norm2(V, j, sw, v, tw, inv, t2) + double(FLT_EPSILON)));
-    }
-}
-
-// real part of the top-left oh x ow block
-template <class T>
-__global__ void k_crop_real(const cx<T> *z, int Lh, int Lw, T *out, int oh, int ow) {
-    const int win = blockIdx.y;
-    const int tot = oh * ow;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
-        const int r = i / ow, c = i - r * ow;
-        out[size_t(win) * tot + i] = z[size_t(win) * Lh * Lw + r * Lw + c].x;
     }
 }
 
