@@ -32,10 +32,17 @@ struct DevBuf {
     template <class U> U *as() const { return static_cast<U *>(ptr); }
 };
 
-// FFT plan: radix schedule + FP32 and FP64 twiddle tables on the device.
+// FFT plan: radix schedules + FP32 and FP64 twiddle tables on the device. FP64 rows of few
+// windows (re-runs of near ties) have a schedule of their own: radices of at most 4 spread a
+// row over more threads (a radix-16 pass of 144 points has 9 butterflies), where many windows
+// give threads enough and a pass less counts.
 struct FftPlan {
+    static constexpr int FEW = 256;       // windows
     int n = 0;
-    FftDesc desc32{}, desc64{};
+    FftDesc desc32{}, desc64{}, desc64_few{};
+    template <class T> const FftDesc &desc(int nwin) const {
+        return sizeof(T) == 4 ? desc32 : nwin < FEW ? desc64_few : desc64;
+    }
     DevBuf tw32, tw64;
     const void *tw(float) const { return tw32.ptr; }
     const void *tw(double) const { return tw64.ptr; }
@@ -192,8 +199,8 @@ struct Engine {
     void run_noalloc(const RunArgs &a);
 };
 
-// FFT schedule for length n (radices in pass order; direct DFT if a prime > 17 remains)
-FftDesc make_schedule(int n, bool f64);
+// FFT schedule for length n (radices in pass order; direct DFT if a prime > 17 remains); few: radices of at most 4
+FftDesc make_schedule(int n, bool few);
 // whether the fused kernels can run a configuration (what AMPCOR_MODE_AUTO goes by), and
 // whether it is one of those that AMPCOR_MODE_FUSED and the allocation-free entry accept
 // (surface oversampling 16 by the FFT)

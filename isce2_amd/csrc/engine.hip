@@ -59,13 +59,11 @@ Engine::~Engine() {
     if (host_counts) (void)hipHostFree(host_counts);
 }
 
-// FP64 rows are few (re-runs of near ties): radices of at most 4 spread a row over more
-// threads (a radix-16 pass of 144 points has 9 butterflies)
-FftDesc make_schedule(int n, bool f64) {
+FftDesc make_schedule(int n, bool few) {
     FftDesc d{};
     d.n = n;
     int m = n;
-    const int pow2[] = {f64 ? 4 : 16, f64 ? 4 : 8, 4, 2};
+    const int pow2[] = {few ? 4 : 16, few ? 4 : 8, 4, 2};
     const int odd[] = {3, 5, 7, 11, 13, 17};
     for (int r : pow2)
         while (m % r == 0 && m > 1) { d.radix[d.npass++] = r; m /= r; }
@@ -84,8 +82,8 @@ const FftPlan &Engine::plan(int n) {
     forbid_in_nosync("build an FFT plan");
     std::unique_ptr<FftPlan> p(new FftPlan());
     p->n = n;
-    p->desc32 = make_schedule(n, false);
-    p->desc64 = make_schedule(n, true);
+    p->desc32 = p->desc64 = make_schedule(n, false);
+    p->desc64_few = make_schedule(n, true);
     std::vector<float> t32(2 * n);
     std::vector<double> t64(2 * n);
     for (int k = 0; k < n; ++k) {
@@ -100,7 +98,7 @@ const FftPlan &Engine::plan(int n) {
     HIP_OK(hipMemcpy(p->tw32.ptr, t32.data(), t32.size() * sizeof(float), hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(p->tw64.ptr, t64.data(), t64.size() * sizeof(double), hipMemcpyHostToDevice));
     p->desc32.tw = p->tw32.ptr;
-    p->desc64.tw = p->tw64.ptr;
+    p->desc64.tw = p->desc64_few.tw = p->tw64.ptr;
     auto &ref = *p;
     plans[n] = std::move(p);
     return ref;
@@ -197,7 +195,7 @@ void Engine::set_fft_radices(int n, const int32_t *radices, int count) {
     }
     if (prod != n) throw Error(AMPCOR_E_ARG, "FFT radices do not multiply to " + std::to_string(n));
     FftPlan &p = const_cast<FftPlan &>(plan(n));
-    for (FftDesc *d : {&p.desc32, &p.desc64}) {
+    for (FftDesc *d : {&p.desc32, &p.desc64, &p.desc64_few}) {
         d->direct = 0;
         d->npass = count;
         for (int i = 0; i < count; ++i) d->radix[i] = radices[i];
@@ -236,8 +234,9 @@ namespace {
 // elems: complex elements one FFT block holds (x2 buffers in LDS), the
 // "fft_block_elems" launch option
 template <class T, int DIR>
-void fft_rows(const FftPlan &pl, cx<T> *data, int64_t nrows, int elems, hipStream_t st) {
-    const FftDesc &d = std::is_same<T, float>::value ? pl.desc32 : pl.desc64;
+void fft_rows(const FftPlan &pl, cx<T> *data, int nimg, int h, int elems, hipStream_t st) {
+    const FftDesc &d = pl.desc<T>(nimg);
+    const int64_t nrows = int64_t(nimg) * h;
     const int g = std::max(1, elems / pl.n);
     const size_t lds = 2 * size_t(g) * pl.n * sizeof(cx<T>);
     const int64_t nblk = (nrows + g - 1) / g;
@@ -260,7 +259,7 @@ int cols_per_block(const FftPlan &pl, int w, int elems, int width) {
 
 template <class T, int DIR>
 void fft_cols(const FftPlan &pl, cx<T> *data, int nimg, int w, int elems, hipStream_t st, int width = 0) {
-    const FftDesc &d = std::is_same<T, float>::value ? pl.desc32 : pl.desc64;
+    const FftDesc &d = pl.desc<T>(nimg);
     const int c = cols_per_block<T>(pl, w, elems, width);
     const size_t lds = 2 * size_t(c) * pl.n * sizeof(cx<T>);
     const int threads = c >= 16 ? 512 : 256;
@@ -282,21 +281,20 @@ template <class T, int DIR, int OUT>
 void fft2_quad(Engine &e, const cx<T> *in, int nimg, int h, int w, cx<T> *work, int H, int W, T *out,
                hipStream_t st) {
     const FftPlan &pr = e.plan(W), &pc = e.plan(H);
-    const bool f32 = std::is_same<T, float>::value;
     const int elems = fft_elems<T>(e), sel = 2 * (h / 2);
     const int g = std::max(1, elems / W);
     hipLaunchKernelGGL((k_fft_rows_quad<T, DIR>), dim3(idivup(nimg * sel, g)), dim3(256),
-                       2 * size_t(g) * W * sizeof(cx<T>), st, in, nimg, h, w, work, H, g, f32 ? pr.desc32 : pr.desc64);
+                       2 * size_t(g) * W * sizeof(cx<T>), st, in, nimg, h, w, work, H, g, pr.desc<T>(nimg));
     const int c = cols_per_block<T>(pc, W, elems, cols_width<T>(e));
     hipLaunchKernelGGL((k_fft_cols_quad<T, DIR, OUT>), dim3(idivup(W, c), nimg), dim3(c >= 16 ? 512 : 256),
-                       2 * size_t(c) * H * sizeof(cx<T>), st, work, W, c, h / 2, f32 ? pc.desc32 : pc.desc64, out);
+                       2 * size_t(c) * H * sizeof(cx<T>), st, work, W, c, h / 2, pc.desc<T>(nimg), out);
 }
 
 // 2D FFT of nimg images h x w (rows then columns), in place
 template <class T, int DIR>
 void fft2(Engine &e, cx<T> *data, int nimg, int h, int w, hipStream_t st) {
     // double elements take twice the LDS: half the element budget (fft_elems)
-    fft_rows<T, DIR>(e.plan(w), data, int64_t(nimg) * h, fft_elems<T>(e), st);
+    fft_rows<T, DIR>(e.plan(w), data, nimg, h, fft_elems<T>(e), st);
     fft_cols<T, DIR>(e.plan(h), data, nimg, w, fft_elems<T>(e), st, cols_width<T>(e));
 }
 
@@ -308,7 +306,7 @@ void fft2_chip(Engine &e, const cx<T> *src, int ih, int iw, const int32_t *start
     const FftPlan &pl = e.plan(w);
     const int g = std::max(1, fft_elems<T>(e) / w);
     hipLaunchKernelGGL((k_fft_rows_chip<T, DIR>), dim3(idivup(nimg * h, g)), dim3(256), 2 * size_t(g) * w * sizeof(cx<T>),
-                       st, src, ih, iw, start, tab, dst, nimg, h, g, sizeof(T) == 4 ? pl.desc32 : pl.desc64);
+                       st, src, ih, iw, start, tab, dst, nimg, h, g, pl.desc<T>(nimg));
     fft_cols<T, DIR>(e.plan(h), dst, nimg, w, fft_elems<T>(e), st, cols_width<T>(e));
 }
 
@@ -408,17 +406,16 @@ void os2_both(Engine &, OsJob<double> a, OsJob<double> b, int nimg, hipStream_t 
 // any even sides, Stockham transforms
 template <class T>
 void os2_general(Engine &e, const OsJob<T> &j, int nimg, hipStream_t st) {
-    const bool f32 = std::is_same<T, float>::value;
     const FftPlan &pc = e.plan(j.h), &pr = e.plan(j.w);
     // up to 16 columns per block (whole 128-byte row segments) within 80 KB of LDS
     const int cb = std::max(1, std::min(j.w, std::min(16, (81920 / int(j.h * sizeof(cx<T>)) - 1) / 2)));
     hipLaunchKernelGGL(k_os2_cols<T>, dim3(idivup(j.w, cb), nimg), dim3(256), (2 * size_t(cb) + 1) * j.h * sizeof(cx<T>), st,
-                       j.chip, j.tab, j.w, cb, f32 ? pc.desc32 : pc.desc64, j.Y);
+                       j.chip, j.tab, j.w, cb, pc.desc<T>(nimg), j.Y);
     // rows per block from the element budget, within 80 KB of LDS
     const int row_bytes = j.w * int(2 * sizeof(cx<T>) + sizeof(T)) + 8;
     const int g = std::max(1, std::min(fft_elems<T>(e) / j.w, (81920 - 8 - j.w * int(sizeof(cx<T>))) / row_bytes));
     hipLaunchKernelGGL(k_os2_rows<T>, dim3(idivup(nimg * 2 * j.h, g)), dim3(256), os2_rows_lds<T>(g, j.w), st, j.chip, j.tab,
-                       j.Y, nimg, j.h, g, f32 ? pr.desc32 : pr.desc64, j.out);
+                       j.Y, nimg, j.h, g, pr.desc<T>(nimg), j.out);
 }
 
 // Row-spectrum transform lengths with an in-place kernel (k_rowspec_f):
@@ -652,13 +649,13 @@ void Engine::run_staged_t(const RunArgs &a) {
         t.blocks = idivup(n * ((t.h + 1) / 2), g);
         hipLaunchKernelGGL(k_rowspec<T>, dim3(t.blocks + idivup(n * ((s.h + 1) / 2), g)), dim3(256),
                            size_t(g) * (2 * L * sizeof(cx<T>) + sizeof(int64_t) + sizeof(T)), st, t, s, n, g,
-                           f32 ? pl.desc32 : pl.desc64);
+                           pl.desc<T>(n));
     };
     // lag sums and their inverse transform (not normalized)
     auto row_correlate = [&](int th, int sh, int L, int NL, int NLw, T *out, int n) {
         const int H1 = L / 2 + 1;
         const FftPlan &pl = plan(L);
-        const FftDesc &d = f32 ? pl.desc32 : pl.desc64;
+        const FftDesc &d = pl.desc<T>(n);
         const int g = std::max(1, fft_elems<T>(*this) / L);
         const size_t lds = 2 * size_t(g) * L * sizeof(cx<T>);
         cx<T> *tspec = rspec, *sspec = rspec + size_t(n) * th * H1;
