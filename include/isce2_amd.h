@@ -89,6 +89,11 @@ int ampcor_destroy(ampcor_ctx *ctx);
  * Replaces cuAmpcorParameter::setupParameters (cuAmpcorParameter.cpp:70-109). */
 int ampcor_setup(ampcor_ctx *ctx, const ampcor_params *params, ampcor_sizes *sizes_out);
 
+/* 1 if AMPCOR_MODE_AUTO runs the fused kernels for the configuration of the last
+ * ampcor_setup, 0 if the staged pipeline (also before any). No counterpart in the
+ * reference. ampcor_sizes.fused says the narrower AMPCOR_MODE_FUSED. */
+int ampcor_auto_fused(const ampcor_ctx *ctx);
+
 /* Run the per-window pipeline for n windows.
  * Replaces cuAmpcorController::runAmpcor's chunk loop and cuAmpcorChunk::run
  * (cuAmpcorController.cpp:107-137; cuAmpcorChunk.cpp:12-217), with images

@@ -27,7 +27,7 @@ EXPORTS = ("ampcor_create", "ampcor_destroy", "ampcor_setup", "ampcor_run_window
            "ampcor_profile", "ampcor_profile_report", "ampcor_last_error", "ampcor_version",
            "ampcor_set_fft_radices", "ampcor_set_option", "ampcor_profile_only",
            "ampcor_start_pixels", "ampcor_check_range", "ampcor_run_windows_noalloc",
-           "ampcor_select_near_ties")
+           "ampcor_select_near_ties", "ampcor_auto_fused")
 
 
 class Params(C.Structure):
@@ -63,6 +63,7 @@ def load() -> C.CDLL:
     lib.ampcor_create.argtypes = [i32, C.POINTER(vp)]
     lib.ampcor_destroy.argtypes = [vp]
     lib.ampcor_setup.argtypes = [vp, C.POINTER(Params), C.POINTER(Sizes)]
+    lib.ampcor_auto_fused.argtypes = [vp]
     run_args = [vp, vp, i64, i64, i64, vp, i64, i64, i64, vp, vp, vp, vp, i32, vp, vp, vp]
     lib.ampcor_run_windows.argtypes = run_args + [i32, i32, vp]
     lib.ampcor_run_windows_debug.argtypes = run_args + [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, vp]
@@ -86,7 +87,7 @@ def load() -> C.CDLL:
                  "ampcor_run_windows_debug", "ampcor_profile", "ampcor_profile_report",
                  "ampcor_set_precision", "ampcor_precision_stats", "ampcor_set_fft_radices",
                  "ampcor_set_option", "ampcor_profile_only", "ampcor_start_pixels", "ampcor_check_range",
-                 "ampcor_run_windows_noalloc", "ampcor_select_near_ties"):
+                 "ampcor_run_windows_noalloc", "ampcor_select_near_ties", "ampcor_auto_fused"):
         getattr(lib, name).restype = C.c_int
     _lib = lib
     return lib

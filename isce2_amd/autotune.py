@@ -3,8 +3,9 @@
 For one window configuration (window, half search) the tuner times candidate
 schedules on a sample of real windows and keeps the fastest:
 
-* execution path: the fused per-window kernels (where they cover the size) or
-  the staged pipeline;
+* execution path: the fused per-window kernels (where they cover the size; by
+  automatic mode for the surfaces that MODE_FUSED does not take) or the staged
+  pipeline;
 * chunk: windows per launch;
 * FFT radix order of every staged transform length (coordinate descent over
   the orderings of each length's factorization into supported radices).
@@ -21,7 +22,7 @@ from dataclasses import asdict, dataclass, field
 
 import torch
 
-from .engine import MODE_FUSED, MODE_STAGED, Engine, WindowParams
+from .engine import MODE_AUTO, MODE_FUSED, MODE_STAGED, Engine, WindowParams
 
 @dataclass
 class Schedule:
@@ -85,6 +86,7 @@ class Autotuner:
         self.sample = sample
         self.radix_sample = radix_sample
         self.cache = {}
+        self.tuned = set()          # keys timed by this object (the others come from the file)
         self.cache_file = cache_file
         if cache_file and os.path.exists(cache_file):
             with open(cache_file) as fh:
@@ -123,9 +125,13 @@ class Autotuner:
         k = self.key(params)
         sizes = eng.setup(params)
         if k in self.cache:
-            if self.cache[k].mode != MODE_FUSED or sizes["fused"]:
+            mode = self.cache[k].mode
+            # kept unless it is a fused schedule for a configuration the fused kernels do not
+            # cover, or a staged one saved before automatic mode ran them for this one
+            if k in self.tuned or not (mode == MODE_FUSED and not sizes["fused"]
+                                       or mode == MODE_STAGED and eng.auto_fused and not sizes["fused"]):
                 return self.cache[k]
-            del self.cache[k]           # a fused schedule for a configuration the fused kernels do not cover
+            del self.cache[k]
         m = min(n, self.sample)
         sub = list(args[:2]) + [t[:m].contiguous() for t in args[2:]]
         prev = eng.precision
@@ -133,8 +139,8 @@ class Autotuner:
         best = None
         try:
             cands = []
-            if sizes["fused"]:
-                cands += [(MODE_FUSED, c) for c in (512, 1024, 2048, 4096)]
+            if eng.auto_fused:
+                cands += [(MODE_FUSED if sizes["fused"] else MODE_AUTO, c) for c in (512, 1024, 2048, 4096)]
             cands += [(MODE_STAGED, c) for c in (64, 256, 1024)]
             for mode, chunk in cands:
                 t = self._time(eng, sub, mode, min(chunk, max(m, 1)), m)
@@ -183,5 +189,6 @@ class Autotuner:
         finally:
             eng.set_precision(prev)
         self.cache[k] = best
+        self.tuned.add(k)
         self.save()
         return best

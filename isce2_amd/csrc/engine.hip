@@ -1294,6 +1294,8 @@ int ampcor_setup(ampcor_ctx *ctx, const ampcor_params *params, ampcor_sizes *siz
     });
 }
 
+int ampcor_auto_fused(const ampcor_ctx *ctx) { return ctx && ctx->eng.fused_auto ? 1 : 0; }
+
 int ampcor_run_windows_debug(ampcor_ctx *ctx, const void *ref_img, int64_t ref_h, int64_t ref_w, int64_t ref_pitch,
                              const void *sec_img, int64_t sec_h, int64_t sec_w, int64_t sec_pitch,
                              const int32_t *ref_d, const int32_t *ref_a, const int32_t *sec_d,

@@ -62,6 +62,7 @@ class Engine:
         self.precision = 1
         self.tau = [TAU_DEFAULT, TAU_DEFAULT]   # precision-1 margin thresholds (coarse, fine)
         self.sizes: dict | None = None
+        self.auto_fused = False
 
     def close(self):
         if getattr(self, "_h", None) is not None and self._h.value:
@@ -80,6 +81,7 @@ class Engine:
         check(self.lib.ampcor_setup(self._h, C.byref(cp), C.byref(s)), self._h)
         self.params = params
         self.sizes = s.as_dict()
+        self.auto_fused = bool(self.lib.ampcor_auto_fused(self._h))   # MODE_AUTO runs the fused kernels
         return self.sizes
 
     def run_windows(self, ref, sec, ref_d, ref_a, sec_d, sec_a, *, mode=MODE_AUTO, chunk=0,

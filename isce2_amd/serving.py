@@ -225,7 +225,7 @@ class OffsetServer:
         large job does not pay for growing them (a free synchronizes the device)."""
         if self.arena.ref.shape[0] < eng.sizes["search_h"] or self.arena.pitch < eng.sizes["search_w"]:
             return
-        fused = mode == MODE_FUSED or (mode == MODE_AUTO and eng.sizes["fused"])
+        fused = mode == MODE_FUSED or (mode == MODE_AUTO and eng.auto_fused)
         m = min(self.max_batch, chunk if chunk > 0 else (self.max_batch if fused else 1024))
         z = torch.zeros(m, dtype=torch.int32, device=self.dev)
         prec = eng.precision
