@@ -106,6 +106,8 @@ int ampcor_auto_fused(const ampcor_ctx *ctx);
  *   out_cov : float[n][3] (cov_down, cov_across, cov_cross).
  *   chunk : windows per launch (0 = engine default: 1024 for the staged
  *           pipeline, 32768 for the fused kernels); mode : AMPCOR_MODE_*.
+ *           A launch's scratch is kept by the context: about 148 KB a window
+ *           in the fused kernels at window 64 (4.8 GB at 32768 windows).
  *   stream : hipStream_t (NULL = default stream). The call is asynchronous
  *   with respect to the host; synchronize the stream before reading outputs.
  * A window whose chips leave their image fails the call with AMPCOR_E_RANGE
@@ -126,7 +128,9 @@ int ampcor_run_windows(ampcor_ctx *ctx,
  * before adjustment), zoom start (i_offsetInitAdjusted), zoom shift
  * (i_maxLocShift) and oversampled-surface argmax (i_offsetZoomIn), plus the raw
  * peak value (r_maxval). Names follow CUAMPCOR_DEBUG (cuAmpcorChunk.cpp:82-198).
- * The fused path also reports each window's argmax margins (float[n]).
+ * The argmax margins (float[n]) are top-1 minus top-2 of the normalized surfaces;
+ * a fine margin above 2^-12 of the largest sample may leave out a runner-up
+ * in a surface column that cannot hold the maximum.
  * out_offset_fp64 (double[n][2], down/across) is an FP64 sub-pixel refinement
  * with no counterpart in the reference (whose offset is the bare argmax on the
  * 1/(surf_ovs*raw_ovs) grid, cuOffset.cu:137-187): the FFT-interpolated surface

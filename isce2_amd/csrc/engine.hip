@@ -552,9 +552,9 @@ void Engine::run_staged_t(const RunArgs &a) {
     // 1024 search columns) no mean-free template image is needed: the mean is subtracted as
     // the template rows load, and the raw stage's rows are the amplitudes of chips read in place
     const bool lean_raw = S_w <= 1024, lean_os = OSw <= 1024;
-    // the separable oversampler covers the x2 interpolation of even-sided chips (an
-    // odd side loses its middle spectrum line to the quadrant padding, which does
-    // not factor into the half-sample form)
+    // the separable oversampler covers the x2 interpolation of even-sided chips (an odd
+    // side loses its middle spectrum line to the quadrant padding, which changes the even
+    // samples too: the kernels have no such form)
     const bool sep_os = oversampler >= 2 && p.raw_ovs == 2 && sz.os_win_h == 2 * W_h && sz.os_win_w == 2 * W_w &&
                         OSh == 2 * sz.zoom_in_h && OSw == 2 * sz.zoom_in_w && W_h % 2 == 0 && W_w % 2 == 0 &&
                         sz.zoom_in_h % 2 == 0 && sz.zoom_in_w % 2 == 0;
@@ -660,8 +660,8 @@ void Engine::run_staged_t(const RunArgs &a) {
         const size_t lds = 2 * size_t(g) * L * sizeof(cx<T>);
         cx<T> *tspec = rspec, *sspec = rspec + size_t(n) * th * H1;
         // lags per thread: 17 once there is more than one group of 9 (each group
-        // re-reads every spectrum; the sums themselves do not depend on the
-        // grouping), unless that leaves too few workgroups to fill the GPU
+        // re-reads every spectrum), unless that leaves too few workgroups to fill the
+        // GPU (a sum's two or four parts round differently in its last bits)
         if (NL > 9 && n * idivup(H1, 64) >= 2048)
             hipLaunchKernelGGL((k_mac_lags<T, 17, 2>), dim3(idivup(H1, 64), idivup(NL, 17), n), dim3(128), 0, st, tspec,
                                th, sspec, sh, NL, L, rq, T(1.0 / double(L)));

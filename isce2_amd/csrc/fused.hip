@@ -837,7 +837,7 @@ __global__ void __launch_bounds__(NTH, T == 64 ? 6 : 2) k_fine(FineArgs a, const
 // arrive, with the first and last NL - 1 rows kept for the slides. The lag sums run on
 // the matrix cores from the transforms of packed row pairs (lag_sums), without the pass
 // that splits the pairs.
-// Bound by vector and matrix issue (about 29.7k + 2.9k instructions a window, 70% of its
+// Bound by vector and matrix issue (about 30.9k + 2.9k instructions a window, 70% of its
 // time) and, with two workgroups a CU, by the waits between its short phases: of 3.1 ms
 // for 31,248 windows the chip loads take 0.8, the row transforms 0.5, the lag sums 0.6,
 // the normalization 0.25, the inverse 0.1 and the surface 0.45 ms. With split spectra and
@@ -1060,8 +1060,8 @@ void launch_fine2(int surf, const FineArgs &a, const cf *tw, int n, int w0, size
 // Surface oversampling factors the fused kernels evaluate: 2..32 (FFT: one thread
 // per surface column of a 512-thread workgroup; sinc: the patch's rows fit in LDS).
 // Factor 1 and above 32 stay with the staged pipeline. 3,844 windows of 64, half
-// search 20, factor 32: staged 11.8 ms, fused 1.36 ms; 900 with the sinc surface:
-// staged 1.96 ms, fused 0.55 ms.
+// search 20, factor 32: staged 2.66 ms, fused 1.18 ms; 900 with the sinc surface:
+// staged 0.76 ms, fused 0.39 ms.
 bool fused_fits(const ampcor_params &p, const ampcor_sizes &s) {
     using namespace fused;
     if (p.window_h != p.window_w || (p.window_h != 32 && p.window_h != 64)) return false;
