@@ -83,10 +83,10 @@ struct Norms48 {
         r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
         const float h = float(r);
         hi[i] = h;
-        lo[i] = uint16_t(__float_as_uint(float(r - double(h))) >> 16);
+        lo[i] = uint16_t(__float_as_uint(float((r - double(h)) * 0x1p24)) >> 16);   // scaled: normal wherever h is
     }
     template <int L> __device__ __forceinline__ float normalized(float c, int i) const {
-        const double r = double(hi[i]) + double(__uint_as_float(uint32_t(lo[i]) << 16));
+        const double r = fma(double(__uint_as_float(uint32_t(lo[i]) << 16)), 0x1p-24, double(hi[i]));
         return float(double(c) * r * (1.0 / L));
     }
 };

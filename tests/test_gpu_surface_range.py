@@ -1,6 +1,6 @@
 """Surfaces other than factor 16 by the FFT keep the staged pipeline's FP64 normalization in
 the fused kernels that automatic mode runs for them: images whose sums of squares, multiplied,
-leave FP32's range (amplitudes around 1e10; FP32 correlations themselves reach 1e24) give what
+leave FP32's range (amplitudes around 1e10 and 1e15; FP32 correlations themselves reach 1e34) give what
 the FP64 oracle gives, without the FP64 re-run. Bar as in test_gpu_parity where the argmax is
 clear of FP32 rounding (both leads above 2e-6): integer peaks equal, offsets within 0.01 px,
 SNR and covariance within 1e-3.
@@ -19,9 +19,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("W,hs", [(64, 20), (32, 9)])
 @pytest.mark.parametrize("kw", [dict(surf_ovs=32), dict(surf_ovs=5), dict(surf_method=1)])
-@pytest.mark.parametrize("real", [False, True])
-def test_bright_images(W, hs, kw, real):
-    ref, sec = (z * np.float32(1e10) for z in speckle_pair_shift(400, 400, shift=(3.7, -2.4), snr_db=15.0, seed=11))
+@pytest.mark.parametrize("real,scale", [(False, 1e10), (True, 1e10), (False, 1e15)])
+def test_bright_images(W, hs, kw, real, scale):
+    ref, sec = (z * np.float32(scale) for z in speckle_pair_shift(400, 400, shift=(3.7, -2.4), snr_db=15.0, seed=11))
     if real:
         ref, sec = np.abs(ref), np.abs(sec)
     cfg = O.AmpcorConfig(window_h=W, window_w=W, hs_down=hs, hs_across=hs, **kw)
